@@ -216,6 +216,10 @@ int qattn_fwd(qattn_seq q8, const float* q_scale, qattn_seq k8, const float* k_s
  */
 int qattn_v_tile_half(qattn_seq v, int dtype, int64_t B, int64_t L, int64_t H, int64_t D, uint16_t* v16,
                       int64_t Lpad, qattn_stream_t stream);
+/* The same with the tiles' dtype: out_dtype == dtype, or bf16 V rounded to fp16 tiles (RNE), which the fp16-P.V
+ * entries need for bf16 models (the reference converts V first, sparse_sage.py:57, sageattn2.py:880-885). */
+int qattn_v_tile_half_ex(qattn_seq v, int dtype, int out_dtype, int64_t B, int64_t L, int64_t H, int64_t D,
+                         uint16_t* v16, int64_t Lpad, qattn_stream_t stream);
 
 /*
  * The prologue of the INT8-QK / FP8-PV path in four launches: one pass over K and V for their column
@@ -273,6 +277,9 @@ int qattn_quant_qk_varlen_int8(qattn_seq q, qattn_seq k, int dtype, int64_t B, i
 int qattn_v_tile_half_varlen(qattn_seq v, int dtype, int64_t B, int64_t total_k, int64_t max_lk, int64_t H, int64_t D,
                              const int32_t* cu_seqlens_k, const int32_t* cu_vt, uint16_t* v16, int64_t Lpad,
                              qattn_stream_t stream);
+int qattn_v_tile_half_varlen_ex(qattn_seq v, int dtype, int out_dtype, int64_t B, int64_t total_k, int64_t max_lk,
+                                int64_t H, int64_t D, const int32_t* cu_seqlens_k, const int32_t* cu_vt,
+                                uint16_t* v16, int64_t Lpad, qattn_stream_t stream);
 int qattn_fwd_varlen(qattn_seq q8, const float* q_scale, qattn_seq k8, const float* k_scale, const uint16_t* v16,
                      int64_t Lpad, qattn_seq o, int out_dtype, int64_t B, int64_t total_q, int64_t total_k,
                      int64_t max_lq, int64_t max_lk, int64_t Hq, int64_t Hkv, int64_t D, float qk_mult, int causal,
@@ -364,9 +371,10 @@ int qattn_fwd_ex_blocks_per_workgroup(int64_t B, int64_t Lq, int64_t Lk, int64_t
 /*
  * Which kernel a qattn_fwd_ex launch runs (no counterpart in the reference, whose launch is one CTA
  * kernel per query block; for benchmarks and tests):
- *   QATTN_KERNEL_ONE_BLOCK:   one query block (128 rows, 4 waves) per workgroup; half-P.V and
- *                             block-sparse launches always run it, KV-split launches unless they fit
- *                             one round of 128-256 ping-pong workgroups
+ *   QATTN_KERNEL_ONE_BLOCK:   one query block (128 rows, 4 waves) per workgroup; KV-split launches run it unless
+ *                             they fit one round of 128-256 ping-pong workgroups.  Half-P.V, block-sparse and
+ *                             varlen launches report this value too, whatever qattn_set_kernel says: they have a
+ *                             kernel of their own (two wave groups per workgroup, attn_half.hip)
  *   QATTN_KERNEL_MULTI_BLOCK: several query blocks of a head per workgroup through one K/V pipeline
  *                             (short, non-causal FP8 key ranges; see qattn_fwd_ex_blocks_per_workgroup)
  *   QATTN_KERNEL_PINGPONG:    two query blocks per workgroup (8 waves) whose wave groups alternate

@@ -644,46 +644,87 @@ static void launch_v_fp8(int dtype, int64_t D, const uint16_t* p, const qattn_se
 #undef QATTN_VF
 }
 
-template <int D>
+// V in the half tile layout, as given or (CONV) bf16 rounded to fp16 on the way: the fp16 P.V entries take bf16
+// models' V, and a conversion pass of its own cost more than this whole kernel (32760 x 12 x 128: 120 us next to
+// 50).  HBM-bound: 2 B read and 2 B written per element.  A thread holds one key quad (four consecutive slots of the
+// tile) of 8 channels, so the LDS tile is written in 8-byte words; its 16-byte chunks are XOR-swizzled by the channel
+// group so that a wave's words spread over the banks.  The loads of both tiles of a workgroup are issued first.
+template <bool CONV, int D>
 __global__ __launch_bounds__(256) void v_tile_half_kernel(const uint16_t* in, int64_t sb, int64_t sl, int64_t sh,
                                                           int64_t L, int64_t H, uint16_t* v16, int64_t Lpad,
                                                           const int32_t* cu_k = nullptr, const int32_t* cu_vt = nullptr,
                                                           int64_t total_k = 0) {
   constexpr int TPR = D / 8;
-  __shared__ __align__(16) uint16_t tile[D][64];
-  int64_t t = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  __shared__ __align__(16) uint16_t tile[kVTilesPerWG][D][64];
+  const int64_t t0 = (int64_t)blockIdx.x * kVTilesPerWG, h = blockIdx.y;
+  int64_t b = blockIdx.z, col0 = 0;  // col0: first tile column of this entry in v16
   const int tid = threadIdx.x;
-  int64_t tcol = t;  // tile column in v16
   if (cu_k) {  // packed variable-length keys: sequence b's tile t goes to tile column cu_vt[b] + t of entry 0
     int64_t k0;
     varlen_range(cu_k, b, total_k, L, k0, L);
-    tcol = (int64_t)cu_vt[b] + t;
-    if (t * 64 >= L || (tcol + 1) * 64 > Lpad) return;  // (a too small Lpad drops tiles, never overruns)
+    col0 = cu_vt[b];
     in += k0 * sl;
     b = 0;
   }
+  bool act[kVTilesPerWG];  // (packed: a too small Lpad drops tiles, never overruns)
 #pragma unroll
-  for (int i = 0; i < 64 * TPR / 256; i++) {
-    const int c = tid + i * 256;
-    const int row = c / TPR, dc = c % TPR;
-    const int64_t l = t * 64 + row;
-    uint16_t hv[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (l < L) {
-      v4u raw = *reinterpret_cast<const v4u*>(in + b * sb + l * sl + h * sh + dc * 8);
-      __builtin_memcpy(hv, &raw, 16);
+  for (int tt = 0; tt < kVTilesPerWG; tt++)
+    act[tt] = (col0 + t0 + tt + 1) * 64 <= Lpad && !(cu_k && (t0 + tt) * 64 >= L);
+  if (!act[0]) return;
+  const int q = tid / TPR, dc = tid % TPR;  // key quad (keys 4q .. 4q + 3) x 8 channels
+  const bool lane = tid < 16 * TPR;
+  uint16_t hv[kVTilesPerWG][4][8];
+#pragma unroll
+  for (int tt = 0; tt < kVTilesPerWG; tt++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int64_t l = (t0 + tt) * 64 + 4 * q + r;
+      v4u raw = {0u, 0u, 0u, 0u};
+      if (act[tt] && lane && l < L) raw = *reinterpret_cast<const v4u*>(in + b * sb + l * sl + h * sh + dc * 8);
+      __builtin_memcpy(hv[tt][r], &raw, 16);
     }
-    const int pos = vtile_pos(row);
+  const int wi = vtile_pos(4 * q) >> 2;  // 8-byte word of the quad in its channel's row
+  if (lane) {
 #pragma unroll
-    for (int e = 0; e < 8; e++) tile[dc * 8 + e][pos] = hv[e];
+    for (int tt = 0; tt < kVTilesPerWG; tt++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        uint16_t x[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) x[r] = CONV ? f32_to_f16(bf16_to_f32(hv[tt][r][e])) : hv[tt][r][e];
+        v2u word;
+        __builtin_memcpy(&word, x, 8);
+        *reinterpret_cast<v2u*>(&tile[tt][dc * 8 + e][(((wi >> 1) ^ (dc & 7)) * 2 + (wi & 1)) * 4]) = word;
+      }
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < D * 8 / 256; i++) {
-    const int c = tid + i * 256;
-    const int d = c / 8, cc = c % 8;
-    *reinterpret_cast<v4u*>(v16 + ((b * H + h) * D + d) * Lpad + tcol * 64 + cc * 8) =
-        *reinterpret_cast<const v4u*>(&tile[d][cc * 8]);
+  for (int tt = 0; tt < kVTilesPerWG; tt++) {
+    if (!act[tt]) continue;
+#pragma unroll
+    for (int i = 0; i < D * 8 / 256; i++) {
+      const int c = tid + i * 256;
+      const int d = c / 8, cc = c % 8;
+      *reinterpret_cast<v4u*>(v16 + ((b * H + h) * D + d) * Lpad + (col0 + t0 + tt) * 64 + cc * 8) =
+          *reinterpret_cast<const v4u*>(&tile[tt][d][(cc ^ ((d >> 3) & 7)) * 8]);
+    }
   }
+}
+
+static void launch_v_tile_half(dim3 grid, bool conv, int64_t D, const qattn_seq& v, int64_t L, int64_t H, uint16_t* v16,
+                               int64_t Lpad, hipStream_t st, const int32_t* cu_k = nullptr,
+                               const int32_t* cu_vt = nullptr, int64_t total_k = 0) {
+  const uint16_t* p = static_cast<const uint16_t*>(v.data);
+#define QATTN_VT(C, DD) \
+  v_tile_half_kernel<C, DD><<<grid, 256, 0, st>>>(p, v.sb, v.sl, v.sh, L, H, v16, Lpad, cu_k, cu_vt, total_k)
+  if (conv) {
+    if (D == 128) QATTN_VT(true, 128);
+    else QATTN_VT(true, 64);
+  } else {
+    if (D == 128) QATTN_VT(false, 128);
+    else QATTN_VT(false, 64);
+  }
+#undef QATTN_VT
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1028,20 +1069,29 @@ extern "C" int qattn_per_channel_fp8_ex(qattn_seq v, int dtype, int64_t B, int64
   return check_launch("per_channel_fp8");
 }
 
+// the dtype of the half tiles: V's own, or fp16 from bf16
+static int check_tile_dtype(int dtype, int out_dtype) {
+  QATTN_REQUIRE(out_dtype == dtype || (dtype == QATTN_BF16 && out_dtype == QATTN_FP16), QATTN_ERR_DTYPE,
+                "half V tiles are in V's dtype, or fp16 from bf16 (dtype %d, out_dtype %d)", dtype, out_dtype);
+  return QATTN_OK;
+}
+
 extern "C" int qattn_v_tile_half(qattn_seq v, int dtype, int64_t B, int64_t L, int64_t H, int64_t D, uint16_t* v16,
                                  int64_t Lpad, qattn_stream_t stream) {
+  return qattn_v_tile_half_ex(v, dtype, dtype, B, L, H, D, v16, Lpad, stream);
+}
+
+extern "C" int qattn_v_tile_half_ex(qattn_seq v, int dtype, int out_dtype, int64_t B, int64_t L, int64_t H, int64_t D,
+                                    uint16_t* v16, int64_t Lpad, qattn_stream_t stream) {
   int rc;
-  if ((rc = check_common(dtype, D, QATTN_QUANT_CUDA, 64))) return rc;
+  if ((rc = check_common(dtype, D, QATTN_QUANT_CUDA, 64)) || (rc = check_tile_dtype(dtype, out_dtype))) return rc;
   QATTN_REQUIRE(B > 0 && L > 0 && H > 0, QATTN_ERR_SHAPE, "v_tile_half needs non-empty input");
   if ((rc = check_seq("v", v, 2))) return rc;
   QATTN_REQUIRE(Lpad >= (L + 63) / 64 * 64 && Lpad % 64 == 0, QATTN_ERR_SHAPE,
                 "Lpad must be a multiple of 64 and >= L rounded up to 64");
   QATTN_REQUIRE(v16 && aligned16(v16), QATTN_ERR_ALIGN, "v16 must be non-null and 16-byte aligned");
-  hipStream_t st = (hipStream_t)stream;
-  dim3 grid((unsigned)(Lpad / 64), (unsigned)H, (unsigned)B);
-  const uint16_t* p = static_cast<const uint16_t*>(v.data);
-  if (D == 128) v_tile_half_kernel<128><<<grid, 256, 0, st>>>(p, v.sb, v.sl, v.sh, L, H, v16, Lpad);
-  else v_tile_half_kernel<64><<<grid, 256, 0, st>>>(p, v.sb, v.sl, v.sh, L, H, v16, Lpad);
+  const dim3 grid((unsigned)((Lpad / 64 + kVTilesPerWG - 1) / kVTilesPerWG), (unsigned)H, (unsigned)B);
+  launch_v_tile_half(grid, dtype != out_dtype, D, v, L, H, v16, Lpad, (hipStream_t)stream);
   return check_launch("v_tile_half");
 }
 
@@ -1261,18 +1311,21 @@ extern "C" int qattn_v_tile_half_varlen(qattn_seq v, int dtype, int64_t B, int64
                                         int64_t D,
                                         const int32_t* cu_seqlens_k, const int32_t* cu_vt, uint16_t* v16,
                                         int64_t Lpad, qattn_stream_t stream) {
+  return qattn_v_tile_half_varlen_ex(v, dtype, dtype, B, total_k, max_lk, H, D, cu_seqlens_k, cu_vt, v16, Lpad, stream);
+}
+
+extern "C" int qattn_v_tile_half_varlen_ex(qattn_seq v, int dtype, int out_dtype, int64_t B, int64_t total_k,
+                                           int64_t max_lk, int64_t H, int64_t D, const int32_t* cu_seqlens_k,
+                                           const int32_t* cu_vt, uint16_t* v16, int64_t Lpad, qattn_stream_t stream) {
   int rc;
-  if ((rc = check_common(dtype, D, QATTN_QUANT_CUDA, 64))) return rc;
+  if ((rc = check_common(dtype, D, QATTN_QUANT_CUDA, 64)) || (rc = check_tile_dtype(dtype, out_dtype))) return rc;
   QATTN_REQUIRE(B > 0 && total_k >= 0 && max_lk > 0 && H > 0, QATTN_ERR_SHAPE, "v_tile_half_varlen needs non-empty input");
   if ((rc = check_seq("v", v, 2))) return rc;
   QATTN_REQUIRE(Lpad % 64 == 0, QATTN_ERR_SHAPE, "Lpad must be a multiple of 64");
   QATTN_REQUIRE(v16 && aligned16(v16) && cu_seqlens_k && cu_vt, QATTN_ERR_ARG, "null or misaligned pointer");
-  hipStream_t st = (hipStream_t)stream;
-  dim3 grid((unsigned)((max_lk + 63) / 64), (unsigned)H, (unsigned)B);
-  const uint16_t* p = static_cast<const uint16_t*>(v.data);
-  if (D == 128) v_tile_half_kernel<128><<<grid, 256, 0, st>>>(p, v.sb, v.sl, v.sh, max_lk, H, v16, Lpad, cu_seqlens_k, cu_vt, total_k);
-  else v_tile_half_kernel<64><<<grid, 256, 0, st>>>(p, v.sb, v.sl, v.sh, max_lk, H, v16, Lpad, cu_seqlens_k, cu_vt,
-                                                    total_k);
+  const dim3 grid((unsigned)((max_lk + 64 * kVTilesPerWG - 1) / (64 * kVTilesPerWG)), (unsigned)H, (unsigned)B);
+  launch_v_tile_half(grid, dtype != out_dtype, D, v, max_lk, H, v16, Lpad, (hipStream_t)stream, cu_seqlens_k, cu_vt,
+                     total_k);
   return check_launch("v_tile_half_varlen");
 }
 

@@ -245,6 +245,27 @@ def v_tile_half(v: torch.Tensor, tensor_layout: str = "HND") -> torch.Tensor:
     return v16
 
 
+def _tile_input_fp16(v: torch.Tensor):
+    """V for the fp16 tiles of the fp16-P.V entries, as (tensor, its dtype code): fp16 V as it is, bf16 V as it is
+    where the tile kernel can read it (it converts on the way), otherwise its fp16 copy."""
+    if v.dtype == torch.bfloat16 and v.stride(-1) == 1 and v.data_ptr() % 16 == 0 and \
+            all(s % 8 == 0 for s in v.stride()[:-1]):
+        return v, _lib.QATTN_BF16
+    return (v if v.dtype == torch.float16 else v.to(torch.float16)), _lib.QATTN_FP16
+
+
+def v_tile_fp16(v: torch.Tensor, tensor_layout: str = "HND") -> torch.Tensor:
+    """V (bf16 or fp16) rounded to fp16 in the kernels' transposed tile layout: v_tile_half(v.to(torch.float16))."""
+    L = _lib.load()
+    v, dt = _tile_input_fp16(v)
+    b, l, h, d = _dims(v, tensor_layout)
+    lpad = (l + 63) // 64 * 64
+    v16 = torch.empty((b, h, d, lpad), dtype=torch.float16, device=v.device)
+    _lib.check(L.qattn_v_tile_half_ex(_lib.seq(v, tensor_layout), dt, _lib.QATTN_FP16, b, l, h, d, _lib.ptr(v16), lpad,
+                                      _lib.stream_of(v)))
+    return v16
+
+
 def _kv_valid_tensor(kv_valid_len, b: int, device) -> Optional[torch.Tensor]:
     if kv_valid_len is None:
         return None
@@ -637,11 +658,11 @@ def sageattn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlen
         d, _lib.ptr(km) if km is not None else None, _lib.ptr(cq), _lib.ptr(ck), _lib.ptr(cu_qs), _lib.ptr(cu_ks),
         _lib.seq(q8, "NHD"), _lib.seq(k8, "NHD"), _lib.ptr(qsc), _lib.ptr(ksc), sm_scale * LOG2E,
         _lib.QATTN_QUANT_TRITON, st))
-    v16 = v4 if v4.dtype == torch.float16 else v4.to(torch.float16)  # the reference runs P.V in fp16
+    v4, vdt = _tile_input_fp16(v4)  # the reference runs P.V in fp16
     lpad = nkblk * BLKK
     vt = torch.empty((1, hkv, d, lpad), dtype=torch.float16, device=dev)
-    _lib.check(L.qattn_v_tile_half_varlen(_lib.seq(v16, "NHD"), _lib.QATTN_FP16, bsz, tk, max_seqlen_k, hkv, d,
-                                          _lib.ptr(ck), _lib.ptr(cu_vt), _lib.ptr(vt), lpad, st))
+    _lib.check(L.qattn_v_tile_half_varlen_ex(_lib.seq(v4, "NHD"), vdt, _lib.QATTN_FP16, bsz, tk, max_seqlen_k, hkv, d,
+                                             _lib.ptr(ck), _lib.ptr(cu_vt), _lib.ptr(vt), lpad, st))
     o4 = out.unsqueeze(0)
     _lib.check(L.qattn_fwd_varlen(
         _lib.seq(q8, "NHD"), _lib.ptr(qsc), _lib.seq(k8, "NHD"), _lib.ptr(ksc), _lib.ptr(vt), lpad,
@@ -678,4 +699,5 @@ __all__ = [
     "sageattn_qk_int8_pv_fp16_cuda",
     "sageattn_qk_int8_pv_fp16_triton",
     "v_tile_half",
+    "v_tile_fp16",
 ]

@@ -50,8 +50,7 @@ def sparse_sageattn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask_id: 
     km = sa.k_mean(k, tensor_layout)
     q8, qs, k8, ks = sa.per_block_int8(q, k, km, sa.BLKQ, sa.BLKK, sm_scale=d ** -0.5, tensor_layout=tensor_layout,
                                        variant="triton")
-    v16 = v if v.dtype == torch.float16 else v.to(torch.float16)  # the reference runs P.V in fp16
-    vt = sa.v_tile_half(v16, tensor_layout)
+    vt = sa.v_tile_fp16(v, tensor_layout)  # the reference runs P.V in fp16
     o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     ns = L.qattn_fwd_block_sparse_num_splits(b, lq, lk, hq)
     wsb = L.qattn_fwd_workspace_size(b, lq, hq, d, ns)

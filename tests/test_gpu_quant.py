@@ -311,3 +311,32 @@ def test_sage_quant_matches_separate_calls(gran, smooth_k, smooth_v, scale_max, 
         assert torch.equal(got[7], vm)
     else:
         assert got[7] is None
+
+
+@pytest.mark.parametrize("layout", ["NHD", "HND"])
+@pytest.mark.parametrize("L,D", [(1, 128), (64, 128), (65, 64), (129, 128), (200, 64)])
+def test_v_tile_fp16_converts_as_torch(layout, L, D):
+    """bf16 V rounded to fp16 inside the tile kernel = the tiles of its torch fp16 copy bit for bit (one, two and an
+    odd number of 64-key tiles; values that overflow fp16, tiny ones and NaN), also for V the kernel cannot read
+    in place (rows that start off a 16-byte boundary)."""
+    dev = require_gpu()
+    from telefuser_amd import sageattn2 as sa
+
+    g = torch.Generator().manual_seed(L + D)
+    v = torch.randn((2, L, 3, D + 4), generator=g)
+    v[0, 0, 0, :4] = torch.tensor([1e30, -7e4, 1e-7, float("nan")])
+    v = v.to(torch.bfloat16).to(dev)
+    for x in (v[..., :D].contiguous(), v[..., 4:]):
+        if layout == "HND":
+            x = x.transpose(1, 2)
+        log(f"v_tile_fp16 {layout} L={L} D={D} strides {x.stride()}")
+        got = sa.v_tile_fp16(x, layout)
+        ref = sa.v_tile_half(x.to(torch.float16).contiguous(), layout)
+        assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+        # the tile layout itself: key 32 kb + 8 g + 4 hf + t of a tile at slot 32 hf + 16 kb + 4 g + t
+        rows = (x if layout == "NHD" else x.transpose(1, 2)).to(torch.float16).cpu()
+        k = torch.arange(L)
+        slot = k // 64 * 64 + (k // 4 % 2) * 32 + (k // 32 % 2) * 16 + (k // 8 % 4) * 4 + k % 4
+        want = torch.zeros(got.shape, dtype=torch.float16)
+        want[..., slot] = rows.permute(0, 2, 3, 1)
+        assert torch.equal(got.cpu().view(torch.int16), want.view(torch.int16))
