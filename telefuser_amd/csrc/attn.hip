@@ -31,268 +31,25 @@
 //     XCDs, so consecutive tiles of one (batch, head) are gathered onto one XCD and share its L2.
 //   * Optional KV split (flash-decoding style) for grids that cannot fill 256 CUs; a combine kernel
 //     merges the partial (O, m, l) triples.
-#include <algorithm>
 #include <mutex>
-#include <type_traits>
 
-#include "common.h"
+#include "attn_device.h"
 
 namespace qattn {
 
-constexpr int kD = 128;
-constexpr int kBQ = 128;  // query quantization block
-constexpr int kWavesPerSimd = 2;  // occupancy target: 2 workgroups of 4 waves per CU
-constexpr int kPrefetch = 2;      // K/V tiles in flight ahead of the one being computed
-constexpr int kNBuf = kPrefetch + 1;
-// k_scales staged in LDS per workgroup (floats).  Sized so that two workgroups per CU still fit in the
-// 160 KiB of LDS next to the K/V buffers: 24 + 24 + 30 KiB (FP8 V) or 24 + 48 + 6 KiB (half V).
-template <int PV> constexpr int ks_lds_floats() { return PV == 0 ? 7680 : 1536; }
-// block-sparse launches (half P.V only) stage the active tiles' ids next to their scales
-constexpr int kSpMaxTiles = 1024;
-// multi-block launches (one workgroup streams up to kMqMaxBlocks query blocks of one head through one
-// K/V pipeline): short key ranges only, so their k_scales and q_scales are staged whole in LDS
-constexpr int kMqMaxTiles = 64;
-// the automatic rule picks multi-block launches below this many key tiles: from 32 tiles on the ping-pong
-// kernel is 4-12 % faster (32760 x 2048 x 12, 8192 x 4096 x 16), at 12 and 16 tiles the two tie
-constexpr int kMqAutoMaxTiles = 24;
-constexpr int kMqMaxBlocks = 64;
-// per-thread K scales: 4 per 64-key tile (one per mma lane-pair class), otherwise 1
-constexpr int ks_per_tile(bool kt) { return kt ? 4 : 1; }
-constexpr int kBK = 64;
-constexpr int kThreads = 256;
-constexpr float kFp8Offset = 8.807f;  // attn_utils.cuh:35 S_FP8_OFFSET
-constexpr float kMInit = -3.0e38f;
-// Lazy-rescale threshold (log2 units), see the softmax below.  After a move of the running max the largest p of
-// the row is 448 / 2^kLazyTau.  Measured against 1 (C4, text cross attention over 512 keys: a few tiles per
-// row, so the max moves on most of them at 1): 8 % faster at 3, RMS error against float64 truth 3.84 % ->
-// 3.90 % (cosine 0.99926 -> 0.99924); C2 / C5 within 1 %, error unchanged.
-constexpr float kLazyTau = 3.0f;
-// The QK accumulators start at kAccBiasBits instead of 0: the int32 result bias + s, read as fp32,
-// is exactly kAccBias + s for |s| < 2^22 (here |s| <= 2^21), so the logits reach the softmax as floats
-// without an int -> float conversion per element; the bias is folded into the exp2 offset.
-constexpr int kAccBiasBits = 0x4B400000;
-constexpr float kAccBias = 12582912.0f;
-// a masked logit as -inf: as int32 (-2^23) it lies below every biased logit, as fp32 its exp2 is 0
-constexpr int kMaskedLogitBits = (int)0xFF800000u;
-
-struct AttnParams {
-  const int8_t* q8;
-  int64_t qsb, qsl, qsh;
-  const int8_t* k8;
-  int64_t ksb, ksl, ksh;
-  const void* v;  // tile-layout V: e4m3 (PV_FP8) or the half dtype, [B, Hkv, D, Lpad]
-  int64_t Lpad;
-  const float* q_scale;  // [B, Hq, nQS]: per 128-row block, per 32-row warp block, or per thread class
-  const float* k_scale;  // [B, Hkv, nKS]: per 64-key tile, or 4 lane-pair classes per tile
-  const float* v_scale;  // [B, Hkv, D] (FP8 P.V only)
-  const float* v_mean;   // [B, Hkv, D] or null: added to the output (smoothed V, FP8 P.V only)
-  void* o;
-  int64_t osb, osl, osh;
-  float* lse;  // [B, Hq, Lq] or null
-  const int32_t* kv_valid;
-  const int8_t* tile_mask;  // block-sparse: [B, Hkv, nQB, nKB] (strides tm_s1 per (b, kv head), tm_s2 per Q block)
-  int64_t tm_s1, tm_s2;
-  float* ws_o;   // split partials [split][B][Hq][Lq][D]
-  float* ws_ml;  // [split][B][Hq][Lq][2]
-  int64_t B, Lq, Lk, Hq, Hkv, nQB, nKB;
-  int64_t nQS, nKS;  // scale entries per (b, h)
-  int qgran;         // QATTN_GRAN_BLOCK / _WARP / _THREAD (q_scale indexing)
-  float q_sm_scale;  // Q quantized per block inside the kernel: the factor multiplied into Q first
-  int qrs;           // log2 of the rows of a warp cell of q_scale: 5 (sm89 tables) or 4 (sm90 tables)
-  int kts;           // key tiles (64 keys) per k_scale block, as a shift: 0 (64-key blocks) or 1 (128)
-  int64_t q_offset;
-  int group;
-  int nsplit;
-  int tiles_per_split;
-  int qpw;       // multi-block launches: query blocks per workgroup
-  int64_t nQC;   // multi-block launches: workgroups per (batch, head)
-  int causal;
-  float qk_mult;
-  // packed variable-length batches (null otherwise): sequence b has query rows cu_q[b] .. cu_q[b + 1] and key
-  // rows cu_k[b] .. cu_k[b + 1] of the packed [1, total, H, D] tensors, its scales start at block cu_qs[b] /
-  // cu_ks[b] of [total_blocks, H] tables, and its V tiles at tile cu_vt[b] of the [1, Hkv, D, Lpad] tile layout
-  const int32_t* cu_q;
-  const int32_t* cu_k;
-  const int32_t* cu_qs;
-  const int32_t* cu_ks;
-  const int32_t* cu_vt;
-  int64_t var_tq, var_tk;  // rows of the packed Q / K tensors
-  // resident-K/V launches: each workgroup takes wb_per_wg consecutive 32-row wave blocks of one head,
-  // n_chunk workgroups per (batch, head)
-  int64_t wb_per_wg;
-  int64_t n_chunk;
-};
-
-__device__ __forceinline__ int64_t xcd_remap(int64_t bid, int64_t n) {
-  const int64_t q = n / 8, r = n % 8;
-  const int64_t xcd = bid % 8, idx = bid / 8;
-  return xcd * q + (xcd < r ? xcd : r) + idx;
-}
-
-// Buffer resource (V#) for raw, unswizzled byte addressing of [base, base + bytes): loads whose offset
-// is at or past `bytes` return zeros instead of touching memory.
-// q_scale entry of query row `row` (< nQB * 128): one per 128-row block, per warp cell of 2^qrs rows, or
-// per row class (rows of a warp cell with equal row % 8: the reference's per-thread grouping).  Clamped
-// to the table: the sm90 tables cover ceil(Lq / 64) * 64 rows, and the rows past that are masked.
-__device__ __forceinline__ int64_t q_scale_index(const AttnParams& p, int64_t row) {
-  const int64_t i = p.qgran == QATTN_GRAN_THREAD ? ((row >> p.qrs) << 3) + (row & 7)
-                    : p.qgran == QATTN_GRAN_WARP ? row >> p.qrs
-                                                 : row >> 7;
-  return i < p.nQS ? i : p.nQS - 1;
-}
-
-// k_scale entry c (< ks) of key tile t in a table of ks entries per k_scale block
-__device__ __forceinline__ int64_t k_scale_index(const AttnParams& p, int64_t t, int c, int ks) {
-  return (t >> p.kts) * ks + c;
-}
-
-__device__ __forceinline__ v4u make_rsrc(const void* base, uint32_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  v4u r;
-  r[0] = __builtin_amdgcn_readfirstlane((uint32_t)a);
-  r[1] = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu);
-  r[2] = __builtin_amdgcn_readfirstlane(bytes);
-  r[3] = 0x00020000u;  // raw buffer, 32-bit data format
-  return r;
-}
-
-// One 16-byte-per-lane buffer -> LDS DMA (buffer_load_dwordx4 ... lds): lane j's 16 bytes, read at
-// base + soff + voff_j, land at LDS address lds + 16 j.  The per-lane offsets are loop-invariant
-// VGPRs and the tile advance is a scalar offset, so issuing a tile costs no VALU work.  Issued through
-// inline asm so the compiler does not treat every later LDS read as a possible alias of the in-flight
-// DMA (it would otherwise put an s_waitcnt vmcnt(0) in front of them and serialise the prefetch);
-// completion is tracked with explicit vmcnt waits instead.
-__device__ __forceinline__ void lds_dma16(uint32_t voff, v4u rsrc, uint32_t soff, uint32_t lds) {
-  asm volatile(
-      "s_mov_b32 m0, %3\n\t"
-      "s_nop 0\n\t"
-      "buffer_load_dwordx4 %0, %1, %2 offen lds"
-      :
-      : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds)
-      : "memory", "m0");
-}
-
-// The 4-byte form (buffer_load_dword ... lds): lane j's dword lands at lds + 4 j.
-__device__ __forceinline__ void lds_dma4(uint32_t voff, v4u rsrc, uint32_t soff, uint32_t lds) {
-  asm volatile(
-      "s_mov_b32 m0, %3\n\t"
-      "s_nop 0\n\t"
-      "buffer_load_dword %0, %1, %2 offen lds"
-      :
-      : "v"(voff), "s"(rsrc), "s"(soff), "s"(lds)
-      : "memory", "m0");
-}
-
-// two floats -> two round-to-nearest-even halves (bf16: v_cvt_pk_bf16_f32), low word first
-template <bool IS_FP16>
-__device__ __forceinline__ uint32_t pack_half2(float a, float b) {
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-  uint32_t r;
-  if constexpr (IS_FP16) {
-    const h2 v = __builtin_convertvector(f2{a, b}, h2);
-    __builtin_memcpy(&r, &v, 4);
-  } else {
-    const b2 v = __builtin_convertvector(f2{a, b}, b2);
-    __builtin_memcpy(&r, &v, 4);
-  }
-  return r;
-}
-
-// One output value: O / l * v_scale (+ v_mean for smoothed V), rounded after every operation (no fused
-// multiply-add), so that every kernel and the split combine produce the same bits.
-template <bool ADD_MEAN>
-__device__ __forceinline__ float epilogue_value(float o, float inv_l, float sc, float vm) {
-#pragma clang fp contract(off)
-  const float x = o * inv_l * sc;
-  if constexpr (ADD_MEAN) return x + vm;
-  else return x;
-}
-
-// P of the FP8 P.V without an exponential.  u = 8 (x - kPLinShift) + 56, rounded to an integer k (RNE) and
-// clamped to [0, 255] by v_cvt_pk_u8_f32, is read as the e4m3 byte of P: exponent field floor(y) + 7 and
-// mantissa round(8 frac(y)) for y = x - kPLinShift, i.e. 2^floor(y) (1 + frac(y)) rounded to the e4m3 grid.
-// This is Schraudolph's exponential ("A fast, compact approximation of the exponential function", Neural
-// Computation 11, 1999: the argument scaled into the exponent field, the mantissa interpolating 2^f
-// linearly) at e4m3 precision.  (1 + f) / 2^f lies in [1, 1.0861] with mean 1.040685 over f in [0, 1); the
-// shift kPLinShift = log2(1.040685) removes that mean, so P is unbiased against exp2(x) on average and within
-// -4.0 % / +4.4 % of it before the e4m3 rounding (RMS 3.15 % relative including the rounding, against
-// 2.66 % for exp2(x) rounded to e4m3).  x <= 8.807 (the FP8 offset) gives k <= 126 (448); k = 127 would
-// be NaN.  x < -7 gives 0; k < 8 are the e4m3 subnormals (P < 2^-6, linear in k).  Costs one full-rate
-// conversion per element against a quarter-rate v_exp_f32 plus half a quarter-rate fp8 pack (measured:
-// 10.3 against 23.9 cycles per element with the fma, two waves per SIMD).
-constexpr float kPLinShift = 0.057539f;
-constexpr float kPLinBias = 56.0f - 8.0f * kPLinShift;  // e4m3 exponent bias 7, in units of 1/8
-__device__ __forceinline__ int p_e4m3_x4(float u0, float u1, float u2, float u3) {
-  uint32_t t = __builtin_amdgcn_cvt_pk_u8_f32(u0, 0, 0u);
-  t = __builtin_amdgcn_cvt_pk_u8_f32(u1, 1, t);
-  t = __builtin_amdgcn_cvt_pk_u8_f32(u2, 2, t);
-  return (int)__builtin_amdgcn_cvt_pk_u8_f32(u3, 3, t);
-}
-
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
-}
-
-// Row sums of P on the matrix pipe (FP8 P.V): one v_mfma_scale_f32_16x16x128_f8f6f4 per tile, D += A . B with
-// B the e4m3 P^T operand of the P.V MFMA read in the 16 x 16 x 128 layout (lane l feeds column l % 16; its 32
-// bytes are, in the 32 x 32 layout, 32 keys of query l % 32, so columns collect query c from lanes c and
-// c + 32 and query c + 16 from lanes c + 16 and c + 48) and A an fp4 (e2m1) selector.  In this layout fp4
-// nibbles 0-15 of A lane 16 a + r meet bytes 0-15 (a = 0, 1: of B lane groups 0, 2) or 16-31 (a = 2, 3) of
-// lane groups 0 / 2, and nibbles 16-31 the same bytes of lane groups 1 / 3 (measured on gfx950).  So row 0 of
-// A is 1.0 on nibbles 0-15 of lanes 0, 16, 32, 48 and row 1 on nibbles 16-31 of lanes 1, 17, 33, 49: row 0
-// of the result is the running sum l of queries 0..15, row 1 that of queries 16..31, and lane c < 16 holds
-// them in elements 0 and 1.  l is thus the sum of the e4m3-rounded P (the reference's accumulate_d sums p
-// before rounding; the difference is the mean FP8 rounding error of P, far inside the attention tolerance);
-// the row sums leave the softmax's VALU stream, and the MFMA costs half the 32 x 32 x 64 form.
-__device__ __forceinline__ v8i row_sum_selector() {
-  const int r = threadIdx.x & 15;
-  const int lo = r == 0 ? 0x22222222 : 0, hi = r == 1 ? 0x22222222 : 0;
-  return v8i{lo, lo, hi, hi, 0, 0, 0, 0};
-}
-__device__ __forceinline__ v4f row_sum_mfma(const v4f& acc, const v8i& pf, const v8i& sel) {
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(sel, pf, acc, 4, 0, 0, 0, 0, 0);
-}
-// online-softmax rescale of the row sums: element 0 of lane c belongs to query c (the lane's own), element 1
-// to query c + 16, whose factor lane c + 16 holds
-__device__ __forceinline__ void row_sum_rescale(v4f& acc, float alpha) {
-  const int lane = threadIdx.x & 63;
-  const float a_hi = __int_as_float(__builtin_amdgcn_ds_bpermute(((lane & 15) + 16) * 4, __float_as_int(alpha)));
-  acc[0] *= alpha;
-  acc[1] *= a_hi;
-}
-// the row sum of query lq (lanes lq and lq + 32 both get it)
-__device__ __forceinline__ float row_sum_value(const v4f& acc, int lq) {
-  const int src = (lq & 15) * 4;
-  const float v0 = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(acc[0])));
-  const float v1 = __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(acc[1])));
-  return lq < 16 ? v0 : v1;
-}
-
-// P.V flavours: e4m3 P x e4m3 V (the reference's fp8 kernel, with the 8.807 offset and v_scale), or
-// P rounded to the half dtype of V x V as given (the Triton / SAGE_ATTN_2_8_16 style), fp32 accumulation.
-enum PvKind { PV_FP8 = 0, PV_BF16 = 1, PV_FP16 = 2 };
-
-template <bool IS_FP16_OUT, bool SPLIT, int PV, bool KT, bool SP = false, bool MQ = false>
+template <bool IS_FP16_OUT, bool SPLIT, bool KT, bool MQ = false>
 __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(AttnParams p) {
-  static_assert(!SP || (PV != PV_FP8 && !KT), "block-sparse launches use half P.V and per-block scales");
-  static_assert(!MQ || (PV == PV_FP8 && !SPLIT && !SP), "multi-block launches: FP8 P.V, no split, dense");
+  static_assert(!MQ || !SPLIT, "multi-block launches: no split");
   constexpr int KS = ks_per_tile(KT);
-  constexpr int kVBytes = PV == PV_FP8 ? 1 : 2;    // bytes per V element
-  constexpr int kVDma = 2 * kVBytes;                // V DMA instructions per wave per tile
-  constexpr float kOffset = PV == PV_FP8 ? kFp8Offset : 0.f;
   __shared__ __align__(16) uint8_t lds_k[kNBuf][kBK * kD];
-  __shared__ __align__(16) uint8_t lds_v[kNBuf][kD * kBK * kVBytes];
-  __shared__ float lds_ks[SP ? kSpMaxTiles : MQ ? kMqMaxTiles * 4 : ks_lds_floats<PV>()];  // k_scales of its key tiles
+  __shared__ __align__(16) uint8_t lds_v[kNBuf][kD * kBK];
+  __shared__ float lds_ks[MQ ? kMqMaxTiles * 4 : kKsLdsFloats];  // k_scales of its key tiles
   // multi-block launches: a wave-private 4 KiB region per wave that receives the next query block's Q
   // rows by DMA and then stages the finished block's O rows; and the q_scales of all its blocks
   __shared__ __align__(16) uint8_t lds_qo[MQ ? 4 * 4096 : 16];
   __shared__ float lds_qs[MQ ? kMqMaxBlocks * 32 : 1];
-  __shared__ __align__(16) float lds_vs[PV == PV_FP8 ? kD : 4];  // v_scale of this head (epilogue)
-  __shared__ __align__(16) float lds_vm[PV == PV_FP8 ? kD : 4];  // v_mean of this head (smoothed V)
-  __shared__ int16_t lds_tid[SP ? kSpMaxTiles : 1];                  // block-sparse: ids of the active tiles
-  __shared__ int lds_nact;
+  __shared__ __align__(16) float lds_vs[kD];  // v_scale of this head (epilogue)
+  __shared__ __align__(16) float lds_vm[kD];  // v_mean of this head (smoothed V)
 
   const int64_t tile_id = xcd_remap(blockIdx.x, gridDim.x);
   int64_t qb, qb_end;  // query blocks [qb, qb_end) of this workgroup
@@ -314,30 +71,12 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
   const int64_t b = rest / p.Hq;
   const int64_t hk = h / p.group;
 
-  // the batch entry's view: a dense batch, or one sequence of a packed variable-length batch
-  int64_t Lq = p.Lq, Lk = p.Lk;
+  const int64_t Lq = p.Lq, Lk = p.Lk;
   const int8_t* q8b = p.q8 + b * p.qsb;
   const int8_t* k8b = p.k8 + b * p.ksb;
-  int64_t vcol0 = 0;  // first key column of this entry in the V tile layout
   const float* qs_tab = p.q_scale + (b * p.Hq + h) * p.nQS;
-  const float* ks_tab = p.k_scale + (b * p.Hkv + hk) * p.nKS;
-  int64_t qs_stride = 1, ks_stride = 1;
+  const float* ks_ptr = p.k_scale + (b * p.Hkv + hk) * p.nKS;
   uint16_t* ob = static_cast<uint16_t*>(p.o) + b * p.osb;
-  if (p.cu_q) {
-    int64_t q0, k0s;
-    varlen_range(p.cu_q, b, p.var_tq, p.Lq, q0, Lq);
-    varlen_range(p.cu_k, b, p.var_tk, p.Lk, k0s, Lk);
-    // (a V tile range past Lpad, from a too small Lpad, leaves the sequence's rows untouched)
-    if (qb * kBQ >= Lq || Lk <= 0 || ((int64_t)p.cu_vt[b] + (Lk + kBK - 1) / kBK) * kBK > p.Lpad) return;
-    q8b = p.q8 + q0 * p.qsl;
-    k8b = p.k8 + k0s * p.ksl;
-    vcol0 = (int64_t)p.cu_vt[b] * kBK;
-    qs_tab = p.q_scale + (int64_t)p.cu_qs[b] * p.Hq + h;
-    ks_tab = p.k_scale + (int64_t)p.cu_ks[b] * p.Hkv + hk;
-    qs_stride = p.Hq;
-    ks_stride = p.Hkv;
-    ob = static_cast<uint16_t*>(p.o) + q0 * p.osl;
-  }
 
   const int tid = threadIdx.x;
   // (wave index in a scalar register, so that every per-wave quantity and branch stays scalar)
@@ -349,34 +88,8 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
   if (p.kv_valid) kv_end = min(kv_end, (int64_t)p.kv_valid[b]);
   if (p.causal) kv_end = min(kv_end, q_first + kBQ + p.q_offset);
   const int64_t n_tiles = kv_end > 0 ? (kv_end + kBK - 1) / kBK : 0;
-  // The loop runs over "slots": every key tile (dense), or the tiles the block-sparse mask keeps for
-  // this query block, in key order (sparse_int8_attn.py:57-58 skips a tile whose k_block_id is 0).
-  int64_t t_begin = SPLIT ? (int64_t)split * p.tiles_per_split : 0;
-  int64_t n_slots = n_tiles;
-  if constexpr (SP) {
-    if (w == 0) {  // wave 0 compacts the mask row with ballots; only this split's slots are stored
-      const int8_t* mrow = p.tile_mask + (b * p.Hkv + hk) * p.tm_s1 + qb * p.tm_s2;
-      int64_t cnt = 0;
-      for (int64_t base = 0; base < n_tiles; base += 64) {
-        const int64_t t = base + lane;
-        const bool act = t < n_tiles && mrow[t] != 0;
-        const uint64_t bal = __ballot(act);
-        const int64_t slot = cnt + __popcll(bal & ((1ull << lane) - 1ull));
-        if (act && slot >= t_begin && slot < t_begin + (SPLIT ? p.tiles_per_split : kSpMaxTiles))
-          lds_tid[slot - t_begin] = (int16_t)t;
-        cnt += __popcll(bal);
-      }
-      if (lane == 0) lds_nact = (int)cnt;
-    }
-    __syncthreads();
-    n_slots = lds_nact;
-  }
-  const int64_t t_end = SPLIT ? min(n_slots, t_begin + p.tiles_per_split) : n_slots;
-  // key tile of slot t (wave-uniform)
-  auto tile_of = [&](int64_t t) -> int64_t {
-    if constexpr (SP) return __builtin_amdgcn_readfirstlane((int)lds_tid[t - t_begin]);
-    else return t;
-  };
+  const int64_t t_begin = SPLIT ? (int64_t)split * p.tiles_per_split : 0;
+  const int64_t t_end = SPLIT ? min(n_tiles, t_begin + p.tiles_per_split) : n_tiles;
 
   // Q fragment (B operand of S^T = K.Q^T): lane owns query row lq of this wave, bytes
   // d = 32*m + 16*hf .. +16 for m = 0..3
@@ -409,41 +122,37 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
     for (int m = 0; m < 4; m++) asm volatile("" ::"v"(qf[m]));
   }
   // q_scale of this lane's query row
-  float qs = qs_tab[q_scale_index(p, qb * kBQ + w * 32 + lq) * qs_stride] * p.qk_mult;
+  float qs = qs_tab[q_scale_index(p, qb * kBQ + w * 32 + lq)] * p.qk_mult;
   // q_scale entries per query block, and this lane's entry within its block
   const int qs_per = p.qgran == QATTN_GRAN_THREAD ? (kBQ >> p.qrs) * 8 : p.qgran == QATTN_GRAN_WARP ? kBQ >> p.qrs : 1;
   const int qs_sub = p.qgran == QATTN_GRAN_BLOCK ? 0 : (int)q_scale_index(p, w * 32 + lq);
-  const float* ks_ptr = ks_tab;
 
   // global -> LDS copies go through the LDS-DMA path (buffer_load_dwordx4 ... lds): lane j of a wave
   // writes the 16 bytes at LDS slot (wave base + 16 j).  The tiles are fragment-major: 1 KiB block f holds
   // MFMA operand fragment f of all 64 lanes (lane l at 16 l), so a lane reads its fragments at one base
   // address plus constant offsets, each read a contiguous, conflict-free 1 KiB:
   //   K block j (0..7): lane l gets K row (j & 1) * 32 + l % 32, bytes 16 (2 (j >> 1) + l / 32) .. + 16
-  //   FP8 V block 2 dblk + h: lane l gets V^T row dblk * 32 + l % 32, bytes 16 (2 (l / 32) + h) .. + 16
-  //   half V block 4 dblk + c: lane l gets V^T row dblk * 32 + l % 32, bytes 16 (4 (l / 32) + c) .. + 16
-  // DMA instruction i of wave w fills block 4 i + w.  Each wave moves 2 x 1 KiB of K and kVDma x 1 KiB of V
+  //   V block 2 dblk + h: lane l gets V^T row dblk * 32 + l % 32, bytes 16 (2 (l / 32) + h) .. + 16
+  // DMA instruction i of wave w fills block 4 i + w.  Each wave moves 2 x 1 KiB of K and 2 x 1 KiB of V
   // per tile; no VGPRs are spent on staging.
   // The K resource of a tile starts at the tile's first row, so K rows at or past Lk fall outside its
   // range and arrive as zeros (masked anyway) without being read (the range check covers the
   // per-lane offset, not the scalar one).
   const int8_t* kbase = k8b + hk * p.ksh;
-  const uint8_t* vbase = static_cast<const uint8_t*>(p.v) + ((p.cu_q ? 0 : b) * p.Hkv + hk) * (int64_t)kD * p.Lpad * kVBytes +
-                         vcol0 * kVBytes;
+  const uint8_t* vbase = static_cast<const uint8_t*>(p.v) + (b * p.Hkv + hk) * (int64_t)kD * p.Lpad;
   const int64_t kbytes = (Lk - 1) * p.ksl + kD;
-  const v4u vrsrc = make_rsrc(vbase, (uint32_t)(((int64_t)kD * p.Lpad - vcol0) * kVBytes));
+  const v4u vrsrc = make_rsrc(vbase, (uint32_t)((int64_t)kD * p.Lpad));
   // per-lane byte offsets relative to the tile start (first K row / first V column)
-  uint32_t koff[2], voff[kVDma];
+  uint32_t koff[2], voff[2];
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     const int j = i * 4 + w;
     koff[i] = (uint32_t)(((j & 1) * 32 + lq) * p.ksl + (2 * (j >> 1) + hf) * 16);
   }
 #pragma unroll
-  for (int i = 0; i < kVDma; i++) {
+  for (int i = 0; i < 2; i++) {
     const int f = i * 4 + w;
-    if constexpr (PV == PV_FP8) voff[i] = (uint32_t)(((f >> 1) * 32 + lq) * p.Lpad + (2 * hf + (f & 1)) * 16);
-    else voff[i] = (uint32_t)(((f >> 2) * 32 + lq) * p.Lpad * 2 + (4 * hf + (f & 3)) * 16);
+    voff[i] = (uint32_t)(((f >> 1) * 32 + lq) * p.Lpad + (2 * hf + (f & 1)) * 16);
   }
   const int64_t k_step = kBK * p.ksl;
   const uint32_t lds_k0 = lds_addr(&lds_k[0][0]) + __builtin_amdgcn_readfirstlane(w) * 1024;
@@ -451,12 +160,12 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
   auto dma_tile = [&](int64_t t, int buf) {
     const int64_t kso = t * k_step;
     const v4u krsrc = make_rsrc(kbase + kso, (uint32_t)(kbytes - kso));
-    const uint32_t vso = (uint32_t)t * (kBK * kVBytes);
-    const uint32_t kl = lds_k0 + buf * (kBK * kD), vl = lds_v0 + buf * (kD * kBK * kVBytes);
+    const uint32_t vso = (uint32_t)t * kBK;
+    const uint32_t kl = lds_k0 + buf * (kBK * kD), vl = lds_v0 + buf * (kD * kBK);
 #pragma unroll
     for (int i = 0; i < 2; i++) lds_dma16(koff[i], krsrc, 0, kl + i * 4096);
 #pragma unroll
-    for (int i = 0; i < kVDma; i++) lds_dma16(voff[i], vrsrc, vso, vl + i * 4096);
+    for (int i = 0; i < 2; i++) lds_dma16(voff[i], vrsrc, vso, vl + i * 4096);
   };
   // multi-block launches: the wave's 32 rows of the next query block go by DMA into its region of
   // lds_qo, in the stage layout (LDS slot (r, c') receives global chunk c' ^ (r & 7)); the resource
@@ -483,8 +192,8 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
   for (int i = 0; i < 4; i++)
 #pragma unroll
     for (int r = 0; r < 16; r++) o[i][r] = 0.f;
-  float m_run = kMInit, l_run = 0.f;
-  v4f lacc = {0.f, 0.f, 0.f, 0.f};  // FP8 P.V: row sums of P on the matrix pipe (row_sum_mfma)
+  float m_run = kMInit;
+  v4f lacc = {0.f, 0.f, 0.f, 0.f};  // row sums of P on the matrix pipe (row_sum_mfma)
   const v8i rs_sel = row_sum_selector();
   v16i kbias;
 #pragma unroll
@@ -495,12 +204,8 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
   // iteration t - 1.  The k_scales of all tiles are staged in LDS once, so the only VMEM traffic in the
   // loop is the 4 DMA instructions per tile and the vmcnt accounting below is exact.
   __syncthreads();  // every wave has its Q fragments out of the LDS stage before the DMA reuses it
-  if constexpr (SP) {
-    for (int64_t i = tid; i < t_end - t_begin; i += kThreads) lds_ks[i] = ks_ptr[lds_tid[i] * ks_stride];
-  } else {
-    for (int64_t i = tid; i < (t_end - t_begin) * KS; i += kThreads) lds_ks[i] = ks_ptr[k_scale_index(p, t_begin + i / KS, i % KS, KS) * ks_stride];
-  }
-  if constexpr (PV == PV_FP8 && !SPLIT)
+  for (int64_t i = tid; i < (t_end - t_begin) * KS; i += kThreads) lds_ks[i] = ks_ptr[k_scale_index(p, t_begin + i / KS, i % KS, KS)];
+  if constexpr (!SPLIT)
     if (tid < kD) {
       lds_vs[tid] = p.v_scale[(b * p.Hkv + hk) * kD + tid];
       lds_vm[tid] = p.v_mean ? p.v_mean[(b * p.Hkv + hk) * kD + tid] : 0.f;
@@ -516,19 +221,13 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
   const int64_t total = MQ ? (qb_end - qb0) * n_kt : n_kt;
 #pragma unroll
   for (int d = 0; d < kPrefetch; d++)
-    if (d < total) dma_tile(tile_of(t_begin + (MQ ? d % n_kt : d)), d);
+    if (d < total) dma_tile(t_begin + (MQ ? d % n_kt : d), d);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 
   // ---- epilogue of the current query block: O / l * v_scale out through the wave's LDS stage ----
   auto finish = [&]() {
-    float l_tot;
-    if constexpr (PV == PV_FP8) {
-      l_tot = row_sum_value(lacc, lq);
-    } else {
-      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
-      l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-    }
+    const float l_tot = row_sum_value(lacc, lq);
     if (SPLIT) {
       if (qrow >= Lq) return;
       const int64_t row = (((int64_t)split * p.B + b) * p.Hq + h) * p.Lq + qrow;
@@ -562,7 +261,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
 #pragma unroll
         for (int g = 0; g < 4; g++) {
           const int d = dblk * 32 + g * 8 + hf * 4;
-          const v4f sc = PV == PV_FP8 ? *reinterpret_cast<const v4f*>(&lds_vs[d]) : v4f{1.f, 1.f, 1.f, 1.f};
+          const v4f sc = *reinterpret_cast<const v4f*>(&lds_vs[d]);
           float f[4];
           const v4f vm = kMean ? *reinterpret_cast<const v4f*>(&lds_vm[d]) : v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -583,7 +282,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     };
-    if (PV == PV_FP8 && p.v_mean) store(std::true_type{});
+    if (p.v_mean) store(std::true_type{});
     else store(std::false_type{});
     if (p.lse && hf == 0 && qrow < Lq)
       p.lse[(b * p.Hq + h) * p.Lq + qrow] = l_tot > 0.f ? __builtin_log2f(l_tot) + m_run : -INFINITY;
@@ -599,7 +298,6 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
 #pragma unroll
       for (int r = 0; r < 16; r++) o[i][r] = 0.f;
     m_run = kMInit;
-    l_run = 0.f;
     lacc = v4f{0.f, 0.f, 0.f, 0.f};
   };
 
@@ -612,7 +310,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
     if constexpr (MQ)
       if (t == 0 && qb + 1 < qb_end) dma_q(qb + 1);
     if (issue) {
-      dma_tile(tile_of(pt), buf == 0 ? kNBuf - 1 : buf - 1);
+      dma_tile(pt, buf == 0 ? kNBuf - 1 : buf - 1);
       pt++;
       if (MQ && pt == t_end) pt = t_begin;
     }
@@ -646,7 +344,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
     }
 
     // ---- masking (tail tile, key padding, causal diagonal) ----
-    const int64_t k0 = tile_of(t) * kBK;
+    const int64_t k0 = t * kBK;
     const bool masked = (k0 + kBK > kv_end) || (p.causal && k0 + kBK - 1 > wrow0 + p.q_offset);
     if (masked) {
       // element r of block kb holds key k0 + c + 4 hf with c = 32 kb + 8 (r / 4) + r % 4; it is masked
@@ -678,7 +376,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
       // <= 2^8.807 = 448 (the e4m3 maximum), so the FP8 range is honoured while the O rescale (64
       // multiplies per lane) is skipped on almost every tile.  A row whose keys in this tile are all
       // masked never moves m.
-      m_tile = mx == INT32_MIN ? kMInit : fmaf(__int_as_float(mx), cs_a, -fmaf(kAccBias, cs_a, kOffset - kLazyTau));
+      m_tile = mx == INT32_MIN ? kMInit : fmaf(__int_as_float(mx), cs_a, -fmaf(kAccBias, cs_a, kFp8Offset - kLazyTau));
     } else {  // two scale classes per lane: max per class, scaled, then across the lane pair
       int ma = INT32_MIN, mb = INT32_MIN;
 #pragma unroll
@@ -688,8 +386,8 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
           if ((r & 3) < 2) ma = max(ma, s[kb][r]);
           else mb = max(mb, s[kb][r]);
         }
-      const float fa = ma == INT32_MIN ? kMInit : fmaf(__int_as_float(ma), cs_a, -fmaf(kAccBias, cs_a, kOffset - kLazyTau));
-      const float fb = mb == INT32_MIN ? kMInit : fmaf(__int_as_float(mb), cs_b, -fmaf(kAccBias, cs_b, kOffset - kLazyTau));
+      const float fa = ma == INT32_MIN ? kMInit : fmaf(__int_as_float(ma), cs_a, -fmaf(kAccBias, cs_a, kFp8Offset - kLazyTau));
+      const float fb = mb == INT32_MIN ? kMInit : fmaf(__int_as_float(mb), cs_b, -fmaf(kAccBias, cs_b, kFp8Offset - kLazyTau));
       float mt = fmaxf(fa, fb);
       const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
       m_tile = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
@@ -698,100 +396,50 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
     if (__any(grow)) {
       const float m_new = grow ? m_tile : m_run;
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-      l_run *= alpha;
 #pragma unroll
       for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int r = 0; r < 16; r++) o[i][r] *= alpha;
-      if constexpr (PV == PV_FP8) row_sum_rescale(lacc, alpha);
+      row_sum_rescale(lacc, alpha);
       m_run = m_new;
     }
-    const float nc_a = -fmaf(kAccBias, cs_a, m_run), nc_b = -fmaf(kAccBias, cs_b, m_run);
-    // p = exp2(s * cs - m); masked logits (INT32_MIN) become p = 0 exactly (the sentinel times a tiny
-    // block scale is not necessarily very negative)
-    auto p4 = [&](int j, float (&pv)[4], auto mk) {
-      const int kb = j >> 2, r0 = (j & 3) * 4;
+    v8i pf;  // P^T as the e4m3 B operand: byte s of the lane = slot s = 16 kb + r
+    // u = 8 (s * cs - m - kPLinShift) + 56 (p_e4m3_x4); masked logits give u = -1, P = 0
+    const float cs8_a = 8.0f * cs_a, cs8_b = 8.0f * cs_b;
+    const float nu_a = fmaf(-8.0f, fmaf(kAccBias, cs_a, m_run), kPLinBias);
+    const float nu_b = fmaf(-8.0f, fmaf(kAccBias, cs_b, m_run), kPLinBias);
+    auto body = [&](auto mk) {
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int sv = s[kb][r0 + e];
-        pv[e] = __builtin_amdgcn_exp2f(fmaf(__int_as_float(sv), e < 2 ? cs_a : cs_b, e < 2 ? nc_a : nc_b));
-        if constexpr (decltype(mk)::value) pv[e] = sv == INT32_MIN ? 0.f : pv[e];
+      for (int j = 0; j < 8; j++) {
+        const int kb = j >> 2, r0 = (j & 3) * 4;
+        float u[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int sv = s[kb][r0 + e];
+          u[e] = fmaf(__int_as_float(sv), e < 2 ? cs8_a : cs8_b, e < 2 ? nu_a : nu_b);
+          if constexpr (decltype(mk)::value) u[e] = sv == INT32_MIN ? -1.f : u[e];
+        }
+        pf[j] = p_e4m3_x4(u[0], u[1], u[2], u[3]);
       }
     };
-    if constexpr (PV == PV_FP8) {
-      v8i pf;  // P^T as the e4m3 B operand: byte s of the lane = slot s = 16 kb + r
-      // u = 8 (s * cs - m - kPLinShift) + 56 (p_e4m3_x4); masked logits give u = -1, P = 0
-      const float cs8_a = 8.0f * cs_a, cs8_b = 8.0f * cs_b;
-      const float nu_a = fmaf(-8.0f, fmaf(kAccBias, cs_a, m_run), kPLinBias);
-      const float nu_b = fmaf(-8.0f, fmaf(kAccBias, cs_b, m_run), kPLinBias);
-      auto body = [&](auto mk) {
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-          const int kb = j >> 2, r0 = (j & 3) * 4;
-          float u[4];
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const int sv = s[kb][r0 + e];
-            u[e] = fmaf(__int_as_float(sv), e < 2 ? cs8_a : cs8_b, e < 2 ? nu_a : nu_b);
-            if constexpr (decltype(mk)::value) u[e] = sv == INT32_MIN ? -1.f : u[e];
-          }
-          pf[j] = p_e4m3_x4(u[0], u[1], u[2], u[3]);
-        }
-      };
-      if (masked) body(std::true_type{});
-      else body(std::false_type{});
+    if (masked) body(std::true_type{});
+    else body(std::false_type{});
 
-      // ---- O^T += V^T . P^T (FP8 MFMA, K = 64 keys) ----
-      v8i vf[4];
+    // ---- O^T += V^T . P^T (FP8 MFMA, K = 64 keys) ----
+    v8i vf[4];
 #pragma unroll
-      for (int dblk = 0; dblk < 4; dblk++) {
-        const v4i a0 = *reinterpret_cast<const v4i*>(&lds_v[buf][(2 * dblk) * 1024 + lane * 16]);
-        const v4i a1 = *reinterpret_cast<const v4i*>(&lds_v[buf][(2 * dblk + 1) * 1024 + lane * 16]);
-        vf[dblk] = v8i{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-      }
-#pragma unroll
-      for (int dblk = 0; dblk < 4; dblk++)
-        o[dblk] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf[dblk], pf, o[dblk], 0, 0, 0, 0, 0, 0);
-      lacc = row_sum_mfma(lacc, pf, rs_sel);
-    } else {
-      // P^T in the half dtype: chunk c (16 keys of the MFMA's K dimension) = slots 8c .. 8c+7
-      typedef __attribute__((ext_vector_type(8))) __bf16 v8bf;
-      typedef __attribute__((ext_vector_type(8))) _Float16 v8h;
-      using HV = std::conditional_t<PV == PV_BF16, v8bf, v8h>;
-      using HS = std::conditional_t<PV == PV_BF16, __bf16, _Float16>;
-      HV ph[4];
-      auto body = [&](auto mk) {
-        float lsum = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-          float pv[4];
-          p4(j, pv, mk);
-          lsum += (pv[0] + pv[1]) + (pv[2] + pv[3]);
-#pragma unroll
-          for (int e = 0; e < 4; e++) ph[j >> 1][(j & 1) * 4 + e] = (HS)pv[e];  // RNE
-        }
-        l_run += lsum;
-      };
-      if (masked) body(std::true_type{});
-      else body(std::false_type{});
-
-      // ---- O^T += V^T . P^T (half MFMA 32x32x16, 4 K-chunks per 32-channel block) ----
-#pragma unroll
-      for (int dblk = 0; dblk < 4; dblk++) {
-        HV vf[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-          vf[c] = *reinterpret_cast<const HV*>(&lds_v[buf][(4 * dblk + c) * 1024 + lane * 16]);
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          if constexpr (PV == PV_BF16) o[dblk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[c], ph[c], o[dblk], 0, 0, 0);
-          else o[dblk] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[c], ph[c], o[dblk], 0, 0, 0);
-        }
-      }
+    for (int dblk = 0; dblk < 4; dblk++) {
+      const v4i a0 = *reinterpret_cast<const v4i*>(&lds_v[buf][(2 * dblk) * 1024 + lane * 16]);
+      const v4i a1 = *reinterpret_cast<const v4i*>(&lds_v[buf][(2 * dblk + 1) * 1024 + lane * 16]);
+      vf[dblk] = v8i{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
     }
+#pragma unroll
+    for (int dblk = 0; dblk < 4; dblk++)
+      o[dblk] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf[dblk], pf, o[dblk], 0, 0, 0, 0, 0, 0);
+    lacc = row_sum_mfma(lacc, pf, rs_sel);
 
     // tile t+1 must have landed; the DMAs of the tiles after it may stay in flight
-    if (issue) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((2 + kVDma) * (kPrefetch - 1)) : "memory");
+    if (issue) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (kPrefetch - 1)) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     buf = buf + 1 == kNBuf ? 0 : buf + 1;
@@ -848,112 +496,6 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void qattn_fwd_kernel(Attn
 constexpr int kPPThreads = 512;
 constexpr int kPPNBuf = 4;
 
-// QF: Q as int8 with its scale table (0), or Q in the output's half type quantized inside the attention
-// kernel: with the per-thread classes of the Triton quantizer (QF_THREAD: rows with equal row % 8 of a wave's
-// 32 share a scale, round half away from x / scale), the per-warp blocks of the CUDA one (QF_WARP: a wave's
-// 32 rows share a scale, RNE of x * 127 / amax), or its per-block form (QF_BLOCK: the
-// 128 rows of a query block, held by four waves of one workgroup, share a scale, x multiplied by
-// sm_scale * log2(e) first) -- the codes and
-// scales of per_thread_int8 / per_warp_int8 / per_block_int8 bit for bit, without writing int8 Q out and
-// reading it back.
-constexpr int QF_INT8 = 0, QF_THREAD = 1, QF_WARP = 2, QF_BLOCK = 3;
-
-// Lane (lq, hf) of a wave whose 32 query rows are lq = lane % 32: the raw half words of its row (row
-// pointer rowp; zeros when !valid) at 32 m + 16 hf .. + 16, m < NQF.
-template <int NQF>
-__device__ __forceinline__ void quant_q_raw(const uint16_t* rowp, bool valid, int hf, v4u (&r)[NQF][2]) {
-#pragma unroll
-  for (int m = 0; m < NQF; m++) {
-    r[m][0] = r[m][1] = v4u{0, 0, 0, 0};
-    if (valid) {
-      r[m][0] = *reinterpret_cast<const v4u*>(rowp + m * 32 + hf * 16);
-      r[m][1] = *reinterpret_cast<const v4u*>(rowp + m * 32 + hf * 16 + 8);
-    }
-  }
-}
-
-// Those values as fp32, times mul when MUL.
-template <bool IS_FP16, int NQF, bool MUL>
-__device__ __forceinline__ void quant_q_unpack(const v4u (&r)[NQF][2], float mul, float (&x)[NQF][16]) {
-#pragma unroll
-  for (int m = 0; m < NQF; m++) {
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      x[m][2 * e] = half_to_f32<IS_FP16>((uint16_t)(r[m][0][e] & 0xffffu));
-      x[m][2 * e + 1] = half_to_f32<IS_FP16>((uint16_t)(r[m][0][e] >> 16));
-      x[m][8 + 2 * e] = half_to_f32<IS_FP16>((uint16_t)(r[m][1][e] & 0xffffu));
-      x[m][8 + 2 * e + 1] = half_to_f32<IS_FP16>((uint16_t)(r[m][1][e] >> 16));
-    }
-    if constexpr (MUL) {
-#pragma unroll
-      for (int e = 0; e < 16; e++) x[m][e] = x[m][e] * mul;
-    }
-  }
-}
-
-// The |x| maximum over the lane's scale group within the wave (per-thread class: lanes lq ^ 8, lq ^ 16 and
-// the other half-row; per-warp / per-block: all 64 lanes, from the CUDA quantizer's 1e-7 floor).
-template <int QF, int NQF>
-__device__ __forceinline__ float quant_q_amax(const float (&x)[NQF][16]) {
-  float am = QF == QF_THREAD ? 0.f : 0.0000001f;
-#pragma unroll
-  for (int m = 0; m < NQF; m++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) am = fmaxf(am, fabsf(x[m][e]));
-  if constexpr (QF != QF_THREAD) {
-    am = fmaxf(am, __shfl_xor(am, 1, 64));
-    am = fmaxf(am, __shfl_xor(am, 2, 64));
-    am = fmaxf(am, __shfl_xor(am, 4, 64));
-  }
-  am = fmaxf(am, __shfl_xor(am, 8, 64));
-  am = fmaxf(am, __shfl_xor(am, 16, 64));
-  am = fmaxf(am, __shfl_xor(am, 32, 64));
-  return am;
-}
-
-// The three steps at once: the lane's values x (times mul when MUL) and their group maximum.
-template <bool IS_FP16, int QF, int NQF, bool MUL = false>
-__device__ __forceinline__ float quant_q_load(const uint16_t* rowp, bool valid, int hf, float mul, float (&x)[NQF][16]) {
-  v4u r[NQF][2];
-  quant_q_raw<NQF>(rowp, valid, hf, r);
-  quant_q_unpack<IS_FP16, NQF, MUL>(r, mul, x);
-  return quant_q_amax<QF, NQF>(x);
-}
-
-// The scale of a group with |x| maximum am (returned) and the int8 codes as the MFMA B fragments qf.
-template <int QF, int NQF>
-__device__ __forceinline__ float quant_q_codes(const float (&x)[NQF][16], float am, v4i (&qf)[NQF]) {
-  constexpr bool TRITON = QF == QF_THREAD;
-  const float sc = TRITON ? quant_scale_triton(am) : quant_scale_cuda(am);
-  const float iv = TRITON ? refined_rcp(sc) : quant_recip_cuda(am);
-#pragma unroll
-  for (int m = 0; m < NQF; m++) {
-    int c[16];
-#pragma unroll
-    for (int e = 0; e < 16; e++) c[e] = TRITON ? quant_code_triton(x[m][e], sc, iv) : quant_code_cuda(x[m][e], iv);
-#pragma unroll
-    for (int g = 0; g < 4; g++)
-      qf[m][g] = (c[4 * g] & 0xff) | ((c[4 * g + 1] & 0xff) << 8) | ((c[4 * g + 2] & 0xff) << 16) | (c[4 * g + 3] << 24);
-  }
-  return sc;
-}
-
-// per-thread / per-warp: both steps within the wave
-template <bool IS_FP16, int QF, int NQF>
-__device__ __forceinline__ float quant_q_rows(const uint16_t* rowp, bool valid, int hf, v4i (&qf)[NQF]) {
-  static_assert(QF == QF_THREAD || QF == QF_WARP, "wave-local scale groups");
-  float x[NQF][16];
-  const float am = quant_q_load<IS_FP16, QF, NQF>(rowp, valid, hf, 1.f, x);
-  return quant_q_codes<QF, NQF>(x, am, qf);
-}
-
-// workgroup barrier that the compiler neither crosses with memory operations nor schedules around
-__device__ __forceinline__ void pp_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_barrier" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 template <bool IS_FP16_OUT, bool KT, bool SPLIT, int HD, int QF = QF_INT8>
 __device__ __forceinline__ void qattn_fwd_pp(const AttnParams& p) {
   // HD: head dimension, 128 or 64.  Per 64-key tile a wave runs HD / 16 Q.K^T MFMAs (two key blocks x HD / 32
@@ -970,7 +512,7 @@ __device__ __forceinline__ void qattn_fwd_pp(const AttnParams& p) {
   auto lds_k = reinterpret_cast<uint8_t (*)[kBK * HD]>(lds_kbuf);
   __shared__ __align__(16) uint8_t lds_v[NB][HD * kBK];
   auto buf_of = [](int t) { return (int)((unsigned)t % (unsigned)NB); };
-  __shared__ float lds_ks[ks_lds_floats<PV_FP8>()];
+  __shared__ float lds_ks[kKsLdsFloats];
   __shared__ __align__(16) float lds_vs[HD];
   __shared__ __align__(16) float lds_vm[HD];
 
@@ -1702,6 +1244,17 @@ __global__ __launch_bounds__(256) void qattn_combine_kernel(AttnParams p) {
   if (p.lse && lane == 0) p.lse[(b * p.Hq + h) * p.Lq + qrow] = L > 0.f ? __builtin_log2f(L) + M : -INFINITY;
 }
 
+void launch_combine(const AttnParams& p, int out_dtype, int64_t D, hipStream_t st) {
+  const int64_t g = (p.B * p.Hq * p.Lq + 3) / 4;
+  if (D == 64) {
+    if (out_dtype == QATTN_BF16) qattn_combine_kernel<false, 64><<<g, 256, 0, st>>>(p);
+    else qattn_combine_kernel<true, 64><<<g, 256, 0, st>>>(p);
+  } else {
+    if (out_dtype == QATTN_BF16) qattn_combine_kernel<false><<<g, 256, 0, st>>>(p);
+    else qattn_combine_kernel<true><<<g, 256, 0, st>>>(p);
+  }
+}
+
 }  // namespace qattn
 
 using namespace qattn;
@@ -1709,10 +1262,7 @@ using namespace qattn;
 static bool is_thread_gran(int g) { return g == QATTN_GRAN_THREAD || g == QATTN_GRAN_THREAD_SM90; }
 
 // key tiles one workgroup can cover (its k_scales are staged in LDS)
-static int64_t max_tiles_per_split(int pv, bool kt) {
-  const int floats = pv == PV_FP8 ? ks_lds_floats<PV_FP8>() : ks_lds_floats<PV_BF16>();
-  return floats / ks_per_tile(kt);
-}
+static int64_t max_tiles_per_split(bool kt) { return kKsLdsFloats / ks_per_tile(kt); }
 
 // Ping-pong KV-split launches take whole pairs of query blocks; an odd block count leaves the last pair's
 // second wave group idle, allowed when that is at most 1/6 of the groups.
@@ -1744,12 +1294,17 @@ static int num_splits_for(int64_t B, int64_t Lq, int64_t Lk, int64_t Hq, int64_t
 }
 
 extern "C" int qattn_fwd_num_splits(int64_t B, int64_t Lq, int64_t Lk, int64_t Hq) {
-  return num_splits_for(B, Lq, Lk, Hq, max_tiles_per_split(PV_FP8, false), true);
+  return num_splits_for(B, Lq, Lk, Hq, max_tiles_per_split(false), true);
+}
+
+// the split count of a dense launch (pv: PvKind)
+static int dense_num_splits(int64_t B, int64_t Lq, int64_t Lk, int64_t Hq, int pv, int gran) {
+  if (pv == PV_FP8) return num_splits_for(B, Lq, Lk, Hq, max_tiles_per_split(is_thread_gran(gran)), true);
+  return half_num_splits(B * Hq, (Lq + kBQ - 1) / kBQ, (Lk + kBK - 1) / kBK, is_thread_gran(gran));
 }
 
 extern "C" int qattn_fwd_ex_num_splits(int64_t B, int64_t Lq, int64_t Lk, int64_t Hq, int v_kind, int qk_quant_gran) {
-  return num_splits_for(B, Lq, Lk, Hq, max_tiles_per_split(v_kind, is_thread_gran(qk_quant_gran)),
-                        v_kind == QATTN_V_FP8);
+  return dense_num_splits(B, Lq, Lk, Hq, v_kind == QATTN_V_FP8 ? PV_FP8 : PV_BF16, qk_quant_gran);
 }
 
 static int blocks_per_workgroup(int64_t bh, int64_t nqb, int64_t nkb);
@@ -1759,7 +1314,7 @@ extern "C" int qattn_fwd_ex_blocks_per_workgroup(int64_t B, int64_t Lq, int64_t 
   if (v_kind != QATTN_V_FP8 || causal || B <= 0 || Lq <= 0 || Lk <= 0 || Hq <= 0) return 1;
   const int64_t nkb = (Lk + kBK - 1) / kBK, nqb = (Lq + kBQ - 1) / kBQ;
   if (nkb >= kMqAutoMaxTiles) return 1;
-  if (num_splits_for(B, Lq, Lk, Hq, max_tiles_per_split(PV_FP8, is_thread_gran(qk_quant_gran)), true) != 1)
+  if (num_splits_for(B, Lq, Lk, Hq, max_tiles_per_split(is_thread_gran(qk_quant_gran)), true) != 1)
     return 1;
   return blocks_per_workgroup(B * Hq, nqb, nkb);
 }
@@ -1771,8 +1326,9 @@ extern "C" size_t qattn_fwd_workspace_size(int64_t B, int64_t Lq, int64_t Hq, in
 
 // Kernel selection.  Dense FP8 launches without a KV split run the ping-pong kernel when its grid (one
 // workgroup per two query blocks, one workgroup per CU) fills the 256 CUs, the multi-block variant of
-// qattn_fwd_kernel for short key ranges (blocks_per_workgroup > 1), and qattn_fwd_kernel otherwise;
-// split, half-P.V and block-sparse launches always run qattn_fwd_kernel.  A thread-local override
+// qattn_fwd_kernel for short key ranges (blocks_per_workgroup > 1), and qattn_fwd_kernel otherwise.
+// Half-P.V launches (dense, block-sparse, varlen) have one kernel of their own (attn_half.hip) and report
+// QATTN_KERNEL_ONE_BLOCK whatever the override.  A thread-local override
 // (qattn_set_kernel) forces one of the applicable kernels, so tests can compare them on small shapes.
 static thread_local int t_kernel_override = QATTN_KERNEL_AUTO;
 static thread_local int t_last_kernel = QATTN_KERNEL_AUTO;
@@ -1839,63 +1395,57 @@ static void resident_layout(int64_t bh, int64_t n_wb, int64_t& wb_per_wg, int64_
   }
 }
 
-template <int PV, bool KT, bool SP = false>
+template <bool KT>
 static int launch_fwd(AttnParams& p, int out_dtype, int ns, void* workspace, size_t workspace_bytes, hipStream_t st,
                       int64_t D, int kernel) {
   t_last_kernel = kernel;
-  if constexpr (PV == PV_FP8 && !SP) {
-    if (kernel == QATTN_KERNEL_MULTI_BLOCK) {
-      p.nsplit = 1;
-      p.tiles_per_split = (int)p.nKB;
-      p.nQC = (p.nQB + p.qpw - 1) / p.qpw;
-      const int64_t g = p.B * p.Hq * p.nQC;
-      QATTN_REQUIRE(g < (1ll << 31), QATTN_ERR_SHAPE, "grid too large");
-      if (out_dtype == QATTN_BF16) qattn_fwd_kernel<false, false, PV, KT, false, true><<<g, kThreads, 0, st>>>(p);
-      else qattn_fwd_kernel<true, false, PV, KT, false, true><<<g, kThreads, 0, st>>>(p);
-      return check_launch("qattn_fwd");
-    }
-    if (kernel == QATTN_KERNEL_RESIDENT) {
-      p.nsplit = 1;
-      p.tiles_per_split = (int)p.nKB;
-      resident_layout(p.B * p.Hq, (p.Lq + 31) / 32, p.wb_per_wg, p.n_chunk);
-      const int64_t g = p.B * p.Hq * p.n_chunk;
-      QATTN_REQUIRE(g < (1ll << 31), QATTN_ERR_SHAPE, "grid too large");
-      if (out_dtype == QATTN_BF16) qattn_fwd_res_kernel<false, KT><<<g, kResThreads, 0, st>>>(p);
-      else qattn_fwd_res_kernel<true, KT><<<g, kResThreads, 0, st>>>(p);
-      return check_launch("qattn_fwd");
-    }
-    if (kernel == QATTN_KERNEL_PINGPONG) {
-      const int64_t g = p.B * p.Hq * ((p.nQB + 1) / 2) * ns;
-      QATTN_REQUIRE(g < (1ll << 31), QATTN_ERR_SHAPE, "grid too large");
-      p.nsplit = ns;
-      p.tiles_per_split = (int)((p.nKB + ns - 1) / ns);
-      if (ns > 1) {
-        QATTN_REQUIRE(workspace && workspace_bytes >= qattn_fwd_workspace_size(p.B, p.Lq, p.Hq, D, ns),
-                      QATTN_ERR_WORKSPACE, "qattn_fwd with %d KV splits needs %zu workspace bytes", ns,
-                      qattn_fwd_workspace_size(p.B, p.Lq, p.Hq, D, ns));
-        p.ws_o = static_cast<float*>(workspace);
-        p.ws_ml = p.ws_o + (int64_t)ns * p.B * p.Hq * p.Lq * D;
-        const int64_t rows = p.B * p.Hq * p.Lq;
-        if (D == 64) {
-          if (out_dtype == QATTN_BF16) qattn_fwd_pp_kernel<false, KT, true, 64><<<g, kPPThreads, 0, st>>>(p);
-          else qattn_fwd_pp_kernel<true, KT, true, 64><<<g, kPPThreads, 0, st>>>(p);
-          if (out_dtype == QATTN_BF16) qattn_combine_kernel<false, 64><<<(rows + 3) / 4, 256, 0, st>>>(p);
-          else qattn_combine_kernel<true, 64><<<(rows + 3) / 4, 256, 0, st>>>(p);
-        } else {
-          if (out_dtype == QATTN_BF16) qattn_fwd_pp_kernel<false, KT, true><<<g, kPPThreads, 0, st>>>(p);
-          else qattn_fwd_pp_kernel<true, KT, true><<<g, kPPThreads, 0, st>>>(p);
-          if (out_dtype == QATTN_BF16) qattn_combine_kernel<false><<<(rows + 3) / 4, 256, 0, st>>>(p);
-          else qattn_combine_kernel<true><<<(rows + 3) / 4, 256, 0, st>>>(p);
-        }
-      } else if (D == 64) {
-        if (out_dtype == QATTN_BF16) qattn_fwd_pp_kernel<false, KT, false, 64><<<g, kPPThreads, 0, st>>>(p);
-        else qattn_fwd_pp_kernel<true, KT, false, 64><<<g, kPPThreads, 0, st>>>(p);
+  if (kernel == QATTN_KERNEL_MULTI_BLOCK) {
+    p.nsplit = 1;
+    p.tiles_per_split = (int)p.nKB;
+    p.nQC = (p.nQB + p.qpw - 1) / p.qpw;
+    const int64_t g = p.B * p.Hq * p.nQC;
+    QATTN_REQUIRE(g < (1ll << 31), QATTN_ERR_SHAPE, "grid too large");
+    if (out_dtype == QATTN_BF16) qattn_fwd_kernel<false, false, KT, true><<<g, kThreads, 0, st>>>(p);
+    else qattn_fwd_kernel<true, false, KT, true><<<g, kThreads, 0, st>>>(p);
+    return check_launch("qattn_fwd");
+  }
+  if (kernel == QATTN_KERNEL_RESIDENT) {
+    p.nsplit = 1;
+    p.tiles_per_split = (int)p.nKB;
+    resident_layout(p.B * p.Hq, (p.Lq + 31) / 32, p.wb_per_wg, p.n_chunk);
+    const int64_t g = p.B * p.Hq * p.n_chunk;
+    QATTN_REQUIRE(g < (1ll << 31), QATTN_ERR_SHAPE, "grid too large");
+    if (out_dtype == QATTN_BF16) qattn_fwd_res_kernel<false, KT><<<g, kResThreads, 0, st>>>(p);
+    else qattn_fwd_res_kernel<true, KT><<<g, kResThreads, 0, st>>>(p);
+    return check_launch("qattn_fwd");
+  }
+  if (kernel == QATTN_KERNEL_PINGPONG) {
+    const int64_t g = p.B * p.Hq * ((p.nQB + 1) / 2) * ns;
+    QATTN_REQUIRE(g < (1ll << 31), QATTN_ERR_SHAPE, "grid too large");
+    p.nsplit = ns;
+    p.tiles_per_split = (int)((p.nKB + ns - 1) / ns);
+    if (ns > 1) {
+      QATTN_REQUIRE(workspace && workspace_bytes >= qattn_fwd_workspace_size(p.B, p.Lq, p.Hq, D, ns),
+                    QATTN_ERR_WORKSPACE, "qattn_fwd with %d KV splits needs %zu workspace bytes", ns,
+                    qattn_fwd_workspace_size(p.B, p.Lq, p.Hq, D, ns));
+      p.ws_o = static_cast<float*>(workspace);
+      p.ws_ml = p.ws_o + (int64_t)ns * p.B * p.Hq * p.Lq * D;
+      if (D == 64) {
+        if (out_dtype == QATTN_BF16) qattn_fwd_pp_kernel<false, KT, true, 64><<<g, kPPThreads, 0, st>>>(p);
+        else qattn_fwd_pp_kernel<true, KT, true, 64><<<g, kPPThreads, 0, st>>>(p);
       } else {
-        if (out_dtype == QATTN_BF16) qattn_fwd_pp_kernel<false, KT, false><<<g, kPPThreads, 0, st>>>(p);
-        else qattn_fwd_pp_kernel<true, KT, false><<<g, kPPThreads, 0, st>>>(p);
+        if (out_dtype == QATTN_BF16) qattn_fwd_pp_kernel<false, KT, true><<<g, kPPThreads, 0, st>>>(p);
+        else qattn_fwd_pp_kernel<true, KT, true><<<g, kPPThreads, 0, st>>>(p);
       }
-      return check_launch("qattn_fwd");
+      launch_combine(p, out_dtype, D, st);
+    } else if (D == 64) {
+      if (out_dtype == QATTN_BF16) qattn_fwd_pp_kernel<false, KT, false, 64><<<g, kPPThreads, 0, st>>>(p);
+      else qattn_fwd_pp_kernel<true, KT, false, 64><<<g, kPPThreads, 0, st>>>(p);
+    } else {
+      if (out_dtype == QATTN_BF16) qattn_fwd_pp_kernel<false, KT, false><<<g, kPPThreads, 0, st>>>(p);
+      else qattn_fwd_pp_kernel<true, KT, false><<<g, kPPThreads, 0, st>>>(p);
     }
+    return check_launch("qattn_fwd");
   }
   const int64_t grid = p.B * p.Hq * p.nQB * ns;
   QATTN_REQUIRE(grid < (1ll << 31), QATTN_ERR_SHAPE, "grid too large");
@@ -1907,14 +1457,12 @@ static int launch_fwd(AttnParams& p, int out_dtype, int ns, void* workspace, siz
                   qattn_fwd_workspace_size(p.B, p.Lq, p.Hq, D, ns));
     p.ws_o = static_cast<float*>(workspace);
     p.ws_ml = p.ws_o + (int64_t)ns * p.B * p.Hq * p.Lq * D;
-    if (out_dtype == QATTN_BF16) qattn_fwd_kernel<false, true, PV, KT, SP><<<grid, kThreads, 0, st>>>(p);
-    else qattn_fwd_kernel<true, true, PV, KT, SP><<<grid, kThreads, 0, st>>>(p);
-    const int64_t rows = p.B * p.Hq * p.Lq;
-    if (out_dtype == QATTN_BF16) qattn_combine_kernel<false><<<(rows + 3) / 4, 256, 0, st>>>(p);
-    else qattn_combine_kernel<true><<<(rows + 3) / 4, 256, 0, st>>>(p);
+    if (out_dtype == QATTN_BF16) qattn_fwd_kernel<false, true, KT><<<grid, kThreads, 0, st>>>(p);
+    else qattn_fwd_kernel<true, true, KT><<<grid, kThreads, 0, st>>>(p);
+    launch_combine(p, out_dtype, D, st);
   } else {
-    if (out_dtype == QATTN_BF16) qattn_fwd_kernel<false, false, PV, KT, SP><<<grid, kThreads, 0, st>>>(p);
-    else qattn_fwd_kernel<true, false, PV, KT, SP><<<grid, kThreads, 0, st>>>(p);
+    if (out_dtype == QATTN_BF16) qattn_fwd_kernel<false, false, KT><<<grid, kThreads, 0, st>>>(p);
+    else qattn_fwd_kernel<true, false, KT><<<grid, kThreads, 0, st>>>(p);
   }
   return check_launch("qattn_fwd");
 }
@@ -1943,8 +1491,11 @@ static int blocks_per_workgroup(int64_t bh, int64_t nqb, int64_t nkb) {
 static void plan_fwd(int64_t B, int64_t Lq, int64_t Lk, int64_t Hq, int pv, int gran, int causal, bool sparse,
                      int num_splits, int& ns, int& qpw, int& kernel) {
   const int64_t nQB = (Lq + kBQ - 1) / kBQ, nKB = (Lk + kBK - 1) / kBK;
-  const int64_t max_tiles = sparse ? kSpMaxTiles : max_tiles_per_split(pv, is_thread_gran(gran));
-  ns = num_splits > 0 ? num_splits : num_splits_for(B, Lq, Lk, Hq, max_tiles, pv == PV_FP8 && !sparse);
+  const int64_t max_tiles = pv == PV_FP8 ? max_tiles_per_split(is_thread_gran(gran))
+                                         : half_max_tiles(nQB, is_thread_gran(gran), sparse);
+  ns = num_splits > 0 ? num_splits
+       : sparse       ? num_splits_for(B, Lq, Lk, Hq, max_tiles, false)
+                      : dense_num_splits(B, Lq, Lk, Hq, pv, gran);
   ns = (int)std::min<int64_t>(ns, nKB);
   if (ns < 1) ns = 1;
   // a workgroup stages the k_scales of at most max_tiles key tiles
@@ -2043,11 +1594,24 @@ static int setup_fwd(AttnParams& p, int& ns, qattn_seq q8, const float* q_scale,
   return QATTN_OK;
 }
 
-template <int PV>
 static int launch_gran(AttnParams& p, int gran, int out_dtype, int ns, void* ws, size_t wsb, hipStream_t st,
                        int64_t D, int kernel) {
-  if (is_thread_gran(gran)) return launch_fwd<PV, true>(p, out_dtype, ns, ws, wsb, st, D, kernel);
-  return launch_fwd<PV, false>(p, out_dtype, ns, ws, wsb, st, D, kernel);
+  if (is_thread_gran(gran)) return launch_fwd<true>(p, out_dtype, ns, ws, wsb, st, D, kernel);
+  return launch_fwd<false>(p, out_dtype, ns, ws, wsb, st, D, kernel);
+}
+
+// half P.V: the workspace of a KV split, then the launch (attn_half.hip)
+static int launch_half_ws(AttnParams& p, bool kt, bool f16v, bool sparse, int out_dtype, int ns, void* ws, size_t wsb,
+                          hipStream_t st) {
+  t_last_kernel = QATTN_KERNEL_ONE_BLOCK;
+  if (ns > 1) {
+    const size_t need = qattn_fwd_workspace_size(p.B, p.Lq, p.Hq, kD, ns);
+    QATTN_REQUIRE(ws && wsb >= need, QATTN_ERR_WORKSPACE, "qattn_fwd with %d KV splits needs %zu workspace bytes", ns,
+                  need);
+    p.ws_o = static_cast<float*>(ws);
+    p.ws_ml = p.ws_o + (int64_t)ns * p.B * p.Hq * p.Lq * kD;
+  }
+  return launch_half(p, kt, f16v, sparse, out_dtype, ns, st);
 }
 
 extern "C" int qattn_fwd_ex(qattn_seq q8, const float* q_scale, qattn_seq k8, const float* k_scale, const void* v,
@@ -2081,11 +1645,11 @@ extern "C" int qattn_fwd_ex2(qattn_seq q8, const float* q_scale, qattn_seq k8, c
     QATTN_REQUIRE(v_scale, QATTN_ERR_ARG, "v_scale is null");
     p.v_scale = v_scale;
     p.v_mean = v_mean;
-    return launch_gran<PV_FP8>(p, qk_quant_gran, out_dtype, ns, workspace, workspace_bytes, st, D, kernel);
+    return launch_gran(p, qk_quant_gran, out_dtype, ns, workspace, workspace_bytes, st, D, kernel);
   }
   p.v_scale = nullptr;
-  if (pv == PV_BF16) return launch_gran<PV_BF16>(p, qk_quant_gran, out_dtype, ns, workspace, workspace_bytes, st, D, kernel);
-  return launch_gran<PV_FP16>(p, qk_quant_gran, out_dtype, ns, workspace, workspace_bytes, st, D, kernel);
+  return launch_half_ws(p, is_thread_gran(qk_quant_gran), pv == PV_FP16, false, out_dtype, ns, workspace,
+                        workspace_bytes, st);
 }
 
 // ---- half Q quantized inside the attention kernel (resident or ping-pong) ----
@@ -2109,11 +1673,9 @@ static void launch_pp_q16(AttnParams& p, int dtype, int ns, hipStream_t st) {
   constexpr bool KT = QF == QF_THREAD;
   const int64_t g = p.B * p.Hq * ((p.nQB + 1) / 2) * ns;
   if (ns > 1) {
-    const int64_t rows = p.B * p.Hq * p.Lq;
     if (dtype == QATTN_BF16) qattn_fwd_pp_kernel<false, KT, true, HD, QF><<<g, kPPThreads, 0, st>>>(p);
     else qattn_fwd_pp_kernel<true, KT, true, HD, QF><<<g, kPPThreads, 0, st>>>(p);
-    if (dtype == QATTN_BF16) qattn_combine_kernel<false, HD><<<(rows + 3) / 4, 256, 0, st>>>(p);
-    else qattn_combine_kernel<true, HD><<<(rows + 3) / 4, 256, 0, st>>>(p);
+    launch_combine(p, dtype, HD, st);
   } else {
     if (dtype == QATTN_BF16) qattn_fwd_pp_kernel<false, KT, false, HD, QF><<<g, kPPThreads, 0, st>>>(p);
     else qattn_fwd_pp_kernel<true, KT, false, HD, QF><<<g, kPPThreads, 0, st>>>(p);
@@ -2220,7 +1782,8 @@ extern "C" int qattn_fwd_varlen(qattn_seq q8, const float* q_scale, qattn_seq k8
   p.var_tk = total_k;
   p.v_scale = nullptr;
   p.qpw = 1;
-  return launch_fwd<PV_FP16, false>(p, out_dtype, 1, nullptr, 0, (hipStream_t)stream, D, QATTN_KERNEL_ONE_BLOCK);
+  t_last_kernel = QATTN_KERNEL_ONE_BLOCK;
+  return launch_half_varlen(p, out_dtype, (hipStream_t)stream);
 }
 
 // ---- allocation-free form of qattn_fwd_ex ----
@@ -2360,6 +1923,5 @@ extern "C" int qattn_fwd_block_sparse(qattn_seq q8, const float* q_scale, qattn_
   p.tm_s1 = mask_sbh;
   p.tm_s2 = mask_sq;
   hipStream_t st = (hipStream_t)stream;
-  if (pv == PV_BF16) return launch_fwd<PV_BF16, false, true>(p, out_dtype, ns, workspace, workspace_bytes, st, D, kernel);
-  return launch_fwd<PV_FP16, false, true>(p, out_dtype, ns, workspace, workspace_bytes, st, D, kernel);
+  return launch_half_ws(p, false, pv == PV_FP16, true, out_dtype, ns, workspace, workspace_bytes, st);
 }

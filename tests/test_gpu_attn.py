@@ -344,6 +344,77 @@ def test_half_pv_causal_split_padding(oracle):
     _run_and_check(oracle, q, k[:, :300], v[:, :300], pv="half", causal=True)
 
 
+@pytest.mark.parametrize("Lq,Lk,Hq,Hkv,kw", [
+    # pairs of query blocks: whole and odd counts, key ranges of 1 .. 5 tiles (three K / V buffers)
+    (256, 1, 2, 2, {}), (200, 64, 2, 2, {}), (640, 65, 2, 1, {}), (256, 192, 2, 2, {}), (641, 300, 1, 1, {}),
+    # a block per group: one and three blocks per head, the groups on one kv head (shared tiles) and on two, an odd
+    # number of blocks in all, key ranges of 1 .. 9 tiles (six shared buffers)
+    (1, 1, 1, 1, {}), (128, 64, 3, 3, {}), (300, 130, 2, 1, {}), (384, 320, 3, 1, {}), (100, 385, 2, 2, {}),
+    (33, 449, 1, 1, {}), (300, 576, 4, 2, {}),
+    # groups of unequal length: causal blocks, with and without an offset; padding; a KV split
+    (384, 384, 1, 1, dict(causal=True)), (300, 900, 2, 1, dict(causal=True, q_offset=500)),
+    (512, 512, 2, 2, dict(causal=True)), (700, 700, 1, 1, dict(causal=True)),
+    (130, 700, 2, 2, dict(kv_valid=[1])), (130, 700, 2, 2, dict(num_splits=3)), (600, 1000, 2, 2, dict(num_splits=4)),
+])
+@pytest.mark.parametrize("gran", ["per_block", "per_thread"])
+def test_half_kernel_forms(oracle, Lq, Lk, Hq, Hkv, kw, gran):
+    """The half-P.V kernel at the edges of its forms (workgroups of a pair of query blocks, or of one block per wave
+    group) against the oracle on the same quantized operands."""
+    q, k, v = qkv(1, Lq, Lk, Hq, Hkv, seed=Lq + 7 * Lk, k_offset_std=0.5)
+    _run_and_check(oracle, q, k, v, pv="half", gran=gran, check_truth=False, **kw)
+
+
+@pytest.mark.parametrize("case", ["equal", "disjoint", "subset", "one_empty", "long", "causal", "odd_blocks"])
+def test_block_sparse_tile_lists(case):
+    """Masks whose neighbouring query blocks share all, none or some of their tiles (the kernel fetches the shared
+    ones once, then each wave group its own): against the block-masked softmax in float64 of the same int8 codes, so
+    that only the fp16 rounding of P and V (2^-11 each) and of the output (bf16, 2^-9) differ: relative error of a
+    row at most ~2^-9 + 2 * 2^-11 = 0.003; 0.006 is asserted."""
+    dev = require_gpu()
+    from telefuser_amd import sageattn2 as sa
+    from telefuser_amd.sparse_sage import sparse_sageattn
+
+    L = {"long": 64 * 21, "odd_blocks": 300}.get(case, 512)
+    H = 3 if case == "odd_blocks" else 2
+    q, k, v = qkv(1, L, L, H, H, seed=77, k_offset_std=0.5)
+    nq, nk = -(-L // 128), -(-L // 64)
+    g = torch.Generator().manual_seed(78)
+    mask = torch.zeros((1, H, nq, nk), dtype=torch.int8)
+    if case == "equal":
+        mask[..., ::2] = 1
+    elif case == "disjoint":
+        mask[:, :, ::2, ::2] = 1
+        mask[:, :, 1::2, 1::2] = 1
+    elif case == "subset":
+        mask[:, :, ::2] = 1
+        mask[:, :, 1::2, 1] = 1
+    elif case == "one_empty":
+        mask[:, :, 1::2, 2:7] = 1
+    elif case == "long":
+        mask[:] = torch.rand(mask.shape, generator=g) < 0.8
+    else:
+        mask[:] = torch.rand(mask.shape, generator=g) < 0.5
+    causal = case == "causal"
+    log(f"block-sparse tile lists {case}")
+    qd, kd, vd = (t.to(dev) for t in (q, k, v))
+    o = sparse_sageattn(qd, kd, vd, mask.to(dev), is_causal=causal, tensor_layout="NHD").float().cpu().double()
+    q8, qs, k8, ks = (t.cpu().double() for t in sa.per_block_int8(qd, kd, sa.k_mean(kd, "NHD"), sm_scale=128 ** -0.5,
+                                                                  tensor_layout="NHD", variant="triton"))
+    for h in range(H):
+        s = (q8[0, :, h] @ k8[0, :, h].T) * qs[0, h].repeat_interleave(128)[:L, None] * \
+            ks[0, h].repeat_interleave(64)[None, :L]
+        keep = mask[0, h].bool().repeat_interleave(128, 0)[:L].repeat_interleave(64, 1)[:, :L]
+        if causal:
+            keep = keep & torch.ones(L, L, dtype=torch.bool).tril()
+        p = torch.where(keep, torch.exp2(s - s.max()), torch.zeros_like(s))
+        den = p.sum(1, keepdim=True)
+        ref = (p @ v[0, :, h].to(torch.float16).double()) / den.clamp_min(1e-300)
+        assert not o[0, :, h][den[:, 0] == 0].any()
+        rows = den[:, 0] > 0
+        err = (o[0, rows, h] - ref[rows]).norm(dim=1) / ref[rows].norm(dim=1)
+        assert float(err.max()) < 0.006, float(err.max())
+
+
 def test_pv16_api_entry_points(oracle):
     dev = require_gpu()
     from telefuser_amd import sageattn2 as sa
