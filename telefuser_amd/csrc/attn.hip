@@ -516,16 +516,9 @@ __device__ __forceinline__ void qattn_fwd_pp(const AttnParams& p) {
   __shared__ __align__(16) float lds_vs[HD];
   __shared__ __align__(16) float lds_vm[HD];
 
-  const int64_t nQP = (p.nQB + 1) / 2;
-  const int64_t wg_id = xcd_remap(blockIdx.x, gridDim.x);
-  // KV split: split-major order, so the workgroups of one key range of a head run next to each other
-  const int64_t n_pairs = p.B * p.Hq * nQP;
-  const int split = SPLIT ? (int)(wg_id / n_pairs) : 0;
-  const int64_t tile_id = SPLIT ? wg_id - (int64_t)split * n_pairs : wg_id;
-  const int64_t qp = tile_id % nQP;
-  const int64_t rest = tile_id / nQP;
-  const int64_t h = rest % p.Hq;
-  const int64_t b = rest / p.Hq;
+  int split;
+  int64_t b, h, qp;
+  pair_of_workgroup<SPLIT>(p, split, b, h, qp);
   const int64_t hk = h / p.group;
 
   const int tid = threadIdx.x;

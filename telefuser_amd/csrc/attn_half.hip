@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kHFThreads) void qattn_fwd_half_kernel(AttnParams p
     nqb_wg_last = (int64_t)vq * 2 + 1;
   } else if constexpr (OWN) {
     const uint32_t units = (uint32_t)(p.B * p.Hq * p.nQB), wgs = (units + 1) / 2;
-    const uint32_t wg = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t wg = xcd_remap(blockIdx.x, gridDim.x);
     split = SPLIT ? (int)(wg / wgs) : 0;
     unit0 = (wg - (uint32_t)split * wgs) * 2;
     const uint32_t u = unit0 + grp;
@@ -144,15 +144,10 @@ __global__ __launch_bounds__(kHFThreads) void qattn_fwd_half_kernel(AttnParams p
     h = bh - (uint32_t)b * (uint32_t)p.Hq;
     nqb_wg_last = qb;
   } else {
-    // (index math in 32 bits: the grid is below 2^31 workgroups)
-    const uint32_t nQP = (uint32_t)(p.nQB + 1) / 2, n_pairs = (uint32_t)(p.B * p.Hq) * nQP;
-    const uint32_t wg = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);
-    split = SPLIT ? (int)(wg / n_pairs) : 0;
-    const uint32_t id = wg - (uint32_t)split * n_pairs, bh = id / nQP, qp = id - bh * nQP;
-    b = bh / (uint32_t)p.Hq;
-    h = bh - (uint32_t)b * (uint32_t)p.Hq;
-    qb = (int64_t)qp * 2 + grp;  // == nQB for the empty second group of an odd block count
-    nqb_wg_last = min((int64_t)qp * 2 + 1, p.nQB - 1);
+    int64_t qp;
+    pair_of_workgroup<SPLIT>(p, split, b, h, qp);
+    qb = qp * 2 + grp;  // == nQB for the empty second group of an odd block count
+    nqb_wg_last = min(qp * 2 + 1, p.nQB - 1);
   }
   const int64_t hk = (uint32_t)h / (uint32_t)p.group;
 
