@@ -210,6 +210,14 @@ int qattn_fwd(qattn_seq q8, const float* q_scale, qattn_seq k8, const float* k_s
               qattn_stream_t stream);
 
 /*
+ * The kernels' LSE (log2 domain, against the smoothed keys K - k_mean) to the natural-log LSE of the original keys, in
+ * place: lse / 1.44269504 + (q . k_mean) * sm_scale per row (sageattn2.py:1334-1354,1450-1455; the dot product in
+ * fp32).  lse [B, Hq, Lq]; q bf16 / fp16 rows of D = 64 or 128 elements; k_mean [B, Hkv, D] in q's dtype.
+ */
+int qattn_lse_finish(float* lse, qattn_seq q, int dtype, const void* k_mean, int64_t B, int64_t Lq, int64_t Hq,
+                     int64_t Hkv, int64_t D, float sm_scale, qattn_stream_t stream);
+
+/*
  * V (bf16/fp16) copied into the same transposed, tile-permuted layout as qattn_per_channel_fp8 uses,
  * in its own dtype: v16 [B, H, D, Lpad].  Replaces the V preparation of the reference's fp16-P.V
  * paths (sageattn_qk_int8_pv_fp16_cuda / _triton, tf-kernel/tf_kernel/sageattn2.py:551-769,930-1194).

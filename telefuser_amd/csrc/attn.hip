@@ -1237,6 +1237,43 @@ __global__ __launch_bounds__(256) void qattn_combine_kernel(AttnParams p) {
   if (p.lse && lane == 0) p.lse[(b * p.Hq + h) * p.Lq + qrow] = L > 0.f ? __builtin_log2f(L) + M : -INFINITY;
 }
 
+// Natural-log LSE of the original K from the kernels' log2-domain LSE against K - km: lse * ln 2 + (q . km) sm_scale,
+// in place.  One pass over Q (HBM-bound: 2 B per element), 16 bytes of a row per lane and the rows in Q's memory order
+// (torch's form took six launches, 70 us of them next to a 140 us attention at 2 x 4096 x 16: the matvec alone 45).
+template <bool IS_FP16, int D>
+__global__ __launch_bounds__(256) void lse_finish_kernel(float* lse, const uint16_t* q, int64_t sb, int64_t sl, int64_t sh,
+                                                         const uint16_t* km, int64_t L, int64_t Hq, int group,
+                                                         int64_t rows, float sm_scale) {
+  constexpr int TPR = D / 8;  // lanes per row
+  const int64_t r = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  const int dc = threadIdx.x % TPR;
+  if (r >= rows) return;  // (whole rows: their lanes leave together)
+  // r counts rows with the smaller of the sequence and head strides innermost
+  int64_t b, h, l;
+  if (sh < sl) {
+    h = r % Hq;
+    l = (r / Hq) % L;
+  } else {
+    l = r % L;
+    h = (r / L) % Hq;
+  }
+  b = r / (Hq * L);
+  const v4u x = *reinterpret_cast<const v4u*>(q + b * sb + l * sl + h * sh + dc * 8);
+  const v4u m = *reinterpret_cast<const v4u*>(km + (b * (Hq / group) + h / group) * D + dc * 8);
+  float s = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    s = fmaf(half_to_f32<IS_FP16>((uint16_t)(x[e] & 0xffffu)), half_to_f32<IS_FP16>((uint16_t)(m[e] & 0xffffu)), s);
+    s = fmaf(half_to_f32<IS_FP16>((uint16_t)(x[e] >> 16)), half_to_f32<IS_FP16>((uint16_t)(m[e] >> 16)), s);
+  }
+#pragma unroll
+  for (int o = 1; o < TPR; o <<= 1) s += __shfl_xor(s, o, 64);
+  if (dc == 0) {
+    float* p = lse + (b * Hq + h) * L + l;
+    *p = *p / 1.44269504f + s * sm_scale;
+  }
+}
+
 void launch_combine(const AttnParams& p, int out_dtype, int64_t D, hipStream_t st) {
   const int64_t g = (p.B * p.Hq * p.Lq + 3) / 4;
   if (D == 64) {
@@ -1868,6 +1905,35 @@ extern "C" int qattn_fwd_ex_noalloc(qattn_seq q8, const float* q_scale, qattn_se
     QATTN_REQUIRE(he == hipSuccess, QATTN_ERR_LAUNCH, "hipEventRecord failed: %s", hipGetErrorString(he));
   }
   return QATTN_OK;
+}
+
+extern "C" int qattn_lse_finish(float* lse, qattn_seq q, int dtype, const void* k_mean, int64_t B, int64_t Lq,
+                                int64_t Hq, int64_t Hkv, int64_t D, float sm_scale, qattn_stream_t stream) {
+  QATTN_REQUIRE(dtype == QATTN_BF16 || dtype == QATTN_FP16, QATTN_ERR_DTYPE, "dtype must be bf16 (0) or fp16 (1)");
+  QATTN_REQUIRE(D == 64 || D == 128, QATTN_ERR_HEAD_DIM, "head_dim must be 64 or 128, got %lld", (long long)D);
+  QATTN_REQUIRE(B >= 0 && Lq >= 0 && Hq > 0 && Hkv > 0, QATTN_ERR_SHAPE, "bad sizes");
+  QATTN_REQUIRE(Hq % Hkv == 0, QATTN_ERR_HEAD_RATIO, "num_qo_heads (%lld) must be divisible by num_kv_heads (%lld)",
+                (long long)Hq, (long long)Hkv);
+  if (B * Lq == 0) return QATTN_OK;
+  QATTN_REQUIRE(lse && k_mean && aligned16(k_mean) && q.data && aligned16(q.data), QATTN_ERR_ALIGN,
+                "null or misaligned pointer");
+  QATTN_REQUIRE(q.sb % 8 == 0 && q.sl % 8 == 0 && q.sh % 8 == 0, QATTN_ERR_STRIDE,
+                "q strides must be multiples of 16 bytes");
+  const int64_t rows = B * Lq * Hq, per = 256 / (D / 8), g = (rows + per - 1) / per;
+  QATTN_REQUIRE(g < (1ll << 31), QATTN_ERR_SHAPE, "grid too large");
+  hipStream_t st = (hipStream_t)stream;
+  const uint16_t *qp = static_cast<const uint16_t*>(q.data), *km = static_cast<const uint16_t*>(k_mean);
+#define QATTN_LF(F16, DD) \
+  lse_finish_kernel<F16, DD><<<g, 256, 0, st>>>(lse, qp, q.sb, q.sl, q.sh, km, Lq, Hq, (int)(Hq / Hkv), rows, sm_scale)
+  if (dtype == QATTN_BF16) {
+    if (D == 128) QATTN_LF(false, 128);
+    else QATTN_LF(false, 64);
+  } else {
+    if (D == 128) QATTN_LF(true, 128);
+    else QATTN_LF(true, 64);
+  }
+#undef QATTN_LF
+  return check_launch("qattn_lse_finish");
 }
 
 extern "C" int qattn_fwd(qattn_seq q8, const float* q_scale, qattn_seq k8, const float* k_scale, const uint8_t* v8,

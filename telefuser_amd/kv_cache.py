@@ -267,10 +267,7 @@ class QuantizedKVCache:
         if not return_lse:
             return res
         o, lse = res
-        hq = q.shape[2]
-        kmb = self.k_mean.repeat_interleave(hq // self.H, dim=1)  # [B, Hq, D]
-        corr = torch.matmul(q.transpose(1, 2), kmb.unsqueeze(-1)).squeeze(-1).to(torch.float32)
-        return o, lse / sa.LOG2E + corr * sm_scale
+        return o, sa._finish_lse(lse, q, self.k_mean, "NHD", sm_scale)
 
 
 __all__ = ["streaming_self_attention", "QuantizedKVCache"]

@@ -513,14 +513,23 @@ def _sage_finish(res, q, km, hq, hkv, head_dim_og, tensor_layout, sm_scale, smoo
     o = o[..., :head_dim_og]
     if not return_lse:
         return o
-    lse = lse / LOG2E
-    if smooth_k:
-        # logits were computed against k - km: add back q.km * sm_scale
+    return o, _finish_lse(lse, q, km if smooth_k else None, tensor_layout, sm_scale)
+
+
+def _finish_lse(lse, q, km, tensor_layout, sm_scale):
+    """The kernels' log2-domain LSE as natural log; with km ([B, Hkv, D]), logits were computed against k - km: q.km *
+    sm_scale is added back, in one launch on lse's own buffer."""
+    if km is None:
+        return lse / LOG2E
+    b, lq, hq, d = _dims(q, tensor_layout)
+    if torch.is_grad_enabled() and q.requires_grad:  # (the correction, in torch, keeps its graph)
         qq = q if tensor_layout == "HND" else q.transpose(1, 2)
-        kmb = km.repeat_interleave(hq // hkv, dim=1)  # [B, Hq, D]
-        corr = torch.matmul(qq, kmb.unsqueeze(-1)).squeeze(-1).to(torch.float32)
-        lse = lse + corr * sm_scale
-    return o, lse
+        corr = torch.matmul(qq, km.repeat_interleave(hq // km.shape[1], dim=1).unsqueeze(-1)).squeeze(-1)
+        return lse / LOG2E + corr.to(torch.float32) * sm_scale
+    _lib.check(_lib.load().qattn_lse_finish(_lib.ptr(lse), _lib.seq(q, tensor_layout), _lib.dtype_code(q.dtype),
+                                            _lib.ptr(km), b, lq, hq, km.shape[1], d, float(sm_scale),
+                                            _lib.stream_of(q)))
+    return lse
 
 
 def sageattn_qk_int8_pv_fp8_cuda(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tensor_layout: str = "HND",

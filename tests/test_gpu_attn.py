@@ -1144,3 +1144,46 @@ def test_dropin_strided_views_of_packed_qkv(gran, lk):
     torch.cuda.synchronize()
     assert torch.equal(o, oc), f"max diff {float((o.float() - oc.float()).abs().max())}"
     assert torch.equal(lse, lsec)
+
+
+@pytest.mark.parametrize("layout", ["NHD", "HND"])
+@pytest.mark.parametrize("B,L,Hq,Hkv,D,dtype", [(1, 1, 1, 1, 128, torch.bfloat16), (2, 17, 3, 1, 128, torch.float16),
+                                                (1, 33, 4, 2, 64, torch.bfloat16), (3, 100, 2, 2, 64, torch.float16)])
+def test_lse_finish(layout, B, L, Hq, Hkv, D, dtype):
+    """lse * ln 2 + (q . km) sm_scale in one launch, against float64: the dot product is a fp32 sum of D products
+    (error at most D * 2^-24 of the sum of magnitudes), the rest two fp32 roundings; rows without keys stay -inf."""
+    dev = require_gpu()
+    from telefuser_amd import sageattn2 as sa
+
+    g = torch.Generator().manual_seed(L)
+    q = torch.randn((B, L, Hq, 2 * D), generator=g).to(dtype)[..., :D]  # (rows 2 D apart)
+    km = torch.randn((B, Hkv, D), generator=g).to(dtype)
+    lse = torch.randn((B, Hq, L), generator=g) * 10
+    lse[0, 0, 0] = -float("inf")
+    log(f"lse_finish {layout} B={B} L={L} H={Hq}/{Hkv} D={D} {dtype}")
+    qd = q.to(dev) if layout == "NHD" else q.to(dev).transpose(1, 2)
+    got = sa._finish_lse(lse.to(dev), qd, km.to(dev), layout, 0.3).cpu().double()
+    prod = q.double().transpose(1, 2) * km.double().repeat_interleave(Hq // Hkv, 1)[:, :, None]
+    want = lse.double() / 1.44269504 + prod.sum(-1) * 0.3
+    bound = 0.3 * D * 2.0 ** -24 * prod.abs().sum(-1) + 2.0 ** -22 * (lse.abs().double() + prod.sum(-1).abs())
+    fin = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(got), fin) and got[0, 0, 0] == -float("inf")
+    assert bool(((got - want).abs()[fin] <= bound[fin]).all())
+
+
+@pytest.mark.parametrize("B,L,Hq,Hkv,D,q_offset", [(1, 300, 2, 2, 128, 0), (2, 1100, 3, 1, 128, 0), (1, 640, 8, 2, 64, 0),
+                                                   (1, 512, 5, 5, 128, 700)])
+def test_causal_work_order(oracle, B, L, Hq, Hkv, D, q_offset):
+    """Causal ping-pong launches hand out the longest pairs of query blocks first: every (batch, head, pair) is
+    still covered once, for odd pair counts and head counts that are no multiple of 8."""
+    dev = require_gpu()
+    from telefuser_amd import _lib
+
+    q, k, v = qkv(B, L, L + q_offset, Hq, Hkv, D=D, seed=91, k_offset_std=0.5)
+    lib = _lib.load()
+    lib.qattn_set_kernel(_lib.QATTN_KERNEL_PINGPONG)
+    try:
+        _run_and_check(oracle, q, k, v, causal=True, q_offset=q_offset, num_splits=1)
+        assert lib.qattn_last_kernel() == _lib.QATTN_KERNEL_PINGPONG
+    finally:
+        lib.qattn_set_kernel(_lib.QATTN_KERNEL_AUTO)
