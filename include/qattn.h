@@ -230,6 +230,18 @@ int qattn_v_tile_half_ex(qattn_seq v, int dtype, int out_dtype, int64_t B, int64
                          uint16_t* v16, int64_t Lpad, qattn_stream_t stream);
 
 /*
+ * The prologue of the half-P.V paths in one call: K mean, Q / K to INT8 (qk_quant_gran 1 per block with `variant` and
+ * q_sm_scale folded into Q, 2 per warp, 3 per thread), V into half tiles; the same bits as qattn_seq_mean, the
+ * quantizers and qattn_v_tile_half_ex.  dtype: Q and K; v_dtype: V; tile_dtype: v16 (v_dtype, or fp16 from bf16).
+ * Lq = 0: K and V only.  Workspace (with smooth_k): qattn_seq_mean_workspace_size(B, Lk, Hkv, D).
+ */
+int qattn_sage_quant_half(qattn_seq q, qattn_seq k, qattn_seq v, int dtype, int v_dtype, int tile_dtype, int64_t B,
+                          int64_t Lq, int64_t Lk, int64_t Hq, int64_t Hkv, int64_t D, int qk_quant_gran, int variant,
+                          float q_sm_scale, int smooth_k, qattn_seq q_out, float* q_scale, qattn_seq k_out,
+                          float* k_scale, void* k_mean, uint16_t* v16, int64_t Lpad, void* workspace,
+                          size_t workspace_bytes, qattn_stream_t stream);
+
+/*
  * The prologue of the INT8-QK / FP8-PV path in four launches: one pass over K and V for their column
  * statistics (K sum when smooth_k; V max |v|, or sum / max / min when smooth_v), one finalize (k_mean
  * [B, Hkv, D] in the input dtype, v_scale, v_mean), V to FP8 tiles (as qattn_per_channel_fp8_ex), and K then

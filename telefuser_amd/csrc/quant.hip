@@ -728,6 +728,325 @@ static void launch_v_tile_half(dim3 grid, bool conv, int64_t D, const qattn_seq&
 }
 
 // ------------------------------------------------------------------------------------------------
+// small inputs: the finalize steps, V's tiles and the quantizers in one launch
+// ------------------------------------------------------------------------------------------------
+// A prologue of a few MB is bound by its chain of launches, not by its bytes (4680 keys x 12 heads: 33 us in four
+// launches for 14 MB).  Every workgroup here reduces the chunk partials of its own (batch entry, head) itself - a few
+// KiB from L2, in reduce_chunks' order, so the mean and the scales keep their bits - and goes on with its block: a
+// pair of V tiles, 64 K rows or a Q block.  The first workgroup of each head writes the mean and the scales out.
+constexpr int64_t kSmallChunks = 32, kSmallWorkgroups = 4096;
+struct SmallArgs {
+  QuantJob k, q;  // q.nwg = 0: Q is quantized by the attention kernel
+  const float *kpart, *vpart;
+  int64_t nchunk;
+  uint16_t* kmean;  // null: K is not smoothed
+  const uint16_t* v;
+  int64_t vsb, vsl, vsh, L, H;
+  int64_t Lpad;
+  uint32_t nvt;   // V workgroups (pairs of tiles) per (batch entry, head)
+  uint32_t nvwg;  // B * H * nvt
+  uint8_t* v8;    // FP8 V
+  float scale_max;
+  int smooth_v;
+  float *v_scale, *v_mean;
+  uint16_t* v16;  // half V
+  int conv;       // bf16 V to fp16 tiles
+};
+
+// block n of head h of batch entry b that workgroup wg of a job takes
+__device__ __forceinline__ void quant_index(const QuantJob& J, uint32_t wg, uint32_t& n, uint32_t& h, uint32_t& b) {
+  const uint32_t H = (uint32_t)J.H, NB = (uint32_t)J.nblk;
+  // Heads interleaved inside a row (sequence-major layouts): the heads of one row block run next to
+  // each other, so concurrent workgroups read contiguous row segments; head-major layouts walk blocks.
+  if (J.sh < J.sl) {
+    const uint32_t q = wg / H;
+    h = wg - q * H;
+    b = q / NB;
+    n = q - b * NB;
+  } else {
+    const uint32_t bh = wg / NB;
+    n = wg - bh * NB;
+    b = bh / H;
+    h = bh - b * H;
+  }
+}
+
+// quant_per_block_kernel's block without its packed sequences and norm + rope, the row subtracted from every row
+// (mean: D half words in LDS, or null).  The two are kept apart: as one function the general kernel spilled nine
+// registers instead of one (45 -> 51 us for K at 32760 x 12).
+template <bool IS_FP16, int VARIANT, int D, int CR>
+__device__ __forceinline__ void quant_block(const QuantJob& J, uint32_t wg, const uint16_t* mean) {
+  constexpr bool GROUPED = CR != 0;
+  constexpr int NCELL = GROUPED ? 128 / CR : 1;  // cells of a 128-row block
+  constexpr int kQuantThreads = quant_threads<VARIANT>();
+  constexpr int TPR = D / 8;                       // threads (16-byte chunks) per row
+  constexpr int MAXC = 128 * TPR / kQuantThreads;  // chunks per thread at 128 rows
+  constexpr int RPP = kQuantThreads / TPR;         // rows per pass: chunk i of a thread is row RPP i + tid / TPR
+  constexpr int RPW = 64 / TPR;                    // rows per wave and pass
+  constexpr int NW = kQuantThreads / 64;
+  constexpr int NA = GROUPED ? MAXC : 1;           // |x| maxima kept per thread
+  static_assert(RPP % 32 == 0 && 32 % RPW == 0 && MAXC * RPP == 128, "row cells");
+
+  // index math in 32 bits (the grid is below 2^31 workgroups)
+  uint32_t n, h, b;
+  quant_index(J, wg, n, h, b);
+  const int tid = threadIdx.x;
+  const int blk = J.blk;
+  const uint16_t* in_b = J.in + (int64_t)b * J.sb;
+  int8_t* out_b = J.out + (int64_t)b * J.ob;
+  const int64_t Lb = J.L;
+  float* scale_at = J.scale + (((int64_t)b * J.H + h) * J.scale_blocks + (int64_t)n * J.nsub) * J.ncls;
+
+  // the scale class of a row: rows r with equal (r % 8) / (8 / ncls) share a scale.  Every thread
+  // touches rows of a single class (RPP is a multiple of 8).
+  const int cls = ((tid / TPR) & 7) >> J.cls_shift;
+  const int row0 = tid / TPR, dc = tid % TPR;
+
+  float x[MAXC][8];
+  const float amax0 = VARIANT == QATTN_QUANT_CUDA ? 0.0000001f : 0.f;
+  float am[NA];  // |x| maximum of each chunk (GROUPED), or of all of them
+#pragma unroll
+  for (int i = 0; i < NA; i++) am[i] = amax0;
+#pragma unroll
+  for (int i = 0; i < MAXC; i++) {
+    const int r = row0 + RPP * i;
+    const int64_t l = (int64_t)n * blk + r;
+#pragma unroll
+    for (int e = 0; e < 8; e++) x[i][e] = 0.f;
+    if (r < blk && l < Lb) {
+      v4u raw = *reinterpret_cast<const v4u*>(in_b + l * J.sl + (int64_t)h * J.sh + dc * 8);
+      uint16_t hv[8];
+      __builtin_memcpy(hv, &raw, 16);
+      float mv[8];
+      if (mean) {
+        v4u mraw = *reinterpret_cast<const v4u*>(mean + dc * 8);
+        uint16_t mh[8];
+        __builtin_memcpy(mh, &mraw, 16);
+#pragma unroll
+        for (int e = 0; e < 8; e++) mv[e] = half_to_f32<IS_FP16>(mh[e]);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        float v = half_to_f32<IS_FP16>(hv[e]);
+        if (mean) {
+          v = v - mv[e];
+          // Triton paths: k - km is a torch op on half tensors, rounded back to the half type
+          if constexpr (VARIANT != QATTN_QUANT_CUDA) v = round_to_half<IS_FP16>(v);
+        }
+        if (J.has_sm_scale) v = v * J.sm_scale;
+        x[i][e] = v;
+        am[GROUPED ? i : 0] = fmaxf(am[GROUPED ? i : 0], fabsf(v));
+      }
+    }
+  }
+
+  // IEEE division (hipcc default: correctly rounded)
+  auto scale_of = [](float a) {
+    if constexpr (VARIANT == QATTN_QUANT_TRITON_THREAD) return quant_scale_triton(a);
+    else return quant_scale_cuda(a);
+  };
+  // per chunk (GROUPED) or per thread: the scale (Triton rounding) or 127 / amax (CUDA rounding)
+  float sc[NA];
+  if constexpr (VARIANT == QATTN_QUANT_TRITON_THREAD) {
+    // per-thread scale classes: each row's maximum (over its TPR lanes) into LDS, then the maximum over
+    // the rows of a class in the row's scale block (ungrouped: rows r, r + RPP, ... already share theirs)
+    __shared__ float row_max[GROUPED ? 128 : RPP];
+#pragma unroll
+    for (int i = 0; i < NA; i++) {
+      float a = am[i];
+#pragma unroll
+      for (int o = 1; o < TPR; o <<= 1) a = fmaxf(a, __shfl_xor(a, o, 64));
+      if (dc == 0) row_max[RPP * i + row0] = a;
+    }
+    __syncthreads();
+    // rows r of class k in scale block g: (r % 8) in [k * cw, (k + 1) * cw), cw = 8 / ncls (a loop over
+    // those rows only)
+    const int cw = 1 << J.cls_shift;
+    auto class_max = [&](int g, int k) {
+      float a = 0.f;
+      const int r0 = GROUPED ? CR * g : 0, r1 = GROUPED ? r0 + CR : RPP;
+      for (int o = r0; o < r1; o += 8)
+        for (int m = 0; m < cw; m++) a = fmaxf(a, row_max[o + k * cw + m]);
+      return a;
+    };
+#pragma unroll
+    for (int i = 0; i < NA; i++) sc[i] = scale_of(class_max(GROUPED ? (RPP * i + row0) / (GROUPED ? CR : 1) : 0, cls));
+    if (tid < J.nsub * J.ncls) scale_at[tid] = scale_of(class_max(tid / J.ncls, tid % J.ncls));
+  } else {  // one scale per scale block: wave maxima, then over the waves (of each 32-row cell)
+    __shared__ float wave_maxes[NA][NW];
+#pragma unroll
+    for (int i = 0; i < NA; i++) {
+      const float a = wave_max(am[i]);
+      if ((tid & 63) == 0) wave_maxes[i][tid >> 6] = a;
+    }
+    __syncthreads();
+    float cell[NCELL];  // cell c: rows [CR c, CR c + CR) = the waves w of chunk i with (RPP i + RPW w) / CR == c
+#pragma unroll
+    for (int c = 0; c < NCELL; c++) {
+      cell[c] = amax0;
+#pragma unroll
+      for (int i = 0; i < NA; i++)
+#pragma unroll
+        for (int ww = 0; ww < NW; ww++)
+          if (!GROUPED || (RPP * i + RPW * ww) / (GROUPED ? CR : 1) == c) cell[c] = fmaxf(cell[c], wave_maxes[i][ww]);
+    }
+#pragma unroll
+    for (int i = 0; i < NA; i++) {
+      float a = cell[0];
+      if constexpr (CR == 32) {
+        // this thread's cell of chunk i: (RPP i + row0) / 32, row0 / 32 = RPW (tid / 64) / 32
+        a = cell[(RPP * i) / 32];
+        if constexpr (RPP > 32) {
+          if ((RPW * (tid >> 6)) / 32 == 1) a = cell[(RPP * i) / 32 + 1];
+        }
+      } else if constexpr (GROUPED) {
+        // this wave's cell of chunk i (a wave's RPW rows of a pass lie in one cell)
+        const int idx = (RPP * i + RPW * (tid >> 6)) / CR;
+#pragma unroll
+        for (int c = 1; c < NCELL; c++)
+          if (idx == c) a = cell[c];
+      }
+      sc[i] = VARIANT == QATTN_QUANT_CUDA ? quant_recip_cuda(a) : scale_of(a);
+    }
+#pragma unroll
+    for (int c = 0; c < NCELL; c++)
+      if (tid == c && c < J.nsub) scale_at[c] = scale_of(cell[c]);
+  }
+
+#pragma unroll
+  for (int i = 0; i < MAXC; i++) {
+    const int r = row0 + RPP * i;
+    const int64_t l = (int64_t)n * blk + r;
+    if (r < blk && l < Lb) {
+      const float s = sc[GROUPED ? i : 0];
+      const float iv = VARIANT == QATTN_QUANT_CUDA ? s : refined_rcp(s);
+      int8_t qv[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        // |x| <= amax, so the quotients stay within [-127, 127] before rounding (no saturation step);
+        // NaN converts to 0
+        if constexpr (VARIANT == QATTN_QUANT_CUDA) {
+          // cvt.rni.sat.s8.f32: round to nearest even
+          qv[e] = (int8_t)quant_code_cuda(x[i][e], iv);
+        } else {
+          // Triton: t + 0.5 * sign(t) in fp32, truncate toward zero
+          qv[e] = (int8_t)quant_code_triton(x[i][e], s, iv);
+        }
+      }
+      v2u packed;
+      __builtin_memcpy(&packed, qv, 8);
+      *reinterpret_cast<v2u*>(out_b + l * J.ol + (int64_t)h * J.oh + dc * 8) = packed;
+    }
+  }
+}
+
+template <bool IS_FP16, int VARIANT, int D, int QCR, bool HALFV>
+__global__ __launch_bounds__(512) void sage_small_kernel(SmallArgs a) {
+  constexpr int TPR = D / 8;
+  const int tid = threadIdx.x;
+  uint32_t wg = blockIdx.x;
+  if (wg < a.nvwg) {
+    constexpr int kWord = HALFV ? 8 : 4;  // bytes of a key quad in its channel's row
+    __shared__ __align__(16) uint8_t tile[2][D][16 * kWord];
+    __shared__ float recp[D], mean[D];
+    const uint32_t bh = wg / a.nvt, x = wg - bh * a.nvt;
+    const uint32_t b = bh / (uint32_t)a.H, h = bh - b * (uint32_t)a.H;
+    if constexpr (!HALFV) {
+      if (tid < D) {  // as prep_finalize_kernel
+        float am, mn = 0.f;
+        if (a.smooth_v) {
+          const float sum = reduce_chunks<0, D, 3>(a.vpart, bh, a.nchunk, tid, 0);
+          float hi = reduce_chunks<1, D, 3>(a.vpart, bh, a.nchunk, tid, 1);
+          float lo = reduce_chunks<2, D, 3>(a.vpart, bh, a.nchunk, tid, 2);
+          const int64_t l16 = (a.L + 15) / 16 * 16;
+          if (l16 != a.L) {
+            hi = fmaxf(hi, 0.f);
+            lo = fminf(lo, 0.f);
+          }
+          mn = sum / (float)l16;
+          am = fmaxf(fabsf(hi - mn), fabsf(lo - mn));
+        } else {
+          am = reduce_chunks<1, D>(a.vpart, bh, a.nchunk, tid);
+        }
+        recp[tid] = a.scale_max / am;
+        mean[tid] = mn;
+        if (x == 0) {
+          a.v_scale[(int64_t)bh * D + tid] = am / a.scale_max;
+          if (a.smooth_v) a.v_mean[(int64_t)bh * D + tid] = mn;
+        }
+      }
+    }
+    const int half = tid >> 8, t256 = tid & 255;  // each half of the workgroup takes a tile
+    const int64_t t = (int64_t)x * 2 + half;
+    const bool act = (t + 1) * 64 <= a.Lpad;
+    const int q = t256 / TPR, dc = t256 % TPR;
+    const bool lane = act && t256 < 16 * TPR;
+    uint16_t hv[4][8];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int64_t l = t * 64 + 4 * q + r;
+      v4u raw = {0u, 0u, 0u, 0u};
+      if (lane && l < a.L) raw = *reinterpret_cast<const v4u*>(a.v + b * a.vsb + l * a.vsl + h * a.vsh + dc * 8);
+      __builtin_memcpy(hv[r], &raw, 16);
+    }
+    if constexpr (!HALFV) __syncthreads();
+    const int wi = vtile_pos(4 * q) >> 2;
+    if (lane) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const int d = dc * 8 + e;
+        if constexpr (HALFV) {  // as v_tile_half_kernel
+          uint16_t y[4];
+#pragma unroll
+          for (int r = 0; r < 4; r++) y[r] = !IS_FP16 && a.conv ? f32_to_f16(bf16_to_f32(hv[r][e])) : hv[r][e];
+          v2u word;
+          __builtin_memcpy(&word, y, 8);
+          *reinterpret_cast<v2u*>(&tile[half][d][((((wi >> 1) ^ (dc & 7)) << 1) + (wi & 1)) * 8]) = word;
+        } else {  // as v_fp8_kernel
+          uint32_t word = 0;
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const float xf = half_to_f32<IS_FP16>(hv[r][e]);
+            const float y = t * 64 + 4 * q + r < a.L ? (a.smooth_v ? (xf - mean[d]) * recp[d] : xf * recp[d]) : 0.f;
+            word |= (uint32_t)f32_to_e4m3_sat(y) << (8 * r);
+          }
+          *reinterpret_cast<uint32_t*>(&tile[half][d][(wi ^ ((dc & 3) << 2)) * 4]) = word;
+        }
+      }
+    }
+    __syncthreads();
+    if (!act) return;
+    constexpr int CPR = kWord;  // 16-byte chunks per channel row
+    for (int c = t256; c < D * CPR; c += 256) {
+      const int d = c / CPR, cc = c % CPR, sc = cc ^ ((d >> 3) & (CPR - 1));
+      const v4u val = *reinterpret_cast<const v4u*>(&tile[half][d][sc * 16]);
+      if constexpr (HALFV) *reinterpret_cast<v4u*>(a.v16 + ((int64_t)bh * D + d) * a.Lpad + t * 64 + cc * 8) = val;
+      else *reinterpret_cast<v4u*>(a.v8 + ((int64_t)bh * D + d) * a.Lpad + t * 64 + cc * 16) = val;
+    }
+    return;
+  }
+  wg -= a.nvwg;
+  if (wg < (uint32_t)a.k.nwg) {
+    __shared__ __align__(16) uint16_t km[D];
+    if (a.kmean) {
+      uint32_t n, h, b;
+      quant_index(a.k, wg, n, h, b);
+      const int64_t bh = (int64_t)b * a.k.H + h;
+      if (tid < D) {
+        const uint16_t m = f32_to_half<IS_FP16>(reduce_chunks<0, D>(a.kpart, bh, a.nchunk, tid) / (float)a.L);
+        km[tid] = m;
+        if (n == 0) a.kmean[bh * D + tid] = m;
+      }
+      __syncthreads();
+    }
+    quant_block<IS_FP16, VARIANT, D, 0>(a.k, wg, a.kmean ? km : nullptr);
+    return;
+  }
+  wg -= (uint32_t)a.k.nwg;
+  quant_block<IS_FP16, VARIANT, D, QCR>(a.q, wg, nullptr);
+}
+
+// ------------------------------------------------------------------------------------------------
 // RMSNorm statistics: rstd = 1 / sqrt(mean(x^2) + eps) per row, one wave per row.  The squares of half
 // values are exact in fp64 and so is their sum for any realistic row, which makes the mean independent
 // of the summation order; var is then rounded to fp32 and the rest is IEEE fp32 (sqrt, division).
@@ -1333,6 +1652,35 @@ extern "C" int qattn_v_tile_half_varlen_ex(qattn_seq v, int dtype, int out_dtype
 // the whole SAGE prologue: K mean, Q/K INT8, V FP8 in four launches
 // ------------------------------------------------------------------------------------------------
 
+// Whether the prologue runs as column pass + sage_small_kernel: its workgroups re-read their head's partials
+// (nchunk x D floats each), which has to stay small beside the launches saved (measured: see sage_small_kernel).
+static bool small_prologue(const SmallArgs& a) {
+  return a.nchunk <= kSmallChunks && a.nvwg + a.k.nwg + a.q.nwg <= kSmallWorkgroups;
+}
+
+template <bool F16, int VARIANT, int D, int QCR, bool HALFV>
+static void launch_small_one(const SmallArgs& a, hipStream_t st) {
+  sage_small_kernel<F16, VARIANT, D, QCR, HALFV><<<(unsigned)(a.nvwg + a.k.nwg + a.q.nwg), 512, 0, st>>>(a);
+}
+
+// (D 64 on the FP8 V side only; the Triton per-block rounding on the half V side only)
+template <bool HALFV>
+static void launch_small(const SmallArgs& a, int dtype, int64_t D, int variant, int qcr, hipStream_t st) {
+#define QATTN_SM(F16, V, DD, C) launch_small_one<F16, V, DD, C, HALFV>(a, st)
+#define QATTN_SM2(F16, DD)                                                             \
+  if (variant == QATTN_QUANT_TRITON_THREAD) QATTN_SM(F16, QATTN_QUANT_TRITON_THREAD, DD, 32); \
+  else if (HALFV && variant == QATTN_QUANT_TRITON) QATTN_SM(F16, HALFV ? QATTN_QUANT_TRITON : QATTN_QUANT_CUDA, DD, 0); \
+  else if (qcr == 32) QATTN_SM(F16, QATTN_QUANT_CUDA, DD, 32);                         \
+  else QATTN_SM(F16, QATTN_QUANT_CUDA, DD, 0)
+  if (dtype == QATTN_BF16) {
+    if (HALFV || D == 128) { QATTN_SM2(false, 128); } else { QATTN_SM2(false, (HALFV ? 128 : 64)); }
+  } else {
+    if (HALFV || D == 128) { QATTN_SM2(true, 128); } else { QATTN_SM2(true, (HALFV ? 128 : 64)); }
+  }
+#undef QATTN_SM2
+#undef QATTN_SM
+}
+
 extern "C" size_t qattn_sage_quant_workspace_size(int64_t B, int64_t Lk, int64_t Hkv, int64_t D) {
   const int64_t n = B * Hkv * col_chunks(Lk) * D;
   return (size_t)(n + 3 * n + B * Hkv * D) * sizeof(float);
@@ -1387,25 +1735,7 @@ extern "C" int qattn_sage_quant(qattn_seq q, qattn_seq k, qattn_seq v, int dtype
 #undef QATTN_PC2
 #undef QATTN_PC
   }
-  // 2. K mean and V scales, one launch
-  {
-    const int64_t boff = smooth_k ? 0 : BH;
-    const unsigned g = (unsigned)(2 * BH - boff);
-#define QATTN_PF(F16, SV, DD) \
-  prep_finalize_kernel<F16, SV, DD><<<g, DD, 0, st>>>(kpart, vpart, nchunk, Lk, BH, km, scale_max, v_scale, recp, v_mean, boff)
-#define QATTN_PF2(F16, DD) \
-  if (smooth_v) QATTN_PF(F16, true, DD); else QATTN_PF(F16, false, DD)
-    if (dtype == QATTN_BF16) { if (D == 128) { QATTN_PF2(false, 128); } else { QATTN_PF2(false, 64); } }
-    else { if (D == 128) { QATTN_PF2(true, 128); } else { QATTN_PF2(true, 64); } }
-#undef QATTN_PF2
-#undef QATTN_PF
-  }
-  // 3. V to FP8 tiles (V was read by step 1 just before: its second read finds much of it in cache)
-  {
-    const VTileFilter nof{nullptr, {0, 0, 0, 0}};
-    launch_v_fp8(dtype, D, vp, v, Lk, B, Hkv, recp, v8, Lpad, Lpad / 64, nof, smooth_v ? v_mean : nullptr, st);
-  }
-  // 4. K then Q to INT8 in one launch (K first: its rows were read by step 1 as well)
+  // (K first: its rows were read by step 1 as well)
   QuantArgs a{};
   a.njobs = 0;
   // per-thread scales: the Triton rounding for K (and Q); otherwise the CUDA rounding
@@ -1432,6 +1762,118 @@ extern "C" int qattn_sage_quant(qattn_seq q, qattn_seq k, qattn_seq v, int dtype
       }
     }
   }
+  if (!sm90) {
+    SmallArgs sa{};
+    sa.k = a.job[0];
+    if (a.njobs > 1) sa.q = a.job[1];
+    sa.kpart = kpart;
+    sa.vpart = vpart;
+    sa.nchunk = nchunk;
+    sa.kmean = smooth_k ? km : nullptr;
+    sa.v = vp;
+    sa.vsb = v.sb; sa.vsl = v.sl; sa.vsh = v.sh;
+    sa.L = Lk; sa.H = Hkv;
+    sa.Lpad = Lpad;
+    sa.nvt = (uint32_t)((Lpad / 64 + 1) / 2);
+    sa.nvwg = (uint32_t)(BH * sa.nvt);
+    sa.v8 = v8;
+    sa.scale_max = scale_max;
+    sa.smooth_v = smooth_v;
+    sa.v_scale = v_scale; sa.v_mean = v_mean;
+    if (small_prologue(sa)) {
+      launch_small<false>(sa, dtype, D, variant, a.njobs > 1 ? a.job[1].cr : 0, st);
+      return check_launch("sage_quant");
+    }
+  }
+  // 2. K mean and V scales, one launch
+  {
+    const int64_t boff = smooth_k ? 0 : BH;
+    const unsigned g = (unsigned)(2 * BH - boff);
+#define QATTN_PF(F16, SV, DD) \
+  prep_finalize_kernel<F16, SV, DD><<<g, DD, 0, st>>>(kpart, vpart, nchunk, Lk, BH, km, scale_max, v_scale, recp, v_mean, boff)
+#define QATTN_PF2(F16, DD) \
+  if (smooth_v) QATTN_PF(F16, true, DD); else QATTN_PF(F16, false, DD)
+    if (dtype == QATTN_BF16) { if (D == 128) { QATTN_PF2(false, 128); } else { QATTN_PF2(false, 64); } }
+    else { if (D == 128) { QATTN_PF2(true, 128); } else { QATTN_PF2(true, 64); } }
+#undef QATTN_PF2
+#undef QATTN_PF
+  }
+  // 3. V to FP8 tiles (V was read by step 1 just before: its second read finds much of it in cache)
+  {
+    const VTileFilter nof{nullptr, {0, 0, 0, 0}};
+    launch_v_fp8(dtype, D, vp, v, Lk, B, Hkv, recp, v8, Lpad, Lpad / 64, nof, smooth_v ? v_mean : nullptr, st);
+  }
+  // 4. K then Q to INT8 in one launch
   if ((rc = check_launch("sage_quant"))) return rc;
   return run_quant(a, dtype, D, variant, st);
+}
+
+// The prologue of the half-P.V paths: K mean, Q / K to INT8 and V into half tiles, the bits of qattn_seq_mean + the
+// quantizers + qattn_v_tile_half_ex.  Small inputs take two launches, others five.
+extern "C" int qattn_sage_quant_half(qattn_seq q, qattn_seq k, qattn_seq v, int dtype, int v_dtype, int tile_dtype,
+                                     int64_t B, int64_t Lq, int64_t Lk, int64_t Hq, int64_t Hkv, int64_t D,
+                                     int qk_quant_gran, int variant, float q_sm_scale, int smooth_k, qattn_seq q_out,
+                                     float* q_scale, qattn_seq k_out, float* k_scale, void* k_mean, uint16_t* v16,
+                                     int64_t Lpad, void* workspace, size_t workspace_bytes, qattn_stream_t stream) {
+  int rc;
+  if ((rc = check_common(dtype, D, variant, 64)) || (rc = check_common(v_dtype, D, variant, 64)) ||
+      (rc = check_tile_dtype(v_dtype, tile_dtype)))
+    return rc;
+  QATTN_REQUIRE(qk_quant_gran >= 1 && qk_quant_gran <= 3, QATTN_ERR_ARG,
+                "qk_quant_gran must be 1 (per block), 2 (per warp) or 3 (per thread), got %d", qk_quant_gran);
+  QATTN_REQUIRE(B > 0 && Lq >= 0 && Lk > 0 && Hq > 0 && Hkv > 0, QATTN_ERR_SHAPE, "sage_quant_half needs non-empty K / V");
+  if ((Lq > 0 && ((rc = check_seq("q", q, 2)) || (rc = check_seq("q_out", q_out, 1)))) ||
+      (rc = check_seq("k", k, 2)) || (rc = check_seq("v", v, 2)) || (rc = check_seq("k_out", k_out, 1)))
+    return rc;
+  QATTN_REQUIRE((Lq == 0 || q_scale) && k_scale && v16 && aligned16(v16), QATTN_ERR_ARG, "null or misaligned output");
+  QATTN_REQUIRE(!smooth_k || (k_mean && aligned16(k_mean)), QATTN_ERR_ALIGN, "smooth_k needs an aligned k_mean output");
+  QATTN_REQUIRE(Lpad >= (Lk + 63) / 64 * 64 && Lpad % 64 == 0, QATTN_ERR_SHAPE,
+                "Lpad must be a multiple of 64 and >= Lk rounded up to 64");
+  QATTN_REQUIRE(!smooth_k || (workspace && workspace_bytes >= qattn_seq_mean_workspace_size(B, Lk, Hkv, D)),
+                QATTN_ERR_WORKSPACE, "sage_quant_half workspace too small");
+  hipStream_t st = (hipStream_t)stream;
+  const int var = qk_quant_gran == 3 ? QATTN_QUANT_TRITON_THREAD : qk_quant_gran == 2 ? QATTN_QUANT_CUDA : variant;
+  QuantArgs a{};
+  a.njobs = 1;
+  fill_job(a.job[0], k, k_out, B, Lk, Hkv, smooth_k ? k_mean : nullptr, k_scale, 1.0f, 0, 64);
+  if (qk_quant_gran == 3) {
+    a.job[0].ncls = 4;
+    a.job[0].cls_shift = 1;
+  }
+  if (Lq > 0) {
+    QuantJob& J = a.job[a.njobs++];
+    if (qk_quant_gran == 1) {
+      fill_job(J, q, q_out, B, Lq, Hq, nullptr, q_scale, q_sm_scale, 1, 128);
+    } else {
+      fill_job(J, q, q_out, B, Lq, Hq, nullptr, q_scale, 1.0f, 0, 32);
+      warp_block_job(J, B);
+      if (qk_quant_gran == 3) {
+        J.ncls = 8;
+        J.cls_shift = 0;
+      }
+    }
+  }
+  SmallArgs sa{};
+  sa.k = a.job[0];
+  if (a.njobs > 1) sa.q = a.job[1];
+  sa.nchunk = col_chunks(Lk);
+  sa.kpart = static_cast<float*>(workspace);
+  sa.kmean = smooth_k ? static_cast<uint16_t*>(k_mean) : nullptr;
+  sa.v = static_cast<const uint16_t*>(v.data);
+  sa.vsb = v.sb; sa.vsl = v.sl; sa.vsh = v.sh;
+  sa.L = Lk; sa.H = Hkv;
+  sa.Lpad = Lpad;
+  sa.nvt = (uint32_t)((Lpad / 64 + 1) / 2);
+  sa.nvwg = (uint32_t)(B * Hkv * sa.nvt);
+  sa.v16 = v16;
+  sa.conv = v_dtype != tile_dtype;
+  // (the kernel takes q, k and v of one dtype)
+  if (D == 128 && v_dtype == dtype && small_prologue(sa)) {
+    if (smooth_k) launch_col<0>(k, dtype, B, Lk, Hkv, D, sa.nchunk, static_cast<float*>(workspace), st);
+    launch_small<true>(sa, dtype, D, var, a.njobs > 1 ? a.job[1].cr : 0, st);
+    return check_launch("sage_quant_half");
+  }
+  if (smooth_k && (rc = qattn_seq_mean(k, dtype, B, Lk, Hkv, D, k_mean, workspace, workspace_bytes, stream))) return rc;
+  if ((rc = qattn_v_tile_half_ex(v, v_dtype, tile_dtype, B, Lk, Hkv, D, v16, Lpad, stream))) return rc;
+  return run_quant(a, dtype, D, var, st);
 }

@@ -234,6 +234,41 @@ def sage_quant(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tensor_layout:
     return q_int8, q_scale, k_int8, k_scale, km, v_fp8, v_scale, vm
 
 
+def sage_quant_half(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tensor_layout: str = "HND",
+                    qk_quant_gran: str = "per_block", sm_scale: Optional[float] = None, smooth_k: bool = True,
+                    variant: str = "cuda", fp16_v: bool = False):
+    """The prologue of the half-P.V paths: the outputs, bit for bit, of k_mean + per_block_int8 (``variant``) /
+    per_warp_int8 / per_thread_int8 + v_tile_half (``fp16_v``: v_tile_fp16).  Small inputs take two launches.
+    Returns (q_int8, q_scale, k_int8, k_scale, km or None, v_tiles)."""
+    L = _lib.load()
+    if q.dtype != k.dtype:
+        raise ValueError("q and k must have the same dtype")
+    b, lq, hq, d = _dims(q, tensor_layout)
+    _, lk, hkv, _ = _dims(k, tensor_layout)
+    dev = q.device
+    vdt = _lib.dtype_code(v.dtype)
+    if fp16_v:
+        v, vdt = _tile_input_fp16(v)
+    gran, nqb, nkb = _GRAN[qk_quant_gran], *_scale_blocks(lq, lk, False)
+    q_int8 = torch.empty(q.shape, dtype=torch.int8, device=dev)
+    k_int8 = torch.empty(k.shape, dtype=torch.int8, device=dev)
+    q_scale = torch.empty((b, hq, nqb * {1: 1, 2: 4, 3: 32}[gran]), dtype=torch.float32, device=dev)
+    k_scale = torch.empty((b, hkv, nkb * (4 if gran == 3 else 1)), dtype=torch.float32, device=dev)
+    km = torch.empty((b, hkv, d), dtype=k.dtype, device=dev) if smooth_k else None
+    lpad = (lk + 63) // 64 * 64
+    tiles = torch.empty((b, hkv, d, lpad), dtype=torch.float16 if fp16_v else v.dtype, device=dev)
+    ws = torch.empty(L.qattn_seq_mean_workspace_size(b, lk, hkv, d), dtype=torch.uint8, device=dev)
+    if sm_scale is None:
+        sm_scale = d ** -0.5
+    _lib.check(L.qattn_sage_quant_half(
+        _lib.seq(q, tensor_layout), _lib.seq(k, tensor_layout), _lib.seq(v, tensor_layout), _lib.dtype_code(q.dtype),
+        vdt, _lib.dtype_code(tiles.dtype), b, lq, lk, hq, hkv, d, gran,
+        _lib.QATTN_QUANT_TRITON if variant == "triton" else _lib.QATTN_QUANT_CUDA, float(sm_scale * LOG2E),
+        int(bool(smooth_k)), _lib.seq(q_int8, tensor_layout), _lib.ptr(q_scale), _lib.seq(k_int8, tensor_layout),
+        _lib.ptr(k_scale), _lib.ptr(km), _lib.ptr(tiles), lpad, _lib.ptr(ws), ws.numel(), _lib.stream_of(q)))
+    return q_int8, q_scale, k_int8, k_scale, km, tiles
+
+
 def v_tile_half(v: torch.Tensor, tensor_layout: str = "HND") -> torch.Tensor:
     """V in the kernels' transposed tile layout, in its own dtype: [B, H, D, Lpad] (bf16/fp16 P.V path)."""
     L = _lib.load()
@@ -485,21 +520,13 @@ def _sage_forward(q, k, v, tensor_layout, is_causal, qk_quant_gran, sm_scale, pv
         q_int8, q_scale, k_int8, k_scale, km, v_fp8, v_scale, vm = sage_quant(
             q, k, v, tensor_layout=tensor_layout, qk_quant_gran=qk_quant_gran, sm_scale=sm_scale, smooth_k=smooth_k,
             scale_max=scale_max, smooth_v=smooth_v)
-    else:
-        km = k_mean(k, tensor_layout) if smooth_k else None
-        if qk_quant_gran == "per_block":
-            q_int8, q_scale, k_int8, k_scale = per_block_int8(q, k, km, BLKQ, BLKK, sm_scale=sm_scale,
-                                                              tensor_layout=tensor_layout, variant=quant_variant)
-        else:  # sm_scale stays out of Q and is applied by the attention kernel (sm89 kernel :136,318-323)
-            quant = per_thread_int8 if qk_quant_gran == "per_thread" else per_warp_int8
-            q_int8, q_scale, k_int8, k_scale = quant(q, k, km, tensor_layout=tensor_layout)
-        if pv == "fp8":
-            v_fp8, v_scale, vm = per_channel_fp8(v, tensor_layout=tensor_layout, scale_max=scale_max,
-                                                 smooth_v=smooth_v)
-        else:
-            if smooth_v:
-                warnings.warn(f"pv_accum_dtype is '{pv_accum_dtype}', smooth_v will be ignored.")
-            v_fp8, v_scale = v_tile_half(v, tensor_layout), None
+    else:  # half P.V (sm_scale stays out of per-warp / per-thread Q: the attention kernel applies it)
+        if smooth_v:
+            warnings.warn(f"pv_accum_dtype is '{pv_accum_dtype}', smooth_v will be ignored.")
+        q_int8, q_scale, k_int8, k_scale, km, v_fp8 = sage_quant_half(
+            q, k, v, tensor_layout=tensor_layout, qk_quant_gran=qk_quant_gran, sm_scale=sm_scale, smooth_k=smooth_k,
+            variant=quant_variant)
+        v_scale = None
     res = qattn_fwd(q_int8, q_scale, k_int8, k_scale, v_fp8, v_scale, tensor_layout=tensor_layout, out_dtype=dtype,
                     qk_mult=qk_mult, is_causal=is_causal, q_offset=q_offset, kv_valid_len=kv_valid_len,
                     return_lse=return_lse, qk_quant_gran=qk_quant_gran, v_mean=vm,
@@ -698,6 +725,7 @@ __all__ = [
     "quant_per_block_int8",
     "per_channel_fp8",
     "sage_quant",
+    "sage_quant_half",
     "k_mean",
     "qattn_fwd",
     "sageattn",

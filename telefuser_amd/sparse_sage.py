@@ -47,10 +47,9 @@ def sparse_sageattn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask_id: 
     mask = mask_id.to(device=q.device, dtype=torch.int8)
     if mask.stride(-1) != 1 or mask.stride(0) != hkv * mask.stride(1):
         mask = mask.contiguous()
-    km = sa.k_mean(k, tensor_layout)
-    q8, qs, k8, ks = sa.per_block_int8(q, k, km, sa.BLKQ, sa.BLKK, sm_scale=d ** -0.5, tensor_layout=tensor_layout,
-                                       variant="triton")
-    vt = sa.v_tile_fp16(v, tensor_layout)  # the reference runs P.V in fp16
+    # (the reference runs P.V in fp16)
+    q8, qs, k8, ks, _, vt = sa.sage_quant_half(q, k, v, tensor_layout=tensor_layout, sm_scale=d ** -0.5,
+                                               variant="triton", fp16_v=True)
     o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     ns = L.qattn_fwd_block_sparse_num_splits(b, lq, lk, hq)
     wsb = L.qattn_fwd_workspace_size(b, lq, hq, d, ns)

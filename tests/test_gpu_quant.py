@@ -340,3 +340,57 @@ def test_v_tile_fp16_converts_as_torch(layout, L, D):
         want = torch.zeros(got.shape, dtype=torch.float16)
         want[..., slot] = rows.permute(0, 2, 3, 1)
         assert torch.equal(got.cpu().view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("gran,variant", [("per_block", "cuda"), ("per_block", "triton"), ("per_warp", "cuda"),
+                                          ("per_thread", "cuda")])
+@pytest.mark.parametrize("B,Lq,Lk,Hq,Hkv,layout,dtype,D,smooth_k,fp16_v", [
+    (1, 1, 1, 1, 1, "NHD", torch.bfloat16, 128, True, True),
+    (2, 130, 65, 4, 2, "HND", torch.bfloat16, 128, True, False),
+    (1, 300, 700, 3, 3, "NHD", torch.float16, 128, False, False),
+    (1, 64, 32 * 256, 2, 1, "NHD", torch.bfloat16, 128, True, True),      # the last size of the two-launch form
+    (1, 64, 32 * 256 + 1, 2, 1, "NHD", torch.bfloat16, 128, True, True),  # the first of the general one
+    (1, 200, 130, 2, 2, "HND", torch.bfloat16, 64, True, False),          # head_dim 64: general form
+])
+def test_sage_quant_half_matches_separate_calls(gran, variant, B, Lq, Lk, Hq, Hkv, layout, dtype, D, smooth_k, fp16_v):
+    dev = require_gpu()
+    from telefuser_amd import sageattn2 as sa
+
+    q, k, v = (t.to(dev) for t in qkv(B, Lq, Lk, Hq, Hkv, D=D, seed=Lk, k_offset_std=0.5, dtype=dtype))
+    if layout == "HND":
+        q, k, v = (t.transpose(1, 2).contiguous() for t in (q, k, v))
+    log(f"sage_quant_half {gran} {variant} {layout} {dtype} Lq={Lq} Lk={Lk} D={D}")
+    got = sa.sage_quant_half(q, k, v, tensor_layout=layout, qk_quant_gran=gran, smooth_k=smooth_k, variant=variant,
+                             fp16_v=fp16_v)
+    km = sa.k_mean(k, layout) if smooth_k else None
+    if gran == "per_block":
+        want = sa.per_block_int8(q, k, km, tensor_layout=layout, variant=variant)
+    else:
+        want = (sa.per_warp_int8 if gran == "per_warp" else sa.per_thread_int8)(q, k, km, tensor_layout=layout)
+    tiles = sa.v_tile_fp16(v, layout) if fp16_v else sa.v_tile_half(v, layout)
+    for name, x, y in zip(("q_int8", "q_scale", "k_int8", "k_scale", "km", "v"), got, (*want, km, tiles)):
+        assert (x is None and y is None) or torch.equal(x, y), name
+
+
+@pytest.mark.parametrize("Lk", [64, 65, 32 * 256, 32 * 256 + 1])
+@pytest.mark.parametrize("gran", ["per_block", "per_warp", "per_thread"])
+@pytest.mark.parametrize("quantize_q,smooth_v,D", [(True, False, 128), (False, True, 128), (True, True, 64)])
+def test_sage_quant_around_the_small_form(gran, quantize_q, smooth_v, D, Lk):
+    """The two-launch prologue of small inputs and the general one on both sides of its limit: the bits of the
+    separate calls."""
+    dev = require_gpu()
+    from telefuser_amd import sageattn2 as sa
+
+    q, k, v = (t.to(dev) for t in qkv(2, 70, Lk, 2, 1, D=D, seed=Lk, k_offset_std=0.5))
+    log(f"sage_quant small form {gran} Lk={Lk} D={D}")
+    q8, qs, k8, ks, km, v8, vs, vm = sa.sage_quant(q, k, v, tensor_layout="NHD", qk_quant_gran=gran, smooth_v=smooth_v,
+                                                   quantize_q=quantize_q)
+    km2 = sa.k_mean(k, "NHD")
+    quant = {"per_block": sa.per_block_int8, "per_warp": sa.per_warp_int8, "per_thread": sa.per_thread_int8}[gran]
+    want = quant(q, k, km2, tensor_layout="NHD")
+    wv = sa.per_channel_fp8(v, "NHD", smooth_v=smooth_v)
+    if quantize_q:
+        assert torch.equal(q8, want[0]) and torch.equal(qs, want[1])
+    assert torch.equal(k8, want[2]) and torch.equal(ks, want[3]) and torch.equal(km, km2)
+    assert torch.equal(v8.view(torch.uint8), wv[0].view(torch.uint8)) and torch.equal(vs, wv[1])
+    assert vm is None or torch.equal(vm, wv[2])
