@@ -93,39 +93,39 @@ struct AttnParams {
   int64_t n_chunk;
 };
 
-__device__ __forceinline__ uint32_t xcd_remap(uint32_t bid, uint32_t n) {
-  const uint32_t q = n / 8, r = n % 8;
-  const uint32_t xcd = bid % 8, idx = bid / 8;
+__device__ __forceinline__ int64_t xcd_remap(int64_t bid, int64_t n) {
+  const int64_t q = n / 8, r = n % 8;
+  const int64_t xcd = bid % 8, idx = bid / 8;
   return xcd * q + (xcd < r ? xcd : r) + idx;
 }
 
-// The KV split, (batch, head) and pair of query blocks of a workgroup (index math in 32 bits: the grid is below 2^31).
+// The KV split, (batch, head) and pair of query blocks of a workgroup.
 //   * Dense: consecutive pairs of one head on one XCD, sharing its K/V in the XCD's L2; splits outermost, so the
-//     workgroups of one key range of a head run next to each other.
-//   * Causal, unsplit: the longest pairs of all heads first.  Pair i costs about i + 1 key ranges; dealt in ascending
-//     order the long ones started last and the launch ended on a few CUs (2 x 4096 x 16 heads: the call 136 us against 122).
-//     Heads run innermost, so with a multiple of 8 of them a head still stays on one XCD.
-template <bool SPLIT>
+//     workgroups of one key range of a head run next to each other.  (64-bit divisions: with 32-bit ones the start-up
+//     is shorter, and 32760 x 32760 x 12 measured 0.8 % slower in every one of twelve interleaved rounds.)
+//   * Causal, unsplit (CAUSAL): the longest pairs of all heads first.  Pair i costs about i + 1 key ranges; dealt in
+//     ascending order the long ones started last and the launch ended on a few CUs.  Heads run innermost, so with a
+//     multiple of 8 of them a head still stays on one XCD.
+template <bool SPLIT, bool CAUSAL>
 __device__ __forceinline__ void pair_of_workgroup(const AttnParams& p, int& split, int64_t& b, int64_t& h, int64_t& qp) {
-  const uint32_t nQP = (uint32_t)(p.nQB + 1) / 2, BH = (uint32_t)(p.B * p.Hq);
-  uint32_t bh;
-  split = 0;
-  if (!SPLIT && p.causal) {
-    const uint32_t i = blockIdx.x / BH;
-    bh = blockIdx.x - i * BH;
+  const int64_t nQP = (p.nQB + 1) / 2;
+  if constexpr (CAUSAL && !SPLIT) {
+    const uint32_t BH = (uint32_t)(p.B * p.Hq), i = blockIdx.x / BH, bh = blockIdx.x - i * BH;
+    split = 0;
     qp = nQP - 1 - i;
-  } else {
-    uint32_t id = xcd_remap(blockIdx.x, gridDim.x);
-    if constexpr (SPLIT) {
-      split = (int)(id / (BH * nQP));
-      id -= (uint32_t)split * BH * nQP;
-    }
-    bh = id / nQP;
-    qp = id - bh * nQP;
+    const uint32_t bb = bh / (uint32_t)p.Hq;
+    b = bb;
+    h = bh - bb * (uint32_t)p.Hq;
+    return;
   }
-  const uint32_t bb = bh / (uint32_t)p.Hq;
-  b = bb;
-  h = bh - bb * (uint32_t)p.Hq;
+  const int64_t wg_id = xcd_remap(blockIdx.x, gridDim.x);
+  const int64_t n_pairs = p.B * p.Hq * nQP;
+  split = SPLIT ? (int)(wg_id / n_pairs) : 0;
+  const int64_t tile_id = SPLIT ? wg_id - (int64_t)split * n_pairs : wg_id;
+  qp = tile_id % nQP;
+  const int64_t rest = tile_id / nQP;
+  h = rest % p.Hq;
+  b = rest / p.Hq;
 }
 
 // Buffer resource (V#) for raw, unswizzled byte addressing of [base, base + bytes): loads whose offset

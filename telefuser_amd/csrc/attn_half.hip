@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kHFThreads) void qattn_fwd_half_kernel(AttnParams p
     nqb_wg_last = (int64_t)vq * 2 + 1;
   } else if constexpr (OWN) {
     const uint32_t units = (uint32_t)(p.B * p.Hq * p.nQB), wgs = (units + 1) / 2;
-    const uint32_t wg = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t wg = (uint32_t)xcd_remap(blockIdx.x, gridDim.x);
     split = SPLIT ? (int)(wg / wgs) : 0;
     unit0 = (wg - (uint32_t)split * wgs) * 2;
     const uint32_t u = unit0 + grp;
@@ -145,7 +145,8 @@ __global__ __launch_bounds__(kHFThreads) void qattn_fwd_half_kernel(AttnParams p
     nqb_wg_last = qb;
   } else {
     int64_t qp;
-    pair_of_workgroup<SPLIT>(p, split, b, h, qp);
+    if (!SPLIT && p.causal) pair_of_workgroup<SPLIT, true>(p, split, b, h, qp);
+    else pair_of_workgroup<SPLIT, false>(p, split, b, h, qp);
     qb = qp * 2 + grp;  // == nQB for the empty second group of an odd block count
     nqb_wg_last = min(qp * 2 + 1, p.nQB - 1);
   }
