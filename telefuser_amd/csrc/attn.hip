@@ -702,8 +702,14 @@ __device__ __forceinline__ void qattn_fwd_pp(const AttnParams& p) {
   auto stage_m = [&](int t, auto first_t) {
     constexpr bool kFirst = decltype(first_t)::value;
     if (!kFirst) read_v(t - 1);
-    read_k(t);
+    if constexpr (HD == 128) read_k(t);
     if (!kFirst) pv();
+    if constexpr (HD == 64) {
+      // (K's fragments behind P.V: V's registers are free by then, which is what fits 128 VGPRs; their latency is
+      // covered by the queued MFMAs and the SIMD's other pair)
+      __builtin_amdgcn_sched_barrier(0);
+      read_k(t);
+    }
     qk();
     // the logit scales of the tile, for the softmax of the next stage
     read_cs(t);
@@ -879,8 +885,14 @@ __device__ __forceinline__ void qattn_fwd_pp(const AttnParams& p) {
     p.lse[(b * p.Hq + h) * p.Lq + qrow] = l_tot > 0.f ? __builtin_log2f(l_tot) + m_run : -INFINITY;
 }
 
+// Head dim 64: the softmax per query-key pair does not shrink with the head dimension (~450 VALU cycles a tile against
+// 288 MFMA ones), so one pair of waves per SIMD left both pipes waiting.  Unsplit launches are held to 128 VGPRs: two
+// workgroups per CU (80 KiB of LDS each), two pairs per SIMD.  2 x 4680 x 4680 x 24 292 -> 238 us a call, 16000 x
+// 16000 x 12 608 -> 513, 30000 x 300 x 16 98 -> 62.  (Three waves per SIMD as three groups of one workgroup, the
+// softmax cut in two stages by a barrier: 285 us, and 4096 x 4096 x 24 slower, 160 against 136 us.  The KV-split form
+// spills 30 registers at 128 and keeps one workgroup per CU.)
 template <bool IS_FP16_OUT, bool KT, bool SPLIT, int HD, int QF, bool CA>
-__global__ __launch_bounds__(kPPThreads) void qattn_fwd_pp_kernel(AttnParams p) {
+__global__ __launch_bounds__(kPPThreads, HD == 64 && !SPLIT ? 4 : 1) void qattn_fwd_pp_kernel(AttnParams p) {
   qattn_fwd_pp<IS_FP16_OUT, KT, SPLIT, HD, QF, CA>(p);
 }
 
