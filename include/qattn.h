@@ -495,6 +495,18 @@ int qattn_norm_rope_quant_qk(qattn_seq xq, qattn_seq xk, int dtype, int64_t B, i
                              const float* sn, int64_t cs_stride, const void* k_mean, qattn_seq q_out,
                              qattn_seq k_out, float* q_scale, float* k_scale, float sm_scale, int variant,
                              qattn_stream_t stream);
+/*
+ * rstd of Q and K and (k_mean not null) the K mean of the rotated values in one pass: the same rstd bits as
+ * qattn_row_rstd, the mean as qattn_norm_rope_seq_mean with the rows summed in another order.  Rows of H * D values side
+ * by side (sh = D), at most 1536 of them (qattn_norm_rope_stats_supported).  Workspace (with k_mean):
+ * qattn_norm_rope_stats_workspace_size.
+ */
+int qattn_norm_rope_stats_supported(int64_t H, int64_t D);
+size_t qattn_norm_rope_stats_workspace_size(int64_t B, int64_t L, int64_t H, int64_t D);
+int qattn_norm_rope_stats(qattn_seq xq, qattn_seq xk, int dtype, int64_t B, int64_t L, int64_t H, int64_t D, float eps,
+                          const void* wk, const float* cs, const float* sn, int64_t cs_stride, float* rstd_q,
+                          float* rstd_k, void* k_mean, void* workspace, size_t workspace_bytes,
+                          qattn_stream_t stream);
 
 #ifdef __cplusplus
 }

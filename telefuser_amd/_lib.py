@@ -99,6 +99,11 @@ def load() -> ctypes.CDLL:
     L.qattn_fwd.argtypes = [S, vp, S, vp, vp, i64, vp, S, i32, i64, i64, i64, i64, i64, i64, f32, i32, i64, vp, vp,
                             i32, vp, sz, vp]
     L.qattn_v_tile_half.argtypes = [S, i32, i64, i64, i64, i64, vp, i64, vp]
+    L.qattn_norm_rope_stats_supported.argtypes = [i64, i64]
+    L.qattn_norm_rope_stats_supported.restype = i32
+    L.qattn_norm_rope_stats_workspace_size.argtypes = [i64, i64, i64, i64]
+    L.qattn_norm_rope_stats_workspace_size.restype = sz
+    L.qattn_norm_rope_stats.argtypes = [S, S, i32, i64, i64, i64, i64, f32, vp, vp, vp, i64, vp, vp, vp, vp, sz, vp]
     L.qattn_lse_finish.argtypes = [vp, S, i32, vp, i64, i64, i64, i64, i64, f32, vp]
     L.qattn_sage_quant_half.argtypes = [S, S, S, i32, i32, i32, i64, i64, i64, i64, i64, i64, i32, i32, f32, i32, S, vp,
                                         S, vp, vp, vp, i64, vp, sz, vp]
@@ -160,7 +165,7 @@ def load() -> ctypes.CDLL:
     L.qattn_v_tile_half_varlen.argtypes = [S, i32, i64, i64, i64, i64, i64, vp, vp, vp, i64, vp]
     L.qattn_fwd_varlen.argtypes = [S, vp, S, vp, vp, i64, S, i32, i64, i64, i64, i64, i64, i64, i64, i64, f32, i32, vp,
                                    vp, vp, vp, vp, vp]
-    for name in ("qattn_sage_quant_half", "qattn_lse_finish", "qattn_v_tile_half_ex", "qattn_v_tile_half_varlen_ex", "qattn_varlen_offsets", "qattn_quant_qk_varlen_int8", "qattn_v_tile_half_varlen",
+    for name in ("qattn_norm_rope_stats", "qattn_sage_quant_half", "qattn_lse_finish", "qattn_v_tile_half_ex", "qattn_v_tile_half_varlen_ex", "qattn_varlen_offsets", "qattn_quant_qk_varlen_int8", "qattn_v_tile_half_varlen",
                  "qattn_fwd_varlen"):
         getattr(L, name).restype = i32
     for name in ("qattn_row_rstd", "qattn_norm_rope_seq_mean", "qattn_norm_rope_quant_qk", "qattn_fwd_block_sparse", "qattn_quant_qk_per_warp_int8", "qattn_quant_qk_per_thread_int8", "qattn_fwd_ex",

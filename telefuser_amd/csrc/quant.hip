@@ -15,6 +15,18 @@ namespace qattn {
 // per-block INT8 quantizer
 // ------------------------------------------------------------------------------------------------
 
+// fp32 -> half dtype -> fp32, round to nearest even (bf16 through v_cvt_pk_bf16_f32: one instruction
+// instead of the integer sequence; the two differ only in the payload of a NaN, which quantizes to 0)
+template <bool IS_FP16>
+__device__ __forceinline__ float round_to_half(float v) {
+  if constexpr (IS_FP16) {
+    return f16_to_f32(f32_to_f16(v));
+  } else {
+    const __bf16 h = (__bf16)v;
+    return (float)h;
+  }
+}
+
 // Prologue of the Wan self-attention projections, applied on the fly to a 16-byte chunk (8 elements,
 // 4 rotation pairs) of head h, row l of the linear output x:
 //   RMSNorm over the full H*D row: y = half((x * rstd[b, l]) * w[h*D + d])  (norm_infer,
@@ -30,28 +42,35 @@ struct NormRope {
   int64_t cs_stride;
 };
 
+// (the values of the raw chunk hv, rounded to the half type after the norm and after the rotation, as fp32; the rounding
+// by the conversion instruction: the integer form cost ten of the quantizer's VALU instructions per element)
 template <bool IS_FP16>
-__device__ __forceinline__ void norm_rope8(const NormRope& nr, int64_t b, int64_t L, int64_t l, int64_t h, int D,
-                                           int dc, uint16_t (&hv)[8]) {
-  const float r = nr.rstd[b * L + l];
-  const v4u wr = *reinterpret_cast<const v4u*>(nr.w + h * D + dc * 8);
+__device__ __forceinline__ void norm_rope_values(float r, const v4u& wr, const v4f& c4, const v4f& s4,
+                                                 const uint16_t (&hv)[8], float (&out)[8]) {
   uint16_t wv[8];
   __builtin_memcpy(wv, &wr, 16);
-  const v4f c4 = *reinterpret_cast<const v4f*>(nr.cs + l * nr.cs_stride + dc * 4);
-  const v4f s4 = *reinterpret_cast<const v4f*>(nr.sn + l * nr.cs_stride + dc * 4);
   float y[8];
 #pragma unroll
   for (int e = 0; e < 8; e++) {
     const float xr = half_to_f32<IS_FP16>(hv[e]) * r;
-    y[e] = half_to_f32<IS_FP16>(f32_to_half<IS_FP16>(xr * half_to_f32<IS_FP16>(wv[e])));
+    y[e] = round_to_half<IS_FP16>(xr * half_to_f32<IS_FP16>(wv[e]));
   }
 #pragma unroll
   for (int p = 0; p < 4; p++) {
     const float y1 = y[2 * p], y2 = y[2 * p + 1];
     const float a = y1 * c4[p], bb = y2 * c4[p];
-    hv[2 * p] = f32_to_half<IS_FP16>(fmaf(-y2, s4[p], a));
-    hv[2 * p + 1] = f32_to_half<IS_FP16>(fmaf(y1, s4[p], bb));
+    out[2 * p] = round_to_half<IS_FP16>(fmaf(-y2, s4[p], a));
+    out[2 * p + 1] = round_to_half<IS_FP16>(fmaf(y1, s4[p], bb));
   }
+}
+
+template <bool IS_FP16>
+__device__ __forceinline__ void norm_rope8(const NormRope& nr, int64_t b, int64_t L, int64_t l, int64_t h, int D,
+                                           int dc, const uint16_t (&hv)[8], float (&out)[8]) {
+  const v4u wr = *reinterpret_cast<const v4u*>(nr.w + h * D + dc * 8);
+  const v4f c4 = *reinterpret_cast<const v4f*>(nr.cs + l * nr.cs_stride + dc * 4);
+  const v4f s4 = *reinterpret_cast<const v4f*>(nr.sn + l * nr.cs_stride + dc * 4);
+  norm_rope_values<IS_FP16>(nr.rstd[b * L + l], wr, c4, s4, hv, out);
 }
 
 // One quantizer job (Q or K).  A workgroup covers blk rows of one (batch entry, head): one scale block of
@@ -74,7 +93,7 @@ struct QuantJob {
   int64_t nwg;  // B * H * nblk
   int ncls;     // scale classes per scale block: 1 (per block), 8 (per-thread Q), 4 (per-thread K)
   int cls_shift;  // class of row r = (r % 8) >> cls_shift  (3, 0, 1 for the cases above)
-  NormRope nr;    // optional RMSNorm + RoPE prologue on the loaded chunks
+  NormRope nr;    // RMSNorm + RoPE prologue on the loaded chunks (the NR kernels)
   // packed variable-length input (null otherwise): entry b is rows cu_seq[b] .. cu_seq[b + 1] of batch 0, its
   // block n's scale goes to scale[(cu_blk[b] + n) * H + h] (quant_per_block_varlen.py:22-70)
   const int32_t* cu_seq;
@@ -93,27 +112,19 @@ constexpr int QATTN_QUANT_TRITON_THREAD = 2;
 // threads per quantizer workgroup: 512 (4 chunks of 16 bytes per thread at 128 rows and D = 128)
 template <int VARIANT> constexpr int quant_threads() { return 512; }
 
-// fp32 -> half dtype -> fp32, round to nearest even (bf16 through v_cvt_pk_bf16_f32: one instruction
-// instead of the integer sequence; the two differ only in the payload of a NaN, which quantizes to 0)
-template <bool IS_FP16>
-__device__ __forceinline__ float round_to_half(float v) {
-  if constexpr (IS_FP16) {
-    return f16_to_f32(f32_to_f16(v));
-  } else {
-    const __bf16 h = (__bf16)v;
-    return (float)h;
-  }
-}
-
 // One workgroup per block of one (batch entry, head) of a job; a launch covers up to two jobs (Q and K)
 // of equal cell layout (cr): workgroups [0, job[0].nwg) take job 0, the rest job 1.  Two passes over registers: |x|
 // maxima, then the scales and the quantized bytes.  GROUPED (CR = 32 or 16 rows per cell, nsub = blk / CR
 // cells): the block's rows are cells of CR rows with scales of their own, e.g. four
 // 32-row scale blocks; a wave's rows of one pass lie in one of them.
-// The plain kernel is held to 64 VGPRs: 4 workgroups (8 waves per SIMD) per CU instead of 3, worth more than
-// the two registers it spills.
-template <bool IS_FP16, int VARIANT, int D, int CR>
-__global__ __launch_bounds__(quant_threads<VARIANT>()) __attribute__((amdgpu_waves_per_eu(CR ? 7 : 8)))
+// The plain kernel is held to 64 VGPRs: 4 workgroups (8 waves per SIMD) per CU instead of 3.
+// NR: the job's norm + rope prologue on the loaded chunks, as instantiations of their own: the plain form then fits its
+// registers without spills, and this one is given the 66 it takes.  It is bound by the VALU work of the two roundings
+// and by the cos / sin rows, which come from L2 for every head (Q + K at 32760 x 12 x 128: 115 us with the integer
+// rounding, 98 with the conversion instruction).  A kernel that keeps a row's cos / sin in registers and walks the heads
+// took 118 us: it needs 128 registers and spills.
+template <bool IS_FP16, int VARIANT, int D, int CR, bool NR>
+__global__ __launch_bounds__(quant_threads<VARIANT>()) __attribute__((amdgpu_waves_per_eu(NR ? 6 : CR ? 7 : 8)))
 void quant_per_block_kernel(QuantArgs args) {
   constexpr bool GROUPED = CR != 0;
   constexpr int NCELL = GROUPED ? 128 / CR : 1;  // cells of a 128-row block
@@ -187,7 +198,6 @@ void quant_per_block_kernel(QuantArgs args) {
       v4u raw = *reinterpret_cast<const v4u*>(in_b + l * J.sl + (int64_t)h * J.sh + dc * 8);
       uint16_t hv[8];
       __builtin_memcpy(hv, &raw, 16);
-      if (J.nr.rstd) norm_rope8<IS_FP16>(J.nr, b, J.L, l, h, D, dc, hv);
       float mv[8];
       if (J.mean) {
         v4u mraw = *reinterpret_cast<const v4u*>(J.mean + (mb * J.H + h) * D + dc * 8);
@@ -196,9 +206,11 @@ void quant_per_block_kernel(QuantArgs args) {
 #pragma unroll
         for (int e = 0; e < 8; e++) mv[e] = half_to_f32<IS_FP16>(mh[e]);
       }
+      float nv[8];
+      if constexpr (NR) norm_rope8<IS_FP16>(J.nr, b, J.L, l, h, D, dc, hv, nv);
 #pragma unroll
       for (int e = 0; e < 8; e++) {
-        float v = half_to_f32<IS_FP16>(hv[e]);
+        float v = NR ? nv[e] : half_to_f32<IS_FP16>(hv[e]);
         if (J.mean) {
           v = v - mv[e];
           // Triton paths: k - km is a torch op on half tensors, rounded back to the half type
@@ -350,10 +362,16 @@ __device__ __forceinline__ void col_partial_body(const NormRope& nr, const uint1
       if (r + u * RPP < kColChunk && l < L) {
         uint16_t hv[8];
         __builtin_memcpy(hv, &raw[u], 16);
-        if (nr.rstd) norm_rope8<IS_FP16>(nr, b, L, l, h, D, dc, hv);
+        float xv[8];
+        if (nr.rstd) {
+          norm_rope8<IS_FP16>(nr, b, L, l, h, D, dc, hv, xv);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; e++) xv[e] = half_to_f32<IS_FP16>(hv[e]);
+        }
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-          float v = half_to_f32<IS_FP16>(hv[e]);
+          const float v = xv[e];
           if constexpr (MODE == 1) {
             acc[e] = fmaxf(acc[e], fabsf(v));
           } else {
@@ -771,7 +789,7 @@ __device__ __forceinline__ void quant_index(const QuantJob& J, uint32_t wg, uint
   }
 }
 
-// quant_per_block_kernel's block without its packed sequences and norm + rope, the row subtracted from every row
+// quant_per_block_kernel's block without its packed sequences, the row subtracted from every row
 // (mean: D half words in LDS, or null).  The two are kept apart: as one function the general kernel spilled nine
 // registers instead of one (45 -> 51 us for K at 32760 x 12).
 template <bool IS_FP16, int VARIANT, int D, int CR>
@@ -1078,6 +1096,114 @@ __global__ __launch_bounds__(256) void row_rstd_kernel(const uint16_t* x, int64_
 }
 
 // ------------------------------------------------------------------------------------------------
+// norm + rope prologue: rstd of Q and K and the column sums of the rotated K in one pass
+// ------------------------------------------------------------------------------------------------
+// A workgroup takes 16 .. 64 rows of Q or K (stat_rows); a wave takes a row at a time, 64 lanes x 16 bytes, and forms
+// rstd as row_rstd_kernel does (same lanes, same order: same bits).  For K it goes on with the row still in registers:
+// norm, rope and the column sums, for which the separate kernel reads K again and, walking heads outermost, the cos / sin
+// row once per head.  The chunks of a lane all have the same place in their heads (64 lanes are whole heads), so they
+// share the row's cos / sin here.  Q and K in one launch, 53 us at 32760 x 12 x 128 against 2 x 18.6 (rstd) + 44 (column
+// sums).
+struct StatArgs {
+  int64_t rows;             // rows per workgroup
+  const uint16_t *xq, *xk;  // rows of n half words
+  int64_t qsb, qsl, ksb, ksl;
+  int64_t B, L, n;          // n = H * D
+  float eps;
+  float *rstd_q, *rstd_k;   // [B * L]
+  NormRope nr;              // K's weights and the cos / sin tables
+  float* part;              // [B, H, nchunk, D] column sums of the rotated K, or null
+  int64_t nchunk;
+  uint32_t kwgs;            // workgroups of K (then Q's)
+};
+
+template <bool IS_FP16, int D, int JMAX>
+__global__ __launch_bounds__(512) void norm_stats_kernel(StatArgs a) {
+  extern __shared__ float colsum[];  // n floats (K with column sums)
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  uint32_t wg = blockIdx.x;
+  const bool is_k = wg < a.kwgs;
+  if (!is_k) wg -= a.kwgs;
+  const uint32_t nch = (uint32_t)a.nchunk;
+  const int64_t b = wg / nch, c0 = wg % nch;
+  const uint16_t* x = is_k ? a.xk + b * a.ksb : a.xq + b * a.qsb;
+  const int64_t sl = is_k ? a.ksl : a.qsl;
+  float* rstd = (is_k ? a.rstd_k : a.rstd_q) + b * a.L;
+  const bool sums = is_k && a.part;
+  const int nc = (int)(a.n / 8);  // 16-byte chunks per row
+  const int dc = lane % (D / 8);
+  float acc[JMAX][8];
+#pragma unroll
+  for (int j = 0; j < JMAX; j++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[j][e] = 0.f;
+  const int64_t r_end = min((c0 + 1) * a.rows, a.L);
+  v4u raw[JMAX];
+  auto load = [&](int64_t l) {
+#pragma unroll
+    for (int j = 0; j < JMAX; j++) {
+      const int c = lane + 64 * j;
+      raw[j] = v4u{0u, 0u, 0u, 0u};
+      if (c < nc && l < r_end) raw[j] = *reinterpret_cast<const v4u*>(x + l * sl + c * 8);
+    }
+  };
+  load(c0 * a.rows + w);
+  for (int64_t l = c0 * a.rows + w; l < r_end; l += 8) {
+    v4f c4, s4;
+    if (sums) {
+      c4 = *reinterpret_cast<const v4f*>(a.nr.cs + l * a.nr.cs_stride + dc * 4);
+      s4 = *reinterpret_cast<const v4f*>(a.nr.sn + l * a.nr.cs_stride + dc * 4);
+    }
+    uint16_t hv[JMAX][8];
+    double ss = 0.0;
+#pragma unroll
+    for (int j = 0; j < JMAX; j++) {
+      __builtin_memcpy(hv[j], &raw[j], 16);
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const double v = (double)half_to_f32<IS_FP16>(hv[j][e]);
+        ss += v * v;
+      }
+    }
+    load(l + 8);  // the wave's next row, behind this row's arithmetic
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    const float var = (float)(ss / (double)a.n);
+    const float r = 1.0f / sqrtf(var + a.eps);
+    if (lane == 0) rstd[l] = r;
+    if (sums) {
+#pragma unroll
+      for (int j = 0; j < JMAX; j++) {
+        const int c = lane + 64 * j;
+        if (c < nc) {
+          const v4u wr = *reinterpret_cast<const v4u*>(a.nr.w + c * 8);
+          float xv[8];
+          norm_rope_values<IS_FP16>(r, wr, c4, s4, hv[j], xv);
+#pragma unroll
+          for (int e = 0; e < 8; e++) acc[j][e] += xv[e];
+        }
+      }
+    }
+  }
+  if (!sums) return;
+  // the waves' sums, in wave order
+  for (int ww = 0; ww < 8; ww++) {
+    if (w == ww) {
+#pragma unroll
+      for (int j = 0; j < JMAX; j++) {
+        const int c = lane + 64 * j;
+        if (c < nc)
+#pragma unroll
+          for (int e = 0; e < 8; e++) colsum[c * 8 + e] = ww == 0 ? acc[j][e] : colsum[c * 8 + e] + acc[j][e];
+      }
+    }
+    __syncthreads();
+  }
+  const int64_t H = a.n / D;
+  for (int i = tid; i < a.n; i += 512) a.part[((b * H + i / D) * a.nchunk + c0) * D + i % D] = colsum[i];
+}
+
+// ------------------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------------------
 
@@ -1108,7 +1234,6 @@ static bool fill_job(QuantJob& J, const qattn_seq& in, const qattn_seq& out, int
   J.nwg = B * H * J.nblk;
   J.ncls = 1;
   J.cls_shift = 3;
-  J.nr = NormRope{};
   J.cu_seq = J.cu_blk = nullptr;
   J.total = 0;
   return true;
@@ -1131,7 +1256,7 @@ static void warp_block_job(QuantJob& J, int64_t B, int warp_rows = 32) {
 template <int D, int CR>
 static void launch_quant(const QuantArgs& a, int dtype, int variant, int64_t nwg, hipStream_t st) {
   dim3 grid((unsigned)nwg);
-#define QATTN_QK(F16, V) quant_per_block_kernel<F16, V, D, CR><<<grid, quant_threads<V>(), 0, st>>>(a)
+#define QATTN_QK(F16, V) quant_per_block_kernel<F16, V, D, CR, false><<<grid, quant_threads<V>(), 0, st>>>(a)
   if (dtype == QATTN_BF16) {
     if (variant == QATTN_QUANT_CUDA) QATTN_QK(false, QATTN_QUANT_CUDA);
     else if (variant == QATTN_QUANT_TRITON) QATTN_QK(false, QATTN_QUANT_TRITON);
@@ -1535,7 +1660,91 @@ extern "C" int qattn_norm_rope_quant_qk(qattn_seq xq, qattn_seq xk, int dtype, i
   fill_job(a.job[1], xk, k_out, B, L, H, k_mean, k_scale, 1.0f, 0, 64);
   if ((rc = make_norm_rope(a.job[0].nr, rstd_q, wq, cs, sn, cs_stride, D))) return rc;
   if ((rc = make_norm_rope(a.job[1].nr, rstd_k, wk, cs, sn, cs_stride, D))) return rc;
-  return run_quant(a, dtype, D, variant, (hipStream_t)stream);
+  const int64_t g = a.job[0].nwg + a.job[1].nwg;
+  QATTN_REQUIRE(g < (1ll << 31), QATTN_ERR_SHAPE, "quantizer grid too large");
+  hipStream_t st = (hipStream_t)stream;
+#define QATTN_NRQ(F16, V, DD) quant_per_block_kernel<F16, V, DD, 0, true><<<(unsigned)g, quant_threads<V>(), 0, st>>>(a)
+#define QATTN_NRQ2(F16, DD) \
+  if (variant == QATTN_QUANT_CUDA) QATTN_NRQ(F16, QATTN_QUANT_CUDA, DD); else QATTN_NRQ(F16, QATTN_QUANT_TRITON, DD)
+  if (dtype == QATTN_BF16) { if (D == 128) { QATTN_NRQ2(false, 128); } else { QATTN_NRQ2(false, 64); } }
+  else { if (D == 128) { QATTN_NRQ2(true, 128); } else { QATTN_NRQ2(true, 64); } }
+#undef QATTN_NRQ2
+#undef QATTN_NRQ
+  return check_launch("norm_rope_quant_qk");
+}
+
+// rows per workgroup of the statistics pass: enough workgroups of Q and K to fill 256 CUs twice over, 64 rows at most
+// (fewer, larger partial sums)
+static int64_t stat_rows(int64_t B, int64_t L) {
+  int64_t r = 64;
+  while (r > 16 && 2 * B * ((L + r - 1) / r) < 768) r /= 2;
+  return r;
+}
+static int64_t stat_chunks(int64_t B, int64_t L) { return (L + stat_rows(B, L) - 1) / stat_rows(B, L); }
+// widest row: 3 chunks per lane.  With 6 or 10 the row and its sums take 176 and 256 registers, two waves per SIMD, and one
+// pass is no faster than the separate kernels: the prologue at 2 x 3000 x 24 heads takes 64.7 us with those and 69.4 with
+// one pass, at 15399 x 40 heads 250.9 and 249.3
+constexpr int64_t kStatMaxCols = 64 * 8 * 3;
+
+extern "C" size_t qattn_norm_rope_stats_workspace_size(int64_t B, int64_t L, int64_t H, int64_t D) {
+  return (size_t)(B * H * stat_chunks(B, L) * D) * sizeof(float);
+}
+
+extern "C" int qattn_norm_rope_stats_supported(int64_t H, int64_t D) {
+  return (D == 64 || D == 128) && H > 0 && H * D <= kStatMaxCols;
+}
+
+extern "C" int qattn_norm_rope_stats(qattn_seq xq, qattn_seq xk, int dtype, int64_t B, int64_t L, int64_t H, int64_t D,
+                                     float eps, const void* wk, const float* cs, const float* sn, int64_t cs_stride,
+                                     float* rstd_q, float* rstd_k, void* k_mean, void* workspace,
+                                     size_t workspace_bytes, qattn_stream_t stream) {
+  int rc;
+  if ((rc = check_common(dtype, D, QATTN_QUANT_CUDA, 64))) return rc;
+  QATTN_REQUIRE(B > 0 && L > 0 && H > 0, QATTN_ERR_SHAPE, "norm_rope_stats needs non-empty input");
+  QATTN_REQUIRE(qattn_norm_rope_stats_supported(H, D), QATTN_ERR_SHAPE, "norm_rope_stats takes rows of at most %lld values",
+                (long long)kStatMaxCols);
+  if ((rc = check_seq("xq", xq, 2)) || (rc = check_seq("xk", xk, 2))) return rc;
+  QATTN_REQUIRE(xq.sh == D && xk.sh == D, QATTN_ERR_STRIDE, "norm_rope_stats takes rows with their heads side by side");
+  QATTN_REQUIRE(rstd_q && rstd_k, QATTN_ERR_ARG, "rstd is null");
+  StatArgs a{};
+  a.xq = static_cast<const uint16_t*>(xq.data);
+  a.xk = static_cast<const uint16_t*>(xk.data);
+  a.qsb = xq.sb; a.qsl = xq.sl; a.ksb = xk.sb; a.ksl = xk.sl;
+  a.B = B; a.L = L; a.n = H * D;
+  a.eps = eps;
+  a.rstd_q = rstd_q; a.rstd_k = rstd_k;
+  a.rows = stat_rows(B, L);
+  a.nchunk = stat_chunks(B, L);
+  if (k_mean) {
+    if ((rc = make_norm_rope(a.nr, rstd_k, wk, cs, sn, cs_stride, D))) return rc;
+    QATTN_REQUIRE(workspace && workspace_bytes >= qattn_norm_rope_stats_workspace_size(B, L, H, D), QATTN_ERR_WORKSPACE,
+                  "norm_rope_stats workspace too small");
+    a.part = static_cast<float*>(workspace);
+  }
+  const int64_t g = 2 * B * a.nchunk;
+  QATTN_REQUIRE(g < (1ll << 31), QATTN_ERR_SHAPE, "grid too large");
+  a.kwgs = (uint32_t)(B * a.nchunk);
+  hipStream_t st = (hipStream_t)stream;
+  const size_t lds = k_mean ? (size_t)a.n * sizeof(float) : 0;
+#define QATTN_ST(F16, DD, J) norm_stats_kernel<F16, DD, J><<<(unsigned)g, 512, lds, st>>>(a)
+#define QATTN_ST2(F16, DD)                   \
+  if (a.n <= 512) QATTN_ST(F16, DD, 1);      \
+  else QATTN_ST(F16, DD, 3)
+  if (dtype == QATTN_BF16) { if (D == 128) { QATTN_ST2(false, 128); } else { QATTN_ST2(false, 64); } }
+  else { if (D == 128) { QATTN_ST2(true, 128); } else { QATTN_ST2(true, 64); } }
+#undef QATTN_ST2
+#undef QATTN_ST
+  if (k_mean) {
+    uint16_t* m = static_cast<uint16_t*>(k_mean);
+    if (dtype == QATTN_BF16) {
+      if (D == 128) mean_finalize_kernel<false, 128><<<B * H, 128, 0, st>>>(a.part, a.nchunk, L, m);
+      else mean_finalize_kernel<false, 64><<<B * H, 64, 0, st>>>(a.part, a.nchunk, L, m);
+    } else {
+      if (D == 128) mean_finalize_kernel<true, 128><<<B * H, 128, 0, st>>>(a.part, a.nchunk, L, m);
+      else mean_finalize_kernel<true, 64><<<B * H, 64, 0, st>>>(a.part, a.nchunk, L, m);
+    }
+  }
+  return check_launch("norm_rope_stats");
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -24,6 +24,12 @@ def _cos_sin(freqs_cos: torch.Tensor, freqs_sin: torch.Tensor, L: int, half: int
     return cs, sn
 
 
+def _rows16(x: torch.Tensor) -> bool:
+    """x [B, L, N] as rows of 16-byte pieces: what the one-pass statistics read in place."""
+    return x.numel() > 0 and x.stride(-1) == 1 and x.data_ptr() % 16 == 0 and x.stride(0) % 8 == 0 and \
+        x.stride(1) % 8 == 0
+
+
 def row_rstd(x: torch.Tensor, eps: float) -> torch.Tensor:
     """1 / sqrt(mean(x^2, -1) + eps) per row of x [..., N] (fp32, shape x.shape[:-1])."""
     L = _lib.load()
@@ -55,15 +61,24 @@ def norm_rope_quant_qk(xq: torch.Tensor, xk: torch.Tensor, wq: torch.Tensor, wk:
     xq4, xk4 = xq.reshape(b, l, h, d), xk.reshape(b, l, h, d)
     cs, sn = _cos_sin(freqs_cos, freqs_sin, l, d // 2, xq.device)
     wq, wk = wq.to(xq.dtype).contiguous(), wk.to(xq.dtype).contiguous()
-    rq, rk = row_rstd(xq, eps), row_rstd(xk, eps)
     dt = _lib.dtype_code(xq.dtype)
-    km = None
-    if smooth_k:
-        km = torch.empty((b, h, d), dtype=xq.dtype, device=xq.device)
-        ws = torch.empty(L.qattn_seq_mean_workspace_size(b, l, h, d), dtype=torch.uint8, device=xq.device)
-        _lib.check(L.qattn_norm_rope_seq_mean(_lib.seq(xk4, "NHD"), dt, b, l, h, d, _lib.ptr(rk), _lib.ptr(wk),
-                                              _lib.ptr(cs), _lib.ptr(sn), cs.stride(0), _lib.ptr(km), _lib.ptr(ws),
-                                              ws.numel(), _lib.stream_of(xq)))
+    km = torch.empty((b, h, d), dtype=xq.dtype, device=xq.device) if smooth_k else None
+    if L.qattn_norm_rope_stats_supported(h, d) and _rows16(xq) and _rows16(xk):
+        # rstd of both and the K mean in one pass over Q and K
+        rq = torch.empty((b, l), dtype=torch.float32, device=xq.device)
+        rk = torch.empty((b, l), dtype=torch.float32, device=xq.device)
+        ws = torch.empty(L.qattn_norm_rope_stats_workspace_size(b, l, h, d) if smooth_k else 0, dtype=torch.uint8,
+                         device=xq.device)
+        _lib.check(L.qattn_norm_rope_stats(_lib.seq(xq4, "NHD"), _lib.seq(xk4, "NHD"), dt, b, l, h, d, float(eps),
+                                           _lib.ptr(wk), _lib.ptr(cs), _lib.ptr(sn), cs.stride(0), _lib.ptr(rq),
+                                           _lib.ptr(rk), _lib.ptr(km), _lib.ptr(ws), ws.numel(), _lib.stream_of(xq)))
+    else:
+        rq, rk = row_rstd(xq, eps), row_rstd(xk, eps)
+        if smooth_k:
+            ws = torch.empty(L.qattn_seq_mean_workspace_size(b, l, h, d), dtype=torch.uint8, device=xq.device)
+            _lib.check(L.qattn_norm_rope_seq_mean(_lib.seq(xk4, "NHD"), dt, b, l, h, d, _lib.ptr(rk), _lib.ptr(wk),
+                                                  _lib.ptr(cs), _lib.ptr(sn), cs.stride(0), _lib.ptr(km),
+                                                  _lib.ptr(ws), ws.numel(), _lib.stream_of(xq)))
     q8 = torch.empty((b, l, h, d), dtype=torch.int8, device=xq.device)
     k8 = torch.empty_like(q8)
     q_scale = torch.empty((b, h, (l + sa.BLKQ - 1) // sa.BLKQ), dtype=torch.float32, device=xq.device)
