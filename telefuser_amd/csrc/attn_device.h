@@ -355,10 +355,12 @@ __device__ __forceinline__ float quant_q_codes(const float (&x)[NQF][16], float 
   for (int m = 0; m < NQF; m++) {
     int c[16];
 #pragma unroll
-    for (int e = 0; e < 16; e++) c[e] = TRITON ? quant_code_triton(x[m][e], sc, iv) : quant_code_cuda(x[m][e], iv);
+    for (int e = 0; e < 16; e++) c[e] = TRITON ? quant_code_triton<true>(x[m][e], sc, iv) : quant_code_cuda(x[m][e], iv);
 #pragma unroll
     for (int g = 0; g < 4; g++)
-      qf[m][g] = (c[4 * g] & 0xff) | ((c[4 * g + 1] & 0xff) << 8) | ((c[4 * g + 2] & 0xff) << 16) | (c[4 * g + 3] << 24);
+      // (the low bytes of a pair by one v_perm_b32, then lshl_or: 3 instructions)
+      qf[m][g] = (int)(__builtin_amdgcn_perm((uint32_t)c[4 * g + 1], (uint32_t)c[4 * g], 0x0c0c0400u) |
+                       (__builtin_amdgcn_perm((uint32_t)c[4 * g + 3], (uint32_t)c[4 * g + 2], 0x0c0c0400u) << 16));
   }
   return sc;
 }

@@ -103,8 +103,19 @@ __device__ __forceinline__ float quant_scale_cuda(float amax) { return amax / 12
 __device__ __forceinline__ float quant_recip_cuda(float amax) { return 127.0f / amax; }
 __device__ __forceinline__ float quant_scale_triton(float amax) { return amax / 127.0f + 0.0000001f; }
 __device__ __forceinline__ int quant_code_cuda(float x, float recip) { return cvt_i32_trunc_sat(__builtin_rintf(x * recip)); }
+// HALF_X: x is a half-precision value.  With its 11 significant bits one correction of the quotient gives the correctly
+// rounded one for every pair of mantissas and every rcp within an ulp, but for a power of two over 2 - 2^-23, whose
+// neighbour has the same code (all 2^23 x 2^10 pairs were compared); half Q quantized inside the resident kernel spends
+// half of that kernel's VALU work here.
+template <bool HALF_X = false>
 __device__ __forceinline__ int quant_code_triton(float x, float scale, float rcp_scale) {
-  const float t = div_by(x, scale, rcp_scale);
+  float t;
+  if constexpr (HALF_X) {
+    const float q0 = x * rcp_scale;
+    t = fmaf(fmaf(-scale, q0, x), rcp_scale, q0);
+  } else {
+    t = div_by(x, scale, rcp_scale);
+  }
   return cvt_i32_trunc_sat(t + __builtin_copysignf(0.5f, t));
 }
 

@@ -313,7 +313,7 @@ void quant_per_block_kernel(QuantArgs args) {
           qv[e] = (int8_t)quant_code_cuda(x[i][e], iv);
         } else {
           // Triton: t + 0.5 * sign(t) in fp32, truncate toward zero
-          qv[e] = (int8_t)quant_code_triton(x[i][e], s, iv);
+          qv[e] = (int8_t)quant_code_triton<VARIANT == QATTN_QUANT_TRITON_THREAD>(x[i][e], s, iv);
         }
       }
       v2u packed;
@@ -948,7 +948,7 @@ __device__ __forceinline__ void quant_block(const QuantJob& J, uint32_t wg, cons
           qv[e] = (int8_t)quant_code_cuda(x[i][e], iv);
         } else {
           // Triton: t + 0.5 * sign(t) in fp32, truncate toward zero
-          qv[e] = (int8_t)quant_code_triton(x[i][e], s, iv);
+          qv[e] = (int8_t)quant_code_triton<VARIANT == QATTN_QUANT_TRITON_THREAD>(x[i][e], s, iv);
         }
       }
       v2u packed;

@@ -394,3 +394,32 @@ def test_sage_quant_around_the_small_form(gran, quantize_q, smooth_v, D, Lk):
     assert torch.equal(k8, want[2]) and torch.equal(ks, want[3]) and torch.equal(km, km2)
     assert torch.equal(v8.view(torch.uint8), wv[0].view(torch.uint8)) and torch.equal(vs, wv[1])
     assert vm is None or torch.equal(vm, wv[2])
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 128), (torch.float16, 64)])
+def test_per_thread_codes_near_ties(oracle, dtype, D):
+    """The per-thread codes where the quotient's last bit decides: values that are the half number next to a rounding
+    boundary (k + 1/2) scale, and its neighbours, for scales of every mantissa region (power-of-two quotients too)."""
+    dev = require_gpu()
+    from telefuser_amd import sageattn2 as sa
+
+    f16 = dtype is torch.float16
+    g = torch.Generator().manual_seed(5)
+    L, H = 2048, 4
+    nb = L // 32
+    # one |x| maximum per (32-row block, row % 8) class
+    amax = (torch.rand((1, nb, 8, H), generator=g, dtype=torch.float64) * 4 - 2).exp2().to(dtype)
+    scale = (amax.float() / 127 + 1e-7).double()
+    k = torch.randint(-127, 127, (1, nb, 4, 8, H, D), generator=g).double() + 0.5
+    x = (k * scale[:, :, None, :, :, None]).to(dtype)
+    step = torch.randint(-1, 2, x.shape, generator=g).to(torch.int16)
+    x = (x.view(torch.int16) + torch.where(x.abs() > 1e-3, step, torch.zeros_like(step))).view(dtype)
+    x = torch.minimum(torch.maximum(x, -amax[:, :, None, :, :, None]), amax[:, :, None, :, :, None])
+    x[:, :, 0, :, :, 0] = amax
+    x = x.reshape(1, L, H, D).contiguous()
+    log(f"per_thread codes near ties {dtype} D={D}")
+    q8, qs, k8, ks = sa.per_thread_int8(x.to(dev), x.to(dev), tensor_layout="NHD")
+    for (c, s), key in (((q8, qs), False), ((k8, ks), True)):
+        oc, os_ = oracle.quant_per_thread_int8(_as_bits(x), is_key=key, layout="NHD", is_fp16=f16)
+        np.testing.assert_array_equal(c.cpu().numpy(), oc)
+        np.testing.assert_array_equal(s.cpu().numpy().reshape(os_.shape), os_)
