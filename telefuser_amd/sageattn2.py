@@ -309,7 +309,17 @@ def _kv_valid_tensor(kv_valid_len, b: int, device) -> Optional[torch.Tensor]:
         t = t.expand(b)
     if t.numel() != b:
         raise ValueError(f"kv_valid_len must have {b} entries")
-    return t.to(device=device, dtype=torch.int32).contiguous()
+    if t.is_cuda or b == 0:
+        return t.to(device=device, dtype=torch.int32).contiguous()
+    # Host lengths: a copy from pageable memory waits for everything queued before it (the text cross-attention of 75600
+    # queries held the host for 512 us a call, 61 without).  Equal entries are a fill; others go through pinned
+    # memory, which the allocator keeps until the copy has run -- but not under capture, where a replay would read it again.
+    vals = t.reshape(-1).tolist()
+    if vals.count(vals[0]) == b:
+        return torch.full((b,), vals[0], dtype=torch.int32, device=device)
+    if torch.cuda.is_current_stream_capturing():
+        return t.to(device=device).contiguous()
+    return torch.tensor(vals, dtype=torch.int32, pin_memory=True).to(device=device, non_blocking=True)
 
 
 _GRAN = {"per_block": _lib.QATTN_GRAN_BLOCK, "per_warp": _lib.QATTN_GRAN_WARP, "per_thread": _lib.QATTN_GRAN_THREAD}

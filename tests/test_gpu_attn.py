@@ -1187,3 +1187,26 @@ def test_causal_work_order(oracle, B, L, Hq, Hkv, D, q_offset):
         assert lib.qattn_last_kernel() == _lib.QATTN_KERNEL_PINGPONG
     finally:
         lib.qattn_set_kernel(_lib.QATTN_KERNEL_AUTO)
+
+
+def test_kv_valid_len_forms():
+    """Every host form of kv_valid_len (int, equal and differing lists, tensors of either device) gives the lengths on
+    the device, unharmed by a later call that reuses the staging memory while the queue is still busy."""
+    dev = require_gpu()
+    from telefuser_amd.sageattn2 import _kv_valid_tensor
+
+    busy = torch.zeros((4096, 4096), device=dev)
+    forms = [(5, 3), ([7, 7, 7], 3), ([1, 2, 300], 3), (torch.tensor([4, 0]), 2), (torch.tensor([[9], [8]]), 2),
+             (torch.tensor([6, 5], dtype=torch.int64, device=dev), 2), ((11,), 1), ([], 0)]
+    got = []
+    for rep in range(20):
+        busy.add_(1)
+        got += [_kv_valid_tensor(f, b, dev) for f, b in forms]
+    torch.cuda.synchronize()
+    for i, t in enumerate(got):
+        f, b = forms[i % len(forms)]
+        assert t.is_cuda and t.dtype == torch.int32 and t.is_contiguous()
+        assert t.reshape(-1).tolist() == (torch.as_tensor(f).reshape(-1).tolist() * b if isinstance(f, int) else
+                                          torch.as_tensor(f).reshape(-1).tolist())
+    with pytest.raises(ValueError):
+        _kv_valid_tensor([1, 2], 3, dev)
