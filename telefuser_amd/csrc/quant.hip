@@ -590,6 +590,10 @@ __global__ __launch_bounds__(256) void v_fp8_kernel(const uint16_t* in, int64_t 
       act[tt] = (filt.r[0] < hi && lo < filt.r[1]) || (filt.r[2] < hi && lo < filt.r[3]);
     }
   }
+  // A streaming update that grew no scale leaves most tiles as they are: their workgroups end here (uniform, before the
+  // barrier) instead of converting zeros nobody stores (4680 new of 32760 slots x 12 heads: 21.7 -> 17.1 us).
+  static_assert(kVTilesPerWG == 2, "two flags");
+  if (!act[0] && !act[1]) return;
   // thread: key quad q (keys 4q .. 4q + 3 of a tile, which occupy consecutive slots) x 8 channels
   const int q = tid / TPR, dc = tid % TPR;
   const bool lane = tid < 16 * TPR;
