@@ -313,7 +313,7 @@ def _kv_valid_tensor(kv_valid_len, b: int, device) -> Optional[torch.Tensor]:
         return t.to(device=device, dtype=torch.int32).contiguous()
     # Host lengths: a copy from pageable memory waits for everything queued before it (the text cross-attention of 75600
     # queries held the host for 512 us a call, 61 without).  Equal entries are a fill; others go through pinned
-    # memory, which the allocator keeps until the copy has run -- but not under capture, where a replay would read it again.
+    # memory, which the allocator keeps until the copy has run -- but not under capture: a replay would read it again.
     vals = t.reshape(-1).tolist()
     if vals.count(vals[0]) == b:
         return torch.full((b,), vals[0], dtype=torch.int32, device=device)
