@@ -1214,43 +1214,81 @@ __global__ __launch_bounds__(kResThreads) void qattn_fwd_res_kernel(AttnParams p
   if constexpr (QF == QF_BLOCK) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no prefetch left in flight
 }
 
-// Merge the KV-split partials: one wave per query row, 2 channels per lane.
+// Merge the KV-split partials: four channels per lane, so a wave reads 1 KiB of whole rows of each split.  HBM- and
+// latency-bound ((D + 2) 4 bytes per row and split): the partials of four splits are loaded at once, the first four ahead
+// of the maxima, and the row is split into (batch, head, query) by 32-bit divisions where the rows fit them (one row per
+// wave, a split at a time and 64-bit divisions: 1560 x 12 rows 12.9 us, 10.0 now; a call at 300 x 20000 x 8 116 -> 110).
 template <bool IS_FP16_OUT, int HD = kD>
 __global__ __launch_bounds__(256) void qattn_combine_kernel(AttnParams p) {
-  constexpr int E = HD / 64;  // output elements per lane
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);  // over B*Hq*Lq
-  const int lane = threadIdx.x & 63;
+  constexpr int E = 4, TPR = HD / E;  // channels per lane, lanes per row
+  constexpr int NS = 4;               // splits loaded together
+  const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;  // over B*Hq*Lq
+  const int d0 = (threadIdx.x % TPR) * E;
   const int64_t total = p.B * p.Hq * p.Lq;
   if (row >= total) return;
-  const int64_t qrow = row % p.Lq;
-  const int64_t h = (row / p.Lq) % p.Hq;
-  const int64_t b = row / (p.Lq * p.Hq);
+  int64_t b, h, qrow;
+  if (total <= (int64_t)UINT32_MAX) {
+    const uint32_t r = (uint32_t)row, lq = (uint32_t)p.Lq, hq = (uint32_t)p.Hq;
+    const uint32_t bh = r / lq;
+    qrow = r - bh * lq;
+    b = bh / hq;
+    h = bh - (uint32_t)b * hq;
+  } else {
+    qrow = row % p.Lq;
+    h = (row / p.Lq) % p.Hq;
+    b = row / (p.Lq * p.Hq);
+  }
   const int64_t hk = h / p.group;
-  const int64_t sstride = total;
+  const int ns = p.nsplit;
+  // (past the last split the loads repeat it and are not used)
+  v4f part[NS];
+  auto load = [&](int s0) {
+#pragma unroll
+    for (int i = 0; i < NS; i++)
+      part[i] = *reinterpret_cast<const v4f*>(p.ws_o + (min(s0 + i, ns - 1) * total + row) * HD + d0);
+  };
+  load(0);
   float M = kMInit;
-  for (int s = 0; s < p.nsplit; s++) M = fmaxf(M, p.ws_ml[(s * sstride + row) * 2]);
+  for (int s0 = 0; s0 < ns; s0 += NS) {
+    float m[NS];
+#pragma unroll
+    for (int i = 0; i < NS; i++) m[i] = p.ws_ml[(min(s0 + i, ns - 1) * total + row) * 2];
+#pragma unroll
+    for (int i = 0; i < NS; i++) M = fmaxf(M, m[i]);
+  }
   float L = 0.f, a[E];
 #pragma unroll
   for (int e = 0; e < E; e++) a[e] = 0.f;
-  for (int s = 0; s < p.nsplit; s++) {
-    const float ms = p.ws_ml[(s * sstride + row) * 2], ls = p.ws_ml[(s * sstride + row) * 2 + 1];
-    const float f = __builtin_amdgcn_exp2f(ms - M);
-    L += ls * f;
-    const float* wo = p.ws_o + (s * sstride + row) * HD + lane * E;
+  for (int s0 = 0; s0 < ns; s0 += NS) {
+    if (s0) load(s0);
+    float m[NS], l[NS];
 #pragma unroll
-    for (int e = 0; e < E; e++) a[e] += wo[e] * f;
+    for (int i = 0; i < NS; i++) {
+      const float* ml = p.ws_ml + (min(s0 + i, ns - 1) * total + row) * 2;
+      m[i] = ml[0];
+      l[i] = ml[1];
+    }
+#pragma unroll
+    for (int i = 0; i < NS; i++) {
+      if (s0 + i >= ns) break;
+      const float f = __builtin_amdgcn_exp2f(m[i] - M);
+      L += l[i] * f;
+#pragma unroll
+      for (int e = 0; e < E; e++) a[e] += part[i][e] * f;
+    }
   }
   const float inv = L > 0.f ? 1.0f / L : 0.f;
-  const float* vs = p.v_scale ? p.v_scale + (b * p.Hkv + hk) * HD + lane * E : nullptr;
-  uint16_t* orow = static_cast<uint16_t*>(p.o) + b * p.osb + qrow * p.osl + h * p.osh + lane * E;
-  const float* vm = p.v_mean ? p.v_mean + (b * p.Hkv + hk) * HD + lane * E : nullptr;
+  const float* vs = p.v_scale ? p.v_scale + (b * p.Hkv + hk) * HD + d0 : nullptr;
+  const float* vm = p.v_mean ? p.v_mean + (b * p.Hkv + hk) * HD + d0 : nullptr;
+  float r[E];
 #pragma unroll
-  for (int e = 0; e < E; e++) {
-    const float r = vm ? epilogue_value<true>(a[e], inv, vs ? vs[e] : 1.f, vm[e])
-                       : epilogue_value<false>(a[e], inv, vs ? vs[e] : 1.f, 0.f);
-    orow[e] = f32_to_half<IS_FP16_OUT>(r);
-  }
-  if (p.lse && lane == 0) p.lse[(b * p.Hq + h) * p.Lq + qrow] = L > 0.f ? __builtin_log2f(L) + M : -INFINITY;
+  for (int e = 0; e < E; e++)
+    r[e] = vm ? epilogue_value<true>(a[e], inv, vs ? vs[e] : 1.f, vm[e])
+              : epilogue_value<false>(a[e], inv, vs ? vs[e] : 1.f, 0.f);
+  const v2u packed{pack_half2<IS_FP16_OUT>(r[0], r[1]), pack_half2<IS_FP16_OUT>(r[2], r[3])};
+  uint16_t* orow = static_cast<uint16_t*>(p.o) + b * p.osb + qrow * p.osl + h * p.osh + d0;
+  *reinterpret_cast<v2u*>(orow) = packed;
+  if (p.lse && d0 == 0) p.lse[(b * p.Hq + h) * p.Lq + qrow] = L > 0.f ? __builtin_log2f(L) + M : -INFINITY;
 }
 
 // Natural-log LSE of the original K from the kernels' log2-domain LSE against K - km: lse * ln 2 + (q . km) sm_scale,
@@ -1291,7 +1329,7 @@ __global__ __launch_bounds__(256) void lse_finish_kernel(float* lse, const uint1
 }
 
 void launch_combine(const AttnParams& p, int out_dtype, int64_t D, hipStream_t st) {
-  const int64_t g = (p.B * p.Hq * p.Lq + 3) / 4;
+  const int64_t per = 256 / (D / 4), g = (p.B * p.Hq * p.Lq + per - 1) / per;
   if (D == 64) {
     if (out_dtype == QATTN_BF16) qattn_combine_kernel<false, 64><<<g, 256, 0, st>>>(p);
     else qattn_combine_kernel<true, 64><<<g, 256, 0, st>>>(p);

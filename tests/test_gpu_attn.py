@@ -1210,3 +1210,12 @@ def test_kv_valid_len_forms():
                                           torch.as_tensor(f).reshape(-1).tolist())
     with pytest.raises(ValueError):
         _kv_valid_tensor([1, 2], 3, dev)
+
+
+@pytest.mark.parametrize("num_splits", [2, 4, 5, 11])
+def test_combine_split_counts(oracle, num_splits):
+    """The combine over fewer, exactly and more splits than it loads at once, rows that end inside its last workgroup,
+    and a batch entry whose last splits hold no valid key."""
+    require_gpu()
+    q, k, v = qkv(2, 131, 700, 3, 1, seed=77)
+    _run_and_check(oracle, q, k, v, num_splits=num_splits, kv_valid=[700, 150])
