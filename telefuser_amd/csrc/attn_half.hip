@@ -15,7 +15,7 @@
 // Measured against a kernel with one 128-row block and four waves per workgroup, two workgroups per CU, whose waves
 // fell into step (MFMAs, then softmax): 32760 x 32760 x 12 heads per-thread scales 5.31 -> 4.60 ms a call (1.43
 // PFLOP/s; without the softmax 3.4 ms, without the LDS reads 3.9, without the DMA 4.1), 8000 x 8000 x 2 129 -> 80 us,
-// 8 sequences of 257 .. 6240 tokens, 12 heads 1450 -> 390 us in the kernel (mostly HF_VAR's order of the work),
+// 8 sequences of 257 .. 6240 tokens, 12 heads 1467 -> 443 us in the kernel (mostly HF_VAR's order of the work),
 // block-sparse 32760 x 32760 x 12 at a quarter of the tiles 1440 -> 1330 us.
 //
 // Forms (one template axis):
