@@ -183,6 +183,17 @@ def per_channel_fp8(v: torch.Tensor, tensor_layout: str = "HND", scale_max: floa
     return v_fp8, v_scale, vm
 
 
+def _check_kv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout: str, exact: bool) -> None:
+    """The fused prologues address q, k and v with q's batch and head dim and k's heads and length: k and v have to
+    hold all of it (``exact``: and no other batch entries or heads; a v longer than k is read up to k's length)."""
+    b, _, _, d = _dims(q, layout)
+    bk, lk, hkv, dk = _dims(k, layout)
+    bv, lv, hv, dv = _dims(v, layout)
+    if dk != d or dv != d or bk < b or bv < b or hv < hkv or lv < lk or (exact and (bk, bv, hv) != (b, b, hkv)):
+        raise ValueError(f"k must have q's batch and head dim and v the shape of k, got q {tuple(q.shape)}, "
+                         f"k {tuple(k.shape)}, v {tuple(v.shape)} ({layout})")
+
+
 def sage_quant(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tensor_layout: str = "HND",
                qk_quant_gran: str = "per_block", sm_scale: Optional[float] = None, smooth_k: bool = True,
                scale_max: float = 448.0, smooth_v: bool = False, scale_layout: str = "sm89", quantize_q: bool = True):
@@ -204,6 +215,7 @@ def sage_quant(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tensor_layout:
     sm90 = scale_layout == "sm90"
     if sm90 and gran == 1:
         raise ValueError("scale_layout='sm90' needs qk_quant_gran 'per_warp' or 'per_thread'")
+    _check_kv(q, k, v, tensor_layout, False)
     b, lq, hq, d = _dims(q, tensor_layout)
     _, lk, hkv, _ = _dims(k, tensor_layout)
     dev = q.device
@@ -243,6 +255,7 @@ def sage_quant_half(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tensor_la
     L = _lib.load()
     if q.dtype != k.dtype:
         raise ValueError("q and k must have the same dtype")
+    _check_kv(q, k, v, tensor_layout, True)
     b, lq, hq, d = _dims(q, tensor_layout)
     _, lk, hkv, _ = _dims(k, tensor_layout)
     dev = q.device
