@@ -194,7 +194,9 @@ int qattn_per_channel_fp8_ex(qattn_seq v, int dtype, int64_t B, int64_t L, int64
  *   causal:   mask kv_idx > q_idx + q_offset (reference is_causal is top-left aligned, q_offset 0)
  *   kv_valid: NULL or device int32 [B]: keys >= kv_valid[b] are masked (key padding)
  *   lse:      NULL or fp32 [B, Hq, Lq] receiving log2(sum 2^s) of the quantized logits
- *   num_splits: 0 = automatic, 1 = no KV split, n > 1 = split keys over n workgroups
+ *   num_splits: 0 = automatic, 1 = no KV split, n > 1 = split keys over n workgroups.  A workgroup covers at most 7680
+ *               key tiles of 64 with FP8 V and 4096 with half V (per-thread scales: a quarter of that); longer key
+ *               ranges are split as often as that takes, whatever num_splits says
  *   workspace: needed when splitting, qattn_fwd_workspace_size bytes
  * D is 128, or 64 for FP8 V (dense launches: qattn_fwd / qattn_fwd_ex / _ex2 / _noalloc with v_kind FP8).
  * Callers pad other heads as sageattn2.py:1307-1316 does: D < 64 to 64, 64 < D < 128 to 128.  Head

@@ -1584,7 +1584,7 @@ static void plan_fwd(int64_t B, int64_t Lq, int64_t Lk, int64_t Hq, int pv, int 
                      int num_splits, int& ns, int& qpw, int& kernel) {
   const int64_t nQB = (Lq + kBQ - 1) / kBQ, nKB = (Lk + kBK - 1) / kBK;
   const int64_t max_tiles = pv == PV_FP8 ? max_tiles_per_split(is_thread_gran(gran))
-                                         : half_max_tiles(nQB, is_thread_gran(gran), sparse);
+                                         : half_max_tiles(is_thread_gran(gran), sparse);
   ns = num_splits > 0 ? num_splits
        : sparse       ? num_splits_for(B, Lq, Lk, Hq, max_tiles, false)
                       : dense_num_splits(B, Lq, Lk, Hq, pv, gran);

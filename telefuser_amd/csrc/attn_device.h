@@ -388,7 +388,7 @@ void launch_combine(const AttnParams& p, int out_dtype, int64_t D, hipStream_t s
 // split count of a dense launch
 int launch_half(AttnParams& p, bool kt, bool f16v, bool sparse, int out_dtype, int ns, hipStream_t st);
 int launch_half_varlen(AttnParams& p, int out_dtype, hipStream_t st);
-int64_t half_max_tiles(int64_t nqb, bool kt, bool sparse);
+int64_t half_max_tiles(bool kt, bool sparse);
 int half_num_splits(int64_t bh, int64_t nqb, int64_t nkb, bool kt);
 
 }  // namespace qattn

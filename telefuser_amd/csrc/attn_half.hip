@@ -23,7 +23,7 @@
 //   HF_VAR   the same over a packed variable-length batch: the workgroups find their (sequence, head, pair) in
 //            the device tables, longest key ranges first
 //   HF_OWN   each group takes a query block of its own (block-sparse masks, whose rows differ, and dense launches
-//            with one or three query blocks per head, where a pair would be half empty).  The tiles that both
+//            with one or three query blocks per head, where a pair would be half empty, up to half_own_tiles).  The tiles that both
 //            blocks visit come first, fetched once for both and five tiles ahead (their order follows the mask, so
 //            a third of the fetches miss L2); then each group streams what only its block visits.
 #include "attn_device.h"
@@ -626,14 +626,17 @@ __global__ __launch_bounds__(kHFThreads) void qattn_fwd_half_kernel(AttnParams p
 
 // A pair of query blocks per workgroup needs an even block count, or enough blocks that the idle second group of
 // the last pair does not matter (at most 1/6 of the groups); other launches give each group a block of its own.
-static bool half_pairs(int64_t nqb, bool sparse) { return !sparse && (nqb % 2 == 0 || nqb >= 5); }
-
-int64_t half_max_tiles(int64_t nqb, bool kt, bool sparse) {
-  return (half_pairs(nqb, sparse) ? kHFKsPair : kHFKsOwn) / ks_per_tile(kt);
+// A group of its own stages a quarter of a pair's k_scales, so key ranges past that (half_own_tiles) are pairs too.
+static bool half_even(int64_t nqb) { return nqb % 2 == 0 || nqb >= 5; }
+static int64_t half_own_tiles(bool kt) { return kHFKsOwn / ks_per_tile(kt); }
+static bool half_pairs(int64_t nqb, bool kt, bool sparse, int64_t tiles) {
+  return !sparse && (half_even(nqb) || tiles > half_own_tiles(kt));
 }
 
-static int64_t half_workgroups(int64_t bh, int64_t nqb, bool sparse) {
-  return half_pairs(nqb, sparse) ? bh * ((nqb + 1) / 2) : (bh * nqb + 1) / 2;
+int64_t half_max_tiles(bool kt, bool sparse) { return sparse ? half_own_tiles(kt) : kHFKsPair / ks_per_tile(kt); }
+
+static int64_t half_workgroups(int64_t bh, int64_t nqb, bool pairs) {
+  return pairs ? bh * ((nqb + 1) / 2) : (bh * nqb + 1) / 2;
 }
 
 // KV splits of a dense launch: the count that makes rounds of 256 workgroups (one per CU) x (key tiles + start-up
@@ -642,8 +645,9 @@ static int64_t half_workgroups(int64_t bh, int64_t nqb, bool sparse) {
 // a launch (~4 us).
 int half_num_splits(int64_t bh, int64_t nqb, int64_t nkb, bool kt) {
   if (bh <= 0 || nqb <= 0 || nkb <= 0) return 1;
-  const int64_t max_tiles = half_max_tiles(nqb, kt, false), min_s = (nkb + max_tiles - 1) / max_tiles;
-  const int64_t wgs = half_workgroups(bh, nqb, false);
+  const bool pairs = half_even(nqb);
+  const int64_t max_tiles = pairs ? half_max_tiles(kt, false) : half_own_tiles(kt), min_s = (nkb + max_tiles - 1) / max_tiles;
+  const int64_t wgs = half_workgroups(bh, nqb, pairs);
   int64_t best = min_s;
   double best_cost = 1e300;
   for (int64_t s = min_s; s <= std::max<int64_t>(min_s, std::min<int64_t>(32, nkb / 8)); s++) {
@@ -672,10 +676,10 @@ static void launch_form(const AttnParams& p, int64_t g, int out_dtype, bool f16v
 int launch_half(AttnParams& p, bool kt, bool f16v, bool sparse, int out_dtype, int ns, hipStream_t st) {
   p.nsplit = ns;
   p.tiles_per_split = (int)((p.nKB + ns - 1) / ns);
-  const bool pairs = half_pairs(p.nQB, sparse);
-  const int64_t g = half_workgroups(p.B * p.Hq, p.nQB, sparse) * ns;
+  const bool pairs = half_pairs(p.nQB, kt, sparse, p.tiles_per_split);
+  const int64_t g = half_workgroups(p.B * p.Hq, p.nQB, pairs) * ns;
   QATTN_REQUIRE(g < (1ll << 31), QATTN_ERR_SHAPE, "grid too large");
-  QATTN_REQUIRE(p.tiles_per_split <= half_max_tiles(p.nQB, kt, sparse), QATTN_ERR_SHAPE, "too many key tiles per workgroup");
+  QATTN_REQUIRE(p.tiles_per_split <= half_max_tiles(kt, sparse), QATTN_ERR_SHAPE, "too many key tiles per workgroup");
   if (pairs) {
     if (ns > 1) {
       if (kt) launch_form<true, true, HF_PAIR>(p, g, out_dtype, f16v, st);

@@ -1,11 +1,13 @@
 """The C-ABI library loads without a GPU, exports every symbol include/qattn.h declares, and its
-host-side validation reports errors as status codes (no GPU call is reached on these paths)."""
+host-side validation reports errors as status codes (no GPU call is reached on these paths, but for the half-V
+calls at the end, which run only where there is no GPU)."""
 
 import ctypes
 import os
 import re
 
 import pytest
+import torch
 
 from tests.conftest import ROOT
 
@@ -134,3 +136,31 @@ def test_kernel_selection_rule(lib):
     finally:
         lib.qattn_set_kernel(prev)
     assert lib.qattn_set_kernel(0) == 0
+
+
+# Half-V calls on made-up addresses, as far as the host side takes them: 7 is a workspace that does not do.  (On a
+# machine with a GPU they would be launched.)
+needs_no_gpu = pytest.mark.skipif(torch.cuda.is_available(), reason="the addresses are made up")
+
+
+def _half_call(lib, fn, B, Lq, Lk, H, gran, num_splits, ws_bytes=0):
+    s, buf = _seq(1 << 20, Lq * H * 128, H * 128, 128), ctypes.c_void_p(1 << 20)
+    lpad = -(-Lk // 64) * 64
+    args = (s, buf, s, buf, buf, 1, lpad, None, s, 0, B, Lq, Lk, H, H, 128, 1.0, gran, 0, 0, None, None, num_splits)
+    if fn == "noalloc":
+        return lib.qattn_fwd_ex_noalloc(*args, None)
+    return lib.qattn_fwd_ex(*args, buf if ws_bytes else None, ws_bytes, None)
+
+
+@needs_no_gpu
+@pytest.mark.parametrize("Lq,Lk,gran", [(100, 20032, 3), (300, 20032, 5), (128, 24576, 3), (300, 98304, 1),
+                                        (100, 65536, 3), (600, 65536, 3), (300, 262144, 2)])
+def test_one_split_needs_no_workspace(lib, Lq, Lk, gran):
+    assert _half_call(lib, "ex", 1, Lq, Lk, 2, gran, 1) not in (0, 7)
+    assert b"workspace" not in lib.qattn_last_error()
+
+
+@needs_no_gpu
+@pytest.mark.parametrize("Lk,gran", [(65537, 3), (262145, 1)])
+def test_one_split_past_the_staged_scales_is_refused(lib, Lk, gran):
+    assert _half_call(lib, "ex", 1, 300, Lk, 2, gran, 1) == 7

@@ -344,6 +344,19 @@ def test_half_pv_causal_split_padding(oracle):
     _run_and_check(oracle, q, k[:, :300], v[:, :300], pv="half", causal=True)
 
 
+@pytest.mark.parametrize("Lq,Lk,Hq,Hkv,gran,kw", [
+    # one and three query blocks over key ranges at and past what a group of its own stages (256 tiles per thread, 1024
+    # per block): unsplit launches go over to pairs there; the last two with a KV split whose runs are that long
+    (100, 16384, 2, 1, "per_thread", {}), (100, 16385, 2, 1, "per_thread", {}), (100, 20032, 2, 1, "per_thread", {}),
+    (300, 16448, 1, 1, "per_thread", dict(causal=True, q_offset=16148)), (300, 65600, 1, 1, "per_block", {}),
+    (300, 33000, 1, 1, "per_thread", dict(num_splits=2)), (100, 40000, 1, 1, "per_thread", dict(num_splits=2)),
+])
+def test_half_unsplit_long_keys(oracle, Lq, Lk, Hq, Hkv, gran, kw):
+    """num_splits is taken as given where the key range allows it, without a workspace for more splits."""
+    q, k, v = qkv(1, Lq, Lk, Hq, Hkv, seed=Lq + Lk, k_offset_std=0.5)
+    _run_and_check(oracle, q, k, v, pv="half", gran=gran, **dict(dict(num_splits=1), **kw))
+
+
 @pytest.mark.parametrize("Lq,Lk,Hq,Hkv,kw", [
     # pairs of query blocks: whole and odd counts, key ranges of 1 .. 5 tiles (three K / V buffers)
     (256, 1, 2, 2, {}), (200, 64, 2, 2, {}), (640, 65, 2, 1, {}), (256, 192, 2, 2, {}), (641, 300, 1, 1, {}),
