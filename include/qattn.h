@@ -312,7 +312,8 @@ int qattn_fwd_varlen(qattn_seq q8, const float* q_scale, qattn_seq k8, const flo
  * Quantized attention with INT8 Q.K^T and P.V in the half dtype of V (P rounded to that dtype,
  * fp32 accumulation, no FP8 offset or v_scale): the math of the reference's INT8-QK / FP16-PV kernels
  * (qk_int8_sv_f16_accum_f32_attn, common_extension.cc:214-218; Triton attn_qk_int8_per_block.py:46-101).
- * Arguments as qattn_fwd, with v16 from qattn_v_tile_half and v_dtype its dtype.
+ * Arguments as qattn_fwd, with v16 from qattn_v_tile_half and v_dtype its dtype; the workspace is sized with
+ * qattn_fwd_ex_num_splits for that v_kind.
  */
 int qattn_fwd_pv16(qattn_seq q8, const float* q_scale, qattn_seq k8, const float* k_scale, const uint16_t* v16,
                    int v_dtype, int64_t Lpad, qattn_seq o, int out_dtype, int64_t B, int64_t Lq, int64_t Lk,
@@ -378,7 +379,9 @@ int qattn_fwd_q16(qattn_seq q, qattn_seq k8, const float* k_scale, const uint8_t
  * per-thread scales sm_scale is not in Q: pass qk_mult = sm_scale * 1.44269504.
  *   v_kind QATTN_V_FP8: v = e4m3 tile layout + v_scale;  QATTN_V_BF16 / _FP16: v from qattn_v_tile_half.
  * The number of KV splits depends on v_kind and the granularity: size the workspace with
- * qattn_fwd_ex_num_splits (or pass an explicit num_splits >= it).
+ * qattn_fwd_ex_num_splits (or pass an explicit num_splits >= it).  Half V with num_splits = 0 splits no more than the
+ * given workspace holds; its full count evens out the rounds of workgroups of long calls too, whose partials (520 bytes
+ * per query row and split) can take hundreds of MB.
  */
 int qattn_fwd_ex_num_splits(int64_t B, int64_t Lq, int64_t Lk, int64_t Hq, int v_kind, int qk_quant_gran);
 /*
@@ -444,7 +447,8 @@ int qattn_fwd_ex2(qattn_seq q8, const float* q_scale, qattn_seq k8, const float*
  * HIP graph capture, tight serving loops).  No counterpart in the reference.  KV-split partials go to a
  * device array inside the library (one per GPU, held until the process ends) of at most
  * qattn_fwd_noalloc_max_scratch() bytes (128 MiB): a launch whose qattn_fwd_workspace_size(B, Lq, Hq, D,
- * splits) exceeds it fails with QATTN_ERR_WORKSPACE.  Calls never allocate device memory.  Launches that use
+ * splits) exceeds it fails with QATTN_ERR_WORKSPACE.  (Half V with num_splits = 0 splits no more than fits, down to
+ * what the key range needs.)  Calls never allocate device memory.  Launches that use
  * the array (KV-split launches) are ordered on the GPU in the order the host issues them, also from different
  * streams or threads: each waits (hipStreamWaitEvent, no host wait) for the previous one's completion event.
  * On a stream under graph capture that ordering is left to the graph: replays of a captured graph must not

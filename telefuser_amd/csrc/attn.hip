@@ -1692,6 +1692,15 @@ static int launch_gran(AttnParams& p, int gran, int out_dtype, int ns, void* ws,
   return launch_fwd<false>(p, out_dtype, ns, ws, wsb, st, D, kernel);
 }
 
+// half P.V: the automatic split count evens out the rounds of workgroups and takes its partials (520 bytes per row and
+// split, hundreds of MB for long calls) for granted; where the workspace holds fewer, the launch splits less, down to
+// what the staged k_scales need
+static int half_fit_splits(const AttnParams& p, int ns, bool kt, size_t bytes) {
+  const int64_t tiles = half_max_tiles(kt, false), min_ns = (p.nKB + tiles - 1) / tiles;
+  while (ns > min_ns && qattn_fwd_workspace_size(p.B, p.Lq, p.Hq, kD, ns) > bytes) ns--;
+  return ns;
+}
+
 // half P.V: the workspace of a KV split, then the launch (attn_half.hip)
 static int launch_half_ws(AttnParams& p, bool kt, bool f16v, bool sparse, int out_dtype, int ns, void* ws, size_t wsb,
                           hipStream_t st) {
@@ -1740,6 +1749,7 @@ extern "C" int qattn_fwd_ex2(qattn_seq q8, const float* q_scale, qattn_seq k8, c
     return launch_gran(p, qk_quant_gran, out_dtype, ns, workspace, workspace_bytes, st, D, kernel);
   }
   p.v_scale = nullptr;
+  if (num_splits <= 0) ns = half_fit_splits(p, ns, is_thread_gran(qk_quant_gran), workspace ? workspace_bytes : 0);
   return launch_half_ws(p, is_thread_gran(qk_quant_gran), pv == PV_FP16, false, out_dtype, ns, workspace,
                         workspace_bytes, st);
 }
@@ -1921,6 +1931,7 @@ extern "C" int qattn_fwd_ex_noalloc(qattn_seq q8, const float* q_scale, qattn_se
                            causal, q_offset, kv_valid, lse, num_splits, pv, qk_quant_gran, kernel);
   if (rc < 0) return QATTN_OK;
   if (rc) return rc;
+  if (pv != PV_FP8 && num_splits <= 0) ns = half_fit_splits(p, ns, is_thread_gran(qk_quant_gran), kScratchBytes);
   const size_t need = qattn_fwd_workspace_size(B, Lq, Hq, D, ns);
   QATTN_REQUIRE(need <= kScratchBytes, QATTN_ERR_WORKSPACE,
                 "qattn_fwd_ex_noalloc: %d KV splits need %zu bytes of scratch, more than its %zu-byte limit "

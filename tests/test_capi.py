@@ -164,3 +164,22 @@ def test_one_split_needs_no_workspace(lib, Lq, Lk, gran):
 @pytest.mark.parametrize("Lk,gran", [(65537, 3), (262145, 1)])
 def test_one_split_past_the_staged_scales_is_refused(lib, Lk, gran):
     assert _half_call(lib, "ex", 1, 300, Lk, 2, gran, 1) == 7
+
+
+@needs_no_gpu
+@pytest.mark.parametrize("fn", ["noalloc", "ex"])
+@pytest.mark.parametrize("B,H,Lq,Lk,gran", [(1, 12, 12288, 12288, 1), (1, 16, 4680, 16384, 1), (1, 12, 6400, 32760, 1),
+                                            (1, 40, 3600, 65536, 1), (1, 8, 75600, 65536, 3)])
+def test_automatic_splits_fit_the_workspace(lib, fn, B, H, Lq, Lk, gran):
+    """The automatic count of these is more than 128 MiB of partials: it gives way to the scratch array's size, or to a
+    workspace that is not there."""
+    ns = lib.qattn_fwd_ex_num_splits(B, Lq, Lk, H, 1, gran)
+    assert lib.qattn_fwd_workspace_size(B, Lq, H, 128, ns) > lib.qattn_fwd_noalloc_max_scratch()
+    assert _half_call(lib, fn, B, Lq, Lk, H, gran, 0) not in (0, 7)
+    # (a count that the caller asks for is not lowered)
+    assert _half_call(lib, "ex", B, Lq, Lk, H, gran, ns) == 7
+
+
+@needs_no_gpu
+def test_forced_splits_past_the_scratch_are_refused(lib):
+    assert _half_call(lib, "noalloc", 1, 75600, 75600, 40, 3, 0) == 7  # two splits at least: 3.1 GB of partials

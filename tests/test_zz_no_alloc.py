@@ -132,3 +132,31 @@ def test_noalloc_head_dim_64():
         torch.cuda.synchronize()
         assert torch.equal(o0, o1) and torch.equal(l0, l1)
         assert bool(torch.isfinite(o1.float()).all())
+
+
+@pytest.mark.parametrize("Lq,Lk,H,ns", [(12288, 12288, 12, 1), (4680, 16384, 16, 3)])
+def test_noalloc_half_v_splits_what_fits(Lq, Lk, H, ns):
+    """Half V whose automatic count (two and four splits) is more than the scratch holds: as many as fit, the bits of
+    qattn_fwd_ex with that count; and the same for a workspace of that many splits."""
+    dev = require_gpu()
+    from telefuser_amd import _lib
+    from telefuser_amd import sageattn2 as sa
+
+    L = _lib.load()
+    log(f"noalloc half V: Lq={Lq} Lk={Lk} H={H} splits={ns}")
+    assert L.qattn_fwd_ex_num_splits(1, Lq, Lk, H, _lib.QATTN_V_BF16, 1) > ns
+    q, k, v = (t.to(dev) for t in qkv(1, Lq, Lk, H, H, seed=600 + ns, k_offset_std=0.5))
+    q8, qs, k8, ks, _, vt = sa.sage_quant_half(q, k, v, tensor_layout="NHD")
+    wsb = L.qattn_fwd_workspace_size(1, Lq, H, 128, ns)
+    ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device=dev)
+
+    def call(fn, splits, *tail):
+        o = torch.empty_like(q)
+        _lib.check(fn(_lib.seq(q8, "NHD"), _lib.ptr(qs), _lib.seq(k8, "NHD"), _lib.ptr(ks), _lib.ptr(vt),
+                      _lib.QATTN_V_BF16, vt.shape[-1], None, _lib.seq(o, "NHD"), _lib.QATTN_BF16, 1, Lq, Lk, H, H, 128,
+                      1.0, _lib.QATTN_GRAN_BLOCK, 0, 0, None, None, splits, *tail, _lib.stream_of(q8)))
+        return o
+
+    want = call(L.qattn_fwd_ex, ns, _lib.ptr(ws), wsb)
+    assert torch.equal(call(L.qattn_fwd_ex_noalloc, 0), want)
+    assert torch.equal(call(L.qattn_fwd_ex, 0, _lib.ptr(ws), wsb), want)
