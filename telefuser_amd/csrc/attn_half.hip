@@ -51,49 +51,67 @@ struct HalfVec<true> {
   typedef _Float16 elem;
 };
 
-// Work item of workgroup g of a packed batch: sequences in order of decreasing key count (ties by index; within
-// each run of 64 sequences), each as head-major pairs of query blocks, so the longest workgroups start first and
-// the launch ends evenly.  (Dealt by sequence, one long sequence kept a single XCD busy for most of the launch.)
-// Every lane of the wave gets the same answer; false past the last item.
-__device__ __forceinline__ bool varlen_item(const AttnParams& p, int g, int& b_out, int& h_out, int& qp_out, int& n_out) {
-  const int lane = threadIdx.x & 63;
-  int start = 0;  // pairs of the runs before this one
-  for (int base = 0; base < (int)p.B; base += 64) {
-    const int b = base + lane;
+// A sequence of a packed batch: its pairs of query blocks and its key count, none and -1 where it has no keys or its V
+// tile range runs past Lpad (a too small Lpad leaves the sequence's rows untouched).
+__device__ __forceinline__ void varlen_pairs(const AttnParams& p, int b, int& n, int& key) {
+  int64_t r0, lq, lk;
+  varlen_range(p.cu_k, b, p.var_tk, p.Lk, r0, lk);
+  varlen_range(p.cu_q, b, p.var_tq, p.Lq, r0, lq);
+  n = 0;
+  key = -1;
+  if (lk > 0 && ((int64_t)p.cu_vt[b] + (lk + kBK - 1) / kBK) * kBK <= p.Lpad) {
+    n = (int)((lq + 2 * kBQ - 1) / (2 * kBQ));
+    key = (int)lk;
+  }
+}
+
+// Work item of workgroup g of a packed batch.  Every lane of the wave gets the same answer; false if g has none.
+//   * Up to kVarSorted sequences: in order of decreasing key count (ties by index), each as head-major pairs of query
+//     blocks, so the longest workgroups start first and the launch ends evenly.  (Dealt by sequence, one long sequence
+//     kept a single XCD busy for most of the launch.)
+//   * More: in sequence order with the heads innermost.  Sequence b starts at slot (cu_qs[b] + b) / 2 of each head, which
+//     leaves room for its ceil(blocks / 2) pairs and at most one slot more, so that the block offsets are all the
+//     search needs: 64 of them at a time, two loads up to 4096 sequences.  Ordered in runs of 64, every workgroup went
+//     through all runs before its own: VARLEN_FIGURES
+constexpr int kVarSorted = 64;
+__device__ __forceinline__ int varlen_slot(const AttnParams& p, int b) { return (int)(((uint32_t)p.cu_qs[b] + (uint32_t)b) >> 1); }
+__device__ __forceinline__ bool varlen_item(const AttnParams& p, int g, int& b_out, int& h_out, int& qp_out) {
+  const int lane = threadIdx.x & 63, B = (int)p.B, H = (int)p.Hq;
+  if (B <= kVarSorted) {
     int n = 0, key = -1;
-    if (b < (int)p.B) {
-      int64_t r0, lq, lk;
-      varlen_range(p.cu_k, b, p.var_tk, p.Lk, r0, lk);
-      varlen_range(p.cu_q, b, p.var_tq, p.Lq, r0, lq);
-      // (a V tile range past Lpad, from a too small Lpad, leaves the sequence's rows untouched)
-      if (lk > 0 && ((int64_t)p.cu_vt[b] + (lk + kBK - 1) / kBK) * kBK <= p.Lpad) {
-        n = (int)((lq + 2 * kBQ - 1) / (2 * kBQ));
-        key = (int)lk;
-      }
-    }
-    const int m = min(64, (int)p.B - base);
+    if (lane < B) varlen_pairs(p, lane, n, key);
     int before = 0, total = 0;
-    for (int j = 0; j < m; j++) {
+    for (int j = 0; j < B; j++) {
       const int nj = __builtin_amdgcn_readlane(n, j), kj = __builtin_amdgcn_readlane(key, j);
       total += nj;
       if (kj > key || (kj == key && j < lane)) before += nj;
     }
-    if ((int64_t)g >= (int64_t)(start + total) * p.Hq) {
-      start += total;
-      continue;
-    }
-    const int gg = g - start * (int)p.Hq;
-    const uint64_t hit = __ballot(n > 0 && gg >= before * (int)p.Hq && gg < (before + n) * (int)p.Hq);
+    const uint64_t hit = __ballot(n > 0 && g >= before * H && g < (before + n) * H);
     if (hit == 0) return false;
     const int src = __builtin_ctzll(hit);
-    const int ns = __builtin_amdgcn_readlane(n, src), r = gg - __builtin_amdgcn_readlane(before, src) * (int)p.Hq;
-    b_out = base + src;
+    const int ns = __builtin_amdgcn_readlane(n, src), r = g - __builtin_amdgcn_readlane(before, src) * H;
+    b_out = src;
     h_out = r / ns;
     qp_out = p.causal ? ns - 1 - r % ns : r % ns;
-    n_out = ns;
     return true;
   }
-  return false;
+  const int slot = g / H;
+  int lo = 0, hi = B;  // the last sequence of lo .. hi - 1 that starts at or before the slot
+  while (hi - lo > 1) {
+    const int step = (hi - lo + 63) / 64, at = lo + lane * step;
+    const int n_ok = __popcll(__ballot(at < hi && varlen_slot(p, at) <= slot));
+    lo += max(n_ok - 1, 0) * step;
+    hi = min(hi, lo + step);
+  }
+  int n, key;
+  varlen_pairs(p, lo, n, key);
+  n = __builtin_amdgcn_readfirstlane(n);
+  const int qp = slot - __builtin_amdgcn_readfirstlane(varlen_slot(p, lo));
+  if (qp < 0 || qp >= n) return false;
+  b_out = lo;
+  h_out = g - slot * H;
+  qp_out = p.causal ? n - 1 - qp : qp;
+  return true;
 }
 
 template <bool F16OUT, bool F16V, bool KT, bool SPLIT, int FORM>
@@ -125,8 +143,8 @@ __global__ __launch_bounds__(kHFThreads) void qattn_fwd_half_kernel(AttnParams p
   int64_t Lq = p.Lq, Lk = p.Lk;
   int64_t nqb_wg_last;  // last query block of the workgroup (its key range bounds the shared stream)
   if constexpr (VAR) {
-    int vb, vh, vq, vn;
-    if (!varlen_item(p, (int)blockIdx.x, vb, vh, vq, vn)) return;
+    int vb, vh, vq;
+    if (!varlen_item(p, (int)blockIdx.x, vb, vh, vq)) return;
     b = vb;
     h = vh;
     qb = (int64_t)vq * 2 + grp;
@@ -705,8 +723,12 @@ int launch_half_varlen(AttnParams& p, int out_dtype, hipStream_t st) {
   p.nsplit = 1;
   p.tiles_per_split = (int)p.nKB;
   QATTN_REQUIRE(p.nKB <= kHFKsPair, QATTN_ERR_SHAPE, "varlen sequences hold at most %d keys", kHFKsPair * kBK);
-  // sum of ceil(len / 256) over the sequences, bounded on the host without reading their lengths
-  const int64_t g = p.Hq * std::min((p.var_tq + 2 * kBQ - 1) / (2 * kBQ) + p.B, p.B * ((p.nQB + 1) / 2));
+  // pairs of the batch, bounded on the host without reading the lengths: sum of ceil(len / 256), or the slots of a
+  // batch past kVarSorted, half the sum of ceil(len / 128) + 1
+  const int64_t pairs = p.B <= kVarSorted
+                            ? std::min((p.var_tq + 2 * kBQ - 1) / (2 * kBQ) + p.B, p.B * ((p.nQB + 1) / 2))
+                            : std::min(p.var_tq / kBQ + 2 * p.B, p.B * (p.nQB + 1)) / 2;
+  const int64_t g = p.Hq * pairs;
   QATTN_REQUIRE(g < (1ll << 31), QATTN_ERR_SHAPE, "grid too large");
   if (out_dtype == QATTN_BF16) qattn_fwd_half_kernel<false, true, false, false, HF_VAR><<<g, kHFThreads, 0, st>>>(p);
   else qattn_fwd_half_kernel<true, true, false, false, HF_VAR><<<g, kHFThreads, 0, st>>>(p);

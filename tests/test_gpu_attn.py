@@ -544,6 +544,38 @@ def test_sageattn_varlen(oracle, causal):
         assert ct >= COS_E2E
 
 
+@pytest.mark.parametrize("n,causal", [(65, False), (70, True), (130, False), (130, True), (4200, False)])
+def test_sageattn_varlen_many_sequences(n, causal):
+    """Batches of more than 64 sequences find their work by a search instead of the sorted list: the bits of the same
+    sequences in calls of at most 64 (no smoothing, so a sequence does not depend on the others).  Empty sequences, equal
+    lengths, one to five query blocks; at 4200 the search takes three steps."""
+    dev = require_gpu()
+    from telefuser_amd import sageattn2 as sa
+
+    rng = np.random.default_rng(n + causal)
+    sizes = [0, 0, 1, 2, 3] if n > 1000 else [0, 1, 64, 127, 128, 129, 200, 256, 257, 300, 513, 600]
+    lq = rng.choice(sizes, n)
+    lk = lq.copy() if causal else rng.choice(sizes, n)
+    lq[-1] = lk[-1] = lk[0] = 130  # (the first and last slots are taken)
+    lq[0] = 130 if causal else 0
+    log(f"varlen many n={n} causal={causal} rows={lq.sum()} keys={lk.sum()}")
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn((int(m.sum()), 3, 128), generator=g).to(torch.bfloat16).to(dev) for m in (lq, lk, lk))
+
+    def run(a, e):
+        cq, ck = (np.concatenate([[0], np.cumsum(m[a:e])]).astype(np.int32) for m in (lq, lk))
+        q0, k0 = int(lq[:a].sum()), int(lk[:a].sum())
+        kk, vv = (t[k0:k0 + int(ck[-1])] for t in (k, v))
+        return sa.sageattn_varlen(q[q0:q0 + int(cq[-1])], kk, vv, torch.from_numpy(cq).to(dev), torch.from_numpy(ck).to(dev),
+                                  int(lq[a:e].max()), int(lk[a:e].max()), is_causal=causal, smooth_k=False)
+
+    want = torch.cat([run(a, min(a + 64, n)) for a in range(0, n, 64)])
+    got = run(0, n)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want), f"{int((got != want).any(-1).any(-1).sum())} rows differ"
+    assert bool((got.float().abs().amax((1, 2)) > 0).any())
+
+
 def test_sageattn_varlen_malformed_tables():
     """Sequence tables that break the contract (decreasing entries, entries past the packed tensors, a
     sequence longer than max_seqlen) are clamped on the device to disjoint row ranges of the packed
