@@ -1844,9 +1844,9 @@ extern "C" int qattn_fwd_q16(qattn_seq q, qattn_seq k8, const float* k_scale, co
 }
 
 // ---- packed variable-length batches ----
-// One launch over every sequence of a packed batch (attn_qk_int8_block_varlen.py:68-155): the grid covers
-// max_seqlen_q rows per sequence and head, and each workgroup reads its sequence's row range, scale
-// offsets and V tile column from the device tables, so the host never reads cu_seqlens.
+// One launch over every sequence of a packed batch (attn_qk_int8_block_varlen.py:68-155): the grid is a bound, from the
+// packed lengths alone, on the pairs of query blocks of all sequences and heads; each workgroup finds its sequence, head
+// and pair in the device tables (attn_half.hip), so the host never reads cu_seqlens.
 extern "C" int qattn_fwd_varlen(qattn_seq q8, const float* q_scale, qattn_seq k8, const float* k_scale,
                                 const uint16_t* v16, int64_t Lpad, qattn_seq o, int out_dtype, int64_t B,
                                 int64_t total_q, int64_t total_k, int64_t max_lq, int64_t max_lk, int64_t Hq,

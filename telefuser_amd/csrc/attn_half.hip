@@ -72,7 +72,8 @@ __device__ __forceinline__ void varlen_pairs(const AttnParams& p, int b, int& n,
 //   * More: in sequence order with the heads innermost.  Sequence b starts at slot (cu_qs[b] + b) / 2 of each head, which
 //     leaves room for its ceil(blocks / 2) pairs and at most one slot more, so that the block offsets are all the
 //     search needs: 64 of them at a time, two loads up to 4096 sequences.  Ordered in runs of 64, every workgroup went
-//     through all runs before its own: VARLEN_FIGURES
+//     through all runs before its own (a call over 1000 sequences of 64 tokens, 12 heads, 3469 -> 1132 us; 200 of 32 .. 400
+//     tokens 750 -> 533; 100 of 64 .. 8192 tokens, where the order counts most, 4308 -> 4067).
 constexpr int kVarSorted = 64;
 __device__ __forceinline__ int varlen_slot(const AttnParams& p, int b) { return (int)(((uint32_t)p.cu_qs[b] + (uint32_t)b) >> 1); }
 __device__ __forceinline__ bool varlen_item(const AttnParams& p, int g, int& b_out, int& h_out, int& qp_out) {
