@@ -572,7 +572,8 @@ def _finish_lse(lse, q, km, tensor_layout, sm_scale):
     if km is None:
         return lse / LOG2E
     b, lq, hq, d = _dims(q, tensor_layout)
-    if torch.is_grad_enabled() and q.requires_grad:  # (the correction, in torch, keeps its graph)
+    if (torch.is_grad_enabled() and q.requires_grad) or torch.autograd.forward_ad.unpack_dual(q).tangent is not None:
+        # (the correction, in torch, keeps its graph and its tangent)
         qq = q if tensor_layout == "HND" else q.transpose(1, 2)
         corr = torch.matmul(qq, km.repeat_interleave(hq // km.shape[1], dim=1).unsqueeze(-1)).squeeze(-1)
         return lse / LOG2E + corr.to(torch.float32) * sm_scale

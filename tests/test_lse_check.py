@@ -32,3 +32,30 @@ def test_empty_row_output_must_be_zero():
     out[0, 1, 3] = 1e-3
     with pytest.raises(AssertionError):
         lse_max_err(np.array([[1.0, NINF]]), np.array([[1.0, NINF]]), out)
+
+
+def test_finish_lse_keeps_graph_and_tangent(monkeypatch):
+    """The smoothing correction of an LSE stays differentiable in Q, in reverse and in forward mode: neither takes the
+    kernel that writes lse in place."""
+    import torch
+    import torch.autograd.forward_ad as fwd
+
+    from telefuser_amd import _lib
+    from telefuser_amd import sageattn2 as sa
+
+    def no_kernel():
+        raise AssertionError("the kernel was called")
+
+    monkeypatch.setattr(_lib, "load", no_kernel)
+    g = torch.Generator().manual_seed(1)
+    q, t = (torch.randn((2, 5, 4, 64), generator=g) for _ in range(2))  # NHD, grouped heads
+    km, lse = torch.randn((2, 2, 64), generator=g), torch.randn((2, 4, 5), generator=g)
+    want = torch.einsum("blhd,bhd->bhl", t, km.repeat_interleave(2, dim=1)) * 0.125
+    with fwd.dual_level():
+        out = fwd.unpack_dual(sa._finish_lse(lse.clone(), fwd.make_dual(q, t), km, "NHD", 0.125))
+        torch.testing.assert_close(out.tangent, want)
+    qr = q.clone().requires_grad_()
+    got = sa._finish_lse(lse.clone(), qr, km, "NHD", 0.125)
+    torch.testing.assert_close(got.detach(), out.primal)
+    (grad,) = torch.autograd.grad(got.sum(), qr)
+    torch.testing.assert_close(grad, (km.repeat_interleave(2, dim=1) * 0.125)[:, None].expand_as(q))
