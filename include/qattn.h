@@ -244,7 +244,8 @@ int qattn_sage_quant_half(qattn_seq q, qattn_seq k, qattn_seq v, int dtype, int 
                           size_t workspace_bytes, qattn_stream_t stream);
 
 /*
- * The prologue of the INT8-QK / FP8-PV path in four launches: one pass over K and V for their column
+ * The prologue of the INT8-QK / FP8-PV path in four launches (two for small inputs, whose second does the steps
+ * after the column pass): one pass over K and V for their column
  * statistics (K sum when smooth_k; V max |v|, or sum / max / min when smooth_v), one finalize (k_mean
  * [B, Hkv, D] in the input dtype, v_scale, v_mean), V to FP8 tiles (as qattn_per_channel_fp8_ex), and K then
  * Q to INT8 in one launch (qk_quant_gran 1: per block, Q times q_sm_scale = sm_scale * log2(e), CUDA

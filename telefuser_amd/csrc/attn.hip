@@ -1360,7 +1360,9 @@ static int num_splits_for(int64_t B, int64_t Lq, int64_t Lk, int64_t Hq, int64_t
   // 256 CUs x 2 resident workgroups.  Split only when the grid leaves CUs without any workgroup: at
   // 256 or more workgroups the combine traffic of a split costs more than the idle half-slots it fills
   // (C5, 444 workgroups: 0.63 ms unsplit against 0.79 ms with 3 splits); every split still gets at least
-  // 8 key tiles
+  // 8 key tiles.  (Block-sparse launches, pp = false, keep this count of one-block workgroups and all key tiles, though
+  // theirs hold two blocks, one to a CU, and a split takes its share of the kept tiles' list as if all were kept: how
+  // many are is not known here, and no count for them was measured.)
   const int64_t target = 1024;
   const int64_t min_s = (nkb + max_tiles - 1) / max_tiles;
   if (wgs >= target / 4) return (int)min_s;
@@ -2018,7 +2020,7 @@ extern "C" int qattn_fwd_pv16(qattn_seq q8, const float* q_scale, qattn_seq k8, 
 }
 
 extern "C" int qattn_fwd_block_sparse_num_splits(int64_t B, int64_t Lq, int64_t Lk, int64_t Hq) {
-  return num_splits_for(B, Lq, Lk, Hq, kSpMaxTiles, false);
+  return num_splits_for(B, Lq, Lk, Hq, half_max_tiles(false, true), false);
 }
 
 extern "C" int qattn_fwd_block_sparse(qattn_seq q8, const float* q_scale, qattn_seq k8, const float* k_scale,

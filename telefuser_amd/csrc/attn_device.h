@@ -17,8 +17,6 @@ constexpr int kNBuf = kPrefetch + 1;
 // k_scales staged in LDS per workgroup (floats).  Sized so that two workgroups per CU still fit in the
 // 160 KiB of LDS next to the K/V buffers: 24 + 24 + 30 KiB.
 constexpr int kKsLdsFloats = 7680;
-// block-sparse launches (half P.V only) stage the active tiles' ids next to their scales
-constexpr int kSpMaxTiles = 1024;
 // multi-block launches (one workgroup streams up to kMqMaxBlocks query blocks of one head through one
 // K/V pipeline): short key ranges only, so their k_scales and q_scales are staged whole in LDS
 constexpr int kMqMaxTiles = 64;

@@ -13,19 +13,20 @@
 //   group 1:    -  | M(0) | V(0) | M(1) | ...        V(t) = mask, softmax, P(t) to half  (VALU)
 //
 // Measured against a kernel with one 128-row block and four waves per workgroup, two workgroups per CU, whose waves
-// fell into step (MFMAs, then softmax): 32760 x 32760 x 12 heads per-thread scales 5.31 -> 4.60 ms a call (1.43
-// PFLOP/s; without the softmax 3.4 ms, without the LDS reads 3.9, without the DMA 4.1), 8000 x 8000 x 2 129 -> 80 us,
-// 8 sequences of 257 .. 6240 tokens, 12 heads 1467 -> 443 us in the kernel (mostly HF_VAR's order of the work),
-// block-sparse 32760 x 32760 x 12 at a quarter of the tiles 1440 -> 1330 us.
+// fell into step (MFMAs, then softmax): 32760 x 32760 x 12 heads per-thread scales 5.40 (with the combine of the two
+// splits that it needed) -> 4.60 ms (1.43 PFLOP/s; matrix pipe busy 55 %, VALU 62 %), 8 sequences of 257 .. 6240
+// tokens, 12 heads 1475 -> 433 us (mostly HF_VAR's order of the work), block-sparse 32760 x 32760 x 12 at a quarter of
+// the tiles 1555 -> 1475 us.
 //
 // Forms (one template axis):
 //   HF_PAIR  the groups are two adjacent 128-row query blocks of a head: each K/V tile is fetched once for both
 //   HF_VAR   the same over a packed variable-length batch: the workgroups find their (sequence, head, pair) in
-//            the device tables, longest key ranges first
+//            the device tables, longest key ranges first up to 64 sequences
 //   HF_OWN   each group takes a query block of its own (block-sparse masks, whose rows differ, and dense launches
-//            with one or three query blocks per head, where a pair would be half empty, up to half_own_tiles).  The tiles that both
-//            blocks visit come first, fetched once for both and five tiles ahead (their order follows the mask, so
-//            a third of the fetches miss L2); then each group streams what only its block visits.
+//            with one or three query blocks per head, where a pair would be half empty, up to half_own_tiles).  The
+//            tiles that both blocks visit come first, fetched once for both and five tiles ahead (their order follows
+//            the mask: 30 % of the requests miss L2, against 4 % of HF_PAIR's); then each group streams what only its
+//            block visits.
 #include "attn_device.h"
 
 namespace qattn {

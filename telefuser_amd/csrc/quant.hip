@@ -752,9 +752,9 @@ static void launch_v_tile_half(dim3 grid, bool conv, int64_t D, const qattn_seq&
 // ------------------------------------------------------------------------------------------------
 // small inputs: the finalize steps, V's tiles and the quantizers in one launch
 // ------------------------------------------------------------------------------------------------
-// A prologue of a few MB is bound by its chain of launches, not by its bytes (4680 keys x 12 heads: 33 us in four
-// launches for 14 MB).  Every workgroup here reduces the chunk partials of its own (batch entry, head) itself - a few
-// KiB from L2, in reduce_chunks' order, so the mean and the scales keep their bits - and goes on with its block: a
+// A prologue of a few MB is bound by its chain of launches, not by its bytes (4680 keys x 12 heads: 34 us in four
+// launches for 14 MB, 25 in two).  Every workgroup here reduces the chunk partials of its own (batch entry, head)
+// itself - a few KiB from L2, in reduce_chunks' order, so the mean and the scales keep their bits - and goes on with its block: a
 // pair of V tiles, 64 K rows or a Q block.  The first workgroup of each head writes the mean and the scales out.
 constexpr int64_t kSmallChunks = 32, kSmallWorkgroups = 4096;
 struct SmallArgs {
@@ -794,8 +794,9 @@ __device__ __forceinline__ void quant_index(const QuantJob& J, uint32_t wg, uint
 }
 
 // quant_per_block_kernel's block without its packed sequences, the row subtracted from every row
-// (mean: D half words in LDS, or null).  The two are kept apart: as one function the general kernel spilled nine
-// registers instead of one (45 -> 51 us for K at 32760 x 12).
+// (mean: D half words in LDS, or null).  The two are kept apart: as one function the general kernel's instantiations
+// keep their registers within a few, but not their schedules (Q and K at 32760 x 12 x 128: per block 67.8 -> 68.9 us, per
+// warp 77.3 -> 80.5, with the 64 / 128-row tables 90.9 -> 100.9).
 template <bool IS_FP16, int VARIANT, int D, int CR>
 __device__ __forceinline__ void quant_block(const QuantJob& J, uint32_t wg, const uint16_t* mean) {
   constexpr bool GROUPED = CR != 0;
@@ -1685,9 +1686,10 @@ static int64_t stat_rows(int64_t B, int64_t L) {
   return r;
 }
 static int64_t stat_chunks(int64_t B, int64_t L) { return (L + stat_rows(B, L) - 1) / stat_rows(B, L); }
-// widest row: 3 chunks per lane.  With 6 or 10 the row and its sums take 176 and 256 registers, two waves per SIMD, and one
-// pass is no faster than the separate kernels: the prologue at 2 x 3000 x 24 heads takes 64.7 us with those and 69.4 with
-// one pass, at 15399 x 40 heads 250.9 and 249.3
+// widest row: 3 chunks per lane (the whole prologue at 32760 x 12 x 128, 3 chunks: 189 us, 158 with the one pass).  With 4
+// one pass is already behind the separate kernels (32760 x 16 x 128 205 us, 214 with the one pass; 5000 x 16 47 and 52;
+// only 1500 x 16 29 and 25); with 6 or 10 the row and its sums take 176 and 256 registers, two waves per SIMD (a call
+// at 2 x 3000 x 24 heads 64.7 and 69.4, at 15399 x 40 heads 250.9 and 249.3).
 constexpr int64_t kStatMaxCols = 64 * 8 * 3;
 
 extern "C" size_t qattn_norm_rope_stats_workspace_size(int64_t B, int64_t L, int64_t H, int64_t D) {
@@ -1862,11 +1864,14 @@ extern "C" int qattn_v_tile_half_varlen_ex(qattn_seq v, int dtype, int out_dtype
 }
 
 // ------------------------------------------------------------------------------------------------
-// the whole SAGE prologue: K mean, Q/K INT8, V FP8 in four launches
+// the whole SAGE prologue: K mean, Q/K INT8, V FP8 in four launches, or two (small_prologue)
 // ------------------------------------------------------------------------------------------------
 
 // Whether the prologue runs as column pass + sage_small_kernel: its workgroups re-read their head's partials
-// (nchunk x D floats each), which has to stay small beside the launches saved (measured: see sage_small_kernel).
+// (nchunk x D floats each), which has to stay small beside the launches saved.  Kernel time of the separate launches /
+// of two, us, D = 128, 40 heads: FP8 V 3840 workgroups 54 / 49, 5760 72 / 73, 7680 91 / 85 to 90, 11520 132 / 142; half V
+// 5120 workgroups 63 / 52, 10240 121 / 106.  12 heads: 24 chunks 35 / 28, 32 chunks 38 / 32, 48 chunks 51 / 46.  So the
+// count of workgroups stays below where FP8 V crosses over; past 32 chunks the two launches would still be ahead.
 static bool small_prologue(const SmallArgs& a) {
   return a.nchunk <= kSmallChunks && a.nvwg + a.k.nwg + a.q.nwg <= kSmallWorkgroups;
 }

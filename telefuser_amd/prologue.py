@@ -3,9 +3,10 @@
 The reference runs ``q = rope_apply(norm_q(self.q(x)))`` (and the same for K) as separate kernels and
 then quantizes inside the attention call (telefuser/models/wan_video_dit.py:196-207, norm_infer in
 telefuser/kernel/triton/norm.py:469-507, the interleaved rotary kernel in
-telefuser/kernel/triton/rotary.py:21-88).  Here the linear outputs go straight to INT8: a per-row
-RMSNorm statistic pass, one pass for the K mean of the rotated values, and one quantizer launch that
-applies norm + RoPE to every chunk it loads, so the normalized / rotated bf16 tensors never reach HBM.
+telefuser/kernel/triton/rotary.py:21-88).  Here the linear outputs go straight to INT8: one pass
+over Q and K for the RMSNorm statistics of both and the K mean of the rotated values (rows wider than 1536
+values or not in 16-byte pieces: a statistics pass each, then one for the mean), and one quantizer launch
+that applies norm + RoPE to every chunk it loads, so the normalized / rotated bf16 tensors never reach HBM.
 """
 
 from __future__ import annotations

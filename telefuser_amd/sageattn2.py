@@ -198,7 +198,7 @@ def sage_quant(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tensor_layout:
                qk_quant_gran: str = "per_block", sm_scale: Optional[float] = None, smooth_k: bool = True,
                scale_max: float = 448.0, smooth_v: bool = False, scale_layout: str = "sm89", quantize_q: bool = True):
     """The whole prologue of the INT8-QK / FP8-PV path in four launches (column passes of K and V,
-    their finalize, V to FP8, K and Q to INT8): the same outputs, bit for bit, as k_mean + the
+    their finalize, V to FP8, K and Q to INT8), or two for small inputs: the same outputs, bit for bit, as k_mean + the
     per_block / per_warp / per_thread quantizer + per_channel_fp8 (CUDA quantizer variant).
     ``scale_layout="sm90"`` (per_warp / per_thread only) gives the sm90 entry's tables, as per_warp_int8 /
     per_thread_int8 with BLKQ=64, WARPQ=16, BLKK=128.  ``quantize_q=False`` leaves Q out (for qattn_fwd_q16,
@@ -539,7 +539,7 @@ def _sage_forward(q, k, v, tensor_layout, is_causal, qk_quant_gran, sm_scale, pv
                             return_lse=return_lse, qk_quant_gran=qk_quant_gran, v_mean=vm)
         return _sage_finish(res, q, km, hq, hkv, head_dim_og, tensor_layout, sm_scale, smooth_k, return_lse)
     elif pv == "fp8" and quant_variant == "cuda":
-        # K mean, Q/K INT8 and V FP8 in one fused prologue (four launches)
+        # K mean, Q/K INT8 and V FP8 in one fused prologue
         q_int8, q_scale, k_int8, k_scale, km, v_fp8, v_scale, vm = sage_quant(
             q, k, v, tensor_layout=tensor_layout, qk_quant_gran=qk_quant_gran, sm_scale=sm_scale, smooth_k=smooth_k,
             scale_max=scale_max, smooth_v=smooth_v)
@@ -654,7 +654,7 @@ def sageattn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu_seqlen
     (quant_per_block_varlen.py:22-70), V in fp16 and P rounded to fp16 for P.V
     (attn_qk_int8_block_varlen.py:42-65; P.V accumulates in fp32 here).  ``is_causal`` masks per
     sequence, top-left aligned.  The whole batch is four launches (block offsets, Q/K quantizer, V tiles,
-    attention) whose workgroups read the sequence tables on the device: the host never reads cu_seqlens,
+    attention; two more for the K mean) whose workgroups read the sequence tables on the device: the host never reads cu_seqlens,
     and sizes its buffers from the packed lengths and max_seqlen_q / max_seqlen_k alone.  The tables are
     expected to be valid as in the reference (start at 0, non-decreasing, within the packed tensors, every
     length at most its max_seqlen); the kernels clamp each sequence to the packed tensors and to
