@@ -281,6 +281,9 @@ __global__ __launch_bounds__(kHFThreads) void qattn_fwd_half_kernel(AttnParams p
   }
   const int t_end = SPLIT ? min(n_slots, t_lo + p.tiles_per_split) : n_slots;
   const int n_kt = max(t_end - t_lo, 0);  // slots 0 .. n_kt - 1 of this group, from here on
+  // A pair streams the tiles of its last block; those past this block's own diagonal are not multiplied (their p is 0, but
+  // a V that is not finite would make NaN of it, in rows that may not see its key).
+  const int n_live = OWN ? n_kt : max(min((kv_end_s + kBK - 1) / kBK, t_end) - t_lo, 0);
   int n_own = 0;  // slots after the shared ones, of the longer group
   if constexpr (OWN) {
     n_sh = max(min(n_sh, t_end) - t_lo, 0);
@@ -540,17 +543,24 @@ __global__ __launch_bounds__(kHFThreads) void qattn_fwd_half_kernel(AttnParams p
     if (n > DK) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DV * kPer) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    const int live = OWN ? steps : min(n_live, steps);
     int buf = 0;  // slot i's buffer, i % NB
-    auto step = [&](int i, auto first_t) __attribute__((always_inline)) {
+    // live_t: false for the steps past the block's own tiles, which only fetch; the first of them still owes the last P.V
+    auto step = [&](int i, auto first_t, auto live_t) __attribute__((always_inline)) {
+      constexpr bool kLive = decltype(live_t)::value;
       const int prev = buf == 0 ? NB - 1 : buf - 1, prev2 = prev == 0 ? NB - 1 : prev - 1;
       if (SH || i < n) {
         const int left = n - DK - i;  // <= 0 at the stream's end: no K to issue, < 0: no V either
         if (left > 0) dma_k(sh_t, tq[DK], prev);
         if (left >= 0) dma_v(sh_t, tq[DV], prev2);
-        // (raised wave priority: the vector-stage wave of the SIMD cannot delay the issue of the MFMAs)
-        __builtin_amdgcn_s_setprio(1);
-        stage_m(s0 + i, b0 + buf, b0 + prev, first_t);
-        __builtin_amdgcn_s_setprio(0);
+        if constexpr (kLive) {
+          // (raised wave priority: the vector-stage wave of the SIMD cannot delay the issue of the MFMAs)
+          __builtin_amdgcn_s_setprio(1);
+          stage_m(s0 + i, b0 + buf, b0 + prev, first_t);
+          __builtin_amdgcn_s_setprio(0);
+        } else if (i == live && i > 0) {
+          pv(b0 + prev);
+        }
         // This wave's share of K(i + 1) and V(i), issued DV steps ago, has landed; what the last DV steps issued may
         // stay in flight (nothing was issued for slots past the end).
         if (left > 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DV * kPer) : "memory");
@@ -566,7 +576,7 @@ __global__ __launch_bounds__(kHFThreads) void qattn_fwd_half_kernel(AttnParams p
         if constexpr (OWN) {
           if (sparse) nxt = lds_tid[grp * kHFKsOwn + s0 + min(i + DK + 1, n - 1)];
         }
-        stage_v(tq[0]);
+        if constexpr (kLive) stage_v(tq[0]);
 #pragma unroll
         for (int d = 0; d < DK; d++) tq[d] = tq[d + 1];
         tq[DK] = OWN ? __builtin_amdgcn_readfirstlane(nxt) : nxt;
@@ -576,10 +586,12 @@ __global__ __launch_bounds__(kHFThreads) void qattn_fwd_half_kernel(AttnParams p
     };
     static_assert(DV <= 4, "vmcnt cases");
     if (grp == 1) pp_barrier();
-    if (steps > 0) step(0, std::true_type{});
-    for (int i = 1; i < steps; i++) step(i, std::false_type{});
+    if (live > 0) step(0, std::true_type{}, std::true_type{});
+    for (int i = 1; i < live; i++) step(i, std::false_type{}, std::true_type{});
+    if constexpr (!OWN)
+      for (int i = live; i < steps; i++) step(i, std::false_type{}, std::false_type{});
     if (grp == 0) pp_barrier();
-    if (n > 0) pv(b0 + (buf == 0 ? NB - 1 : buf - 1));
+    if (n > 0 && live == steps) pv(b0 + (buf == 0 ? NB - 1 : buf - 1));
   };
   phase(std::true_type{}, 0, n_sh, n_sh, tq_sh);
   if constexpr (OWN) {

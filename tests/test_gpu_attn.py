@@ -344,6 +344,53 @@ def test_half_pv_causal_split_padding(oracle):
     _run_and_check(oracle, q, k[:, :300], v[:, :300], pv="half", causal=True)
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("gran,kw", [("per_block", {}), ("per_thread", dict(num_splits=3)), ("per_warp", dict(q_offset=100))])
+def test_half_causal_later_values_stay_out(gran, kw, bad):
+    """A query block of a causal launch does not multiply key tiles past its own end, though it shares a workgroup with
+    the next block: V rows there that are not finite leave its rows as they are."""
+    dev = require_gpu()
+    from telefuser_amd import sageattn2 as sa
+
+    q, k, v = (t.to(dev) for t in qkv(1, 640, 768, 2, 1, seed=77, k_offset_std=0.5))
+    q8, qs, k8, ks, _, _ = sa.sage_quant_half(q, k, v, tensor_layout="NHD", qk_quant_gran=gran)
+
+    def run(vv):
+        return sa.qattn_fwd(q8, qs, k8, ks, sa.v_tile_half(vv, "NHD"), None, tensor_layout="NHD", is_causal=True,
+                            qk_mult=0.1, qk_quant_gran=gran, **kw)
+
+    off = kw.get("q_offset", 0)
+    want = run(v)
+    for key in (200, 330, 520):  # the first key tile that block i does not visit: past its last row + offset
+        vv = v.clone()
+        vv[:, key] = bad
+        got = run(vv)
+        first = max(key // 64 * 64 - off, 0) // 128 * 128  # (a tile that a block visits in part counts as its own)
+        log(f"half causal {gran} {kw} {bad} key={key}: rows below {first}")
+        assert torch.equal(got[:, :first], want[:, :first])
+        assert not bool(torch.isfinite(got[:, key - off:].float()).any())
+
+
+def test_varlen_causal_later_values_stay_out():
+    dev = require_gpu()
+    from telefuser_amd import sageattn2 as sa
+
+    lens = [300, 640, 100]
+    cu = torch.tensor([0, 300, 940, 1040], dtype=torch.int32, device=dev)
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn((1040, 2, 128), generator=g).to(torch.float16).to(dev) for _ in range(3))
+    run = lambda vv: sa.sageattn_varlen(q, k, vv, cu, cu, max(lens), max(lens), is_causal=True)
+    want = run(v)
+    for b, key in ((0, 130), (1, 200), (1, 400)):
+        vv = v.clone()
+        row = int(cu[b]) + key
+        vv[row] = float("nan")
+        got = run(vv)
+        last = int(cu[b]) + key // 128 * 128
+        assert torch.equal(got[:last], want[:last]) and torch.equal(got[int(cu[b + 1]):], want[int(cu[b + 1]):])
+        assert not bool(torch.isfinite(got[row:int(cu[b + 1])].float()).any())
+
+
 @pytest.mark.parametrize("Lq,Lk,Hq,Hkv,gran,kw", [
     # one and three query blocks over key ranges at and past what a group of its own stages (256 tiles per thread, 1024
     # per block): unsplit launches go over to pairs there; the last two with a KV split whose runs are that long
