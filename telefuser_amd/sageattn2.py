@@ -183,15 +183,18 @@ def per_channel_fp8(v: torch.Tensor, tensor_layout: str = "HND", scale_max: floa
     return v_fp8, v_scale, vm
 
 
-def _check_kv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout: str, exact: bool) -> None:
-    """The fused prologues address q, k and v with q's batch and head dim and k's heads and length: k and v have to
-    hold all of it (``exact``: and no other batch entries or heads; a v longer than k is read up to k's length)."""
-    b, _, _, d = _dims(q, layout)
+def _launch_dims(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout: str, exact: bool):
+    """(B, Lq, Hq, D, Lk, Hkv) of a fused prologue, which addresses q, k and v with q's batch and head dim and k's heads
+    and length: k and v have to hold all of it (``exact``: and no other batch entries or heads; a v longer than k is read
+    up to k's length)."""
+    b, lq, hq, d = _dims(q, layout)
     bk, lk, hkv, dk = _dims(k, layout)
-    bv, lv, hv, dv = _dims(v, layout)
-    if dk != d or dv != d or bk < b or bv < b or hv < hkv or lv < lk or (exact and (bk, bv, hv) != (b, b, hkv)):
-        raise ValueError(f"k must have q's batch and head dim and v the shape of k, got q {tuple(q.shape)}, "
-                         f"k {tuple(k.shape)}, v {tuple(v.shape)} ({layout})")
+    if v.shape != k.shape or bk != b or dk != d:
+        bv, lv, hv, dv = _dims(v, layout)
+        if dk != d or dv != d or bk < b or bv < b or hv < hkv or lv < lk or (exact and (bk, bv, hv) != (b, b, hkv)):
+            raise ValueError(f"k must have q's batch and head dim and v the shape of k, got q {tuple(q.shape)}, "
+                             f"k {tuple(k.shape)}, v {tuple(v.shape)} ({layout})")
+    return b, lq, hq, d, lk, hkv
 
 
 def sage_quant(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tensor_layout: str = "HND",
@@ -215,9 +218,7 @@ def sage_quant(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tensor_layout:
     sm90 = scale_layout == "sm90"
     if sm90 and gran == 1:
         raise ValueError("scale_layout='sm90' needs qk_quant_gran 'per_warp' or 'per_thread'")
-    _check_kv(q, k, v, tensor_layout, False)
-    b, lq, hq, d = _dims(q, tensor_layout)
-    _, lk, hkv, _ = _dims(k, tensor_layout)
+    b, lq, hq, d, lk, hkv = _launch_dims(q, k, v, tensor_layout, False)
     dev = q.device
     nqb, nkb = _scale_blocks(lq, lk, sm90)
     q_per = {1: 1, 2: 4, 3: 32}[gran]
@@ -255,9 +256,7 @@ def sage_quant_half(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tensor_la
     L = _lib.load()
     if q.dtype != k.dtype:
         raise ValueError("q and k must have the same dtype")
-    _check_kv(q, k, v, tensor_layout, True)
-    b, lq, hq, d = _dims(q, tensor_layout)
-    _, lk, hkv, _ = _dims(k, tensor_layout)
+    b, lq, hq, d, lk, hkv = _launch_dims(q, k, v, tensor_layout, True)
     dev = q.device
     vdt = _lib.dtype_code(v.dtype)
     if fp16_v:
